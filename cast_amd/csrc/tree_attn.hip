@@ -71,6 +71,18 @@ struct KvSource {
     int32_t store, cap;
 };
 
+// Division of n in [0, 2^31) by a divisor the host knows: (mulhi(m, n) + n) >> s
+// with s = ceil(log2 d) and m = floor(2^32 * (2^s - d) / d) + 1.
+struct FastDiv {
+    uint32_t m, s;
+    __device__ __forceinline__ int div(int n) const { return (int)((__umulhi(m, (uint32_t)n) + (uint32_t)n) >> s); }
+};
+static FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while (s < 31 && (1u << s) < d) ++s;
+    return {(uint32_t)((((uint64_t)1 << 32) * (((uint64_t)1 << s) - d)) / d + 1), s};
+}
+
 struct AttnArgs {
     const void *q;
     KvSource kv;
@@ -90,7 +102,9 @@ struct AttnArgs {
     int32_t sk_wgs;     // stream-K workgroups (resident at once; a multiple of 2 * xcds)
     int32_t sk_min_tiles;   // shortest stream-K lane (key tiles)
     float *sk_lse;      // stream-K partial lse [2 * sk_wgs][rows_wg] (partial O at part_o)
-    int32_t rows_wg;    // query rows per workgroup
+    int32_t rows_wg;    // query rows per workgroup (a power of two)
+    int32_t rows_shift; // log2(rows_wg)
+    FastDiv by_chunk, by_xcds, by_G;
     int32_t comb_groups;  // combine kernel: head groups per packed token
     float *part_o;      // [part_rows][Hq][D] fp32, normalised partial outputs
     float *part_lse;    // [part_rows][Hq]    fp32, base-2 partial lse
@@ -104,19 +118,32 @@ struct Seq {
     int64_t part_off;   // first partial row of this request (only if ns > 1)
 };
 
+// a / b for a >= 0, b > 0: below 2^22 by the reciprocal in float, whose
+// quotient is off by at most one (about 10 instructions against the 30 of
+// the compiler's 32-bit division, several of which sit in series in front of
+// a workgroup's first load).
+__device__ __forceinline__ int udiv(int a, int b) {
+    if (a >= 1 << 22) return (int)((uint32_t)a / (uint32_t)b);
+    int q = (int)((float)a * __builtin_amdgcn_rcpf((float)b));
+    const int r = a - q * b;
+    q += r >= b ? 1 : 0;
+    return q - (r < 0 ? 1 : 0);
+}
+
 // Reads and checks request b's metadata; `report` raises the device flags.
-__device__ __forceinline__ bool load_seq(const AttnArgs &a, int b, Seq &s, bool report) {
+// All loads are issued before any is used: one round trip.  unordered: cu_q
+// decreases here.
+__device__ __forceinline__ bool load_seq(const AttnArgs &a, int b, Seq &s, bool report, bool &unordered) {
     const int S = a.prefix_len[b], P = a.pack_len[b];
     const int q0 = a.cu_q[b], q1 = a.cu_q[b + 1];
-    int kv0 = 0, kv1 = S + P;
-    bool bad_kv;
-    if (a.kv.store) {
-        bad_kv = S > a.kv.cap;
-    } else {
+    int kv0 = 0, kv1 = 0;
+    if (!a.kv.store) {
         kv0 = a.cu_kv[b];
         kv1 = a.cu_kv[b + 1];
-        bad_kv = kv0 < 0 || kv1 > a.total_kv || kv1 - kv0 != S + P;
     }
+    unordered = q1 < q0;
+    const bool bad_kv =
+        a.kv.store ? S > a.kv.cap : kv0 < 0 || kv1 > a.total_kv || kv1 - kv0 != S + P;
     if ((a.kv.store ? max(S, P) : S + P) > a.max_rows) {
         if (report) raise_flag(a.status, CAST_FLAG_TOO_LONG);
         return false;
@@ -135,10 +162,12 @@ __device__ __forceinline__ bool load_seq(const AttnArgs &a, int b, Seq &s, bool 
     s.T = S + P;
     s.q0 = q0;
     s.kv0 = kv0;
-    s.ns = P == 0 ? 0 : (s.T + a.chunk - 1) / a.chunk;
-    s.rb = (P * a.G + a.rows_wg - 1) / a.rows_wg;
-    const int per = s.ns ? (s.T + s.ns - 1) / s.ns : 0;
-    s.split_len = (per + 63) & ~63;
+    s.ns = P == 0 ? 0 : a.by_chunk.div(s.T - 1) + 1;
+    s.rb = (P * a.G + a.rows_wg - 1) >> a.rows_shift;
+    // ceil(T / ns) rounded up to 64 keys, which is ceil(ceil(T / 64) / ns) tiles
+    const int tiles = (int)(((uint32_t)s.T + 63) >> 6);
+    s.split_len = s.ns <= 1 ? tiles * 64 : udiv(tiles + s.ns - 1, s.ns) * 64;
+    if (P == 0) s.split_len = 0;
     return true;
 }
 
@@ -188,8 +217,8 @@ __device__ __forceinline__ Seq shfl_seq(const Seq &t, int src) {
 __device__ __forceinline__ int sat32(int64_t v) { return (int)min(v, (int64_t)0x7fffffff); }
 __device__ __forceinline__ int items_of(const AttnArgs &a, const Seq &t) { return sat32((int64_t)a.Hkv * t.ns * t.rb); }
 
-// Totals over the requests that pass load_seq (work items, key rows, query
-// rows), and whether any request failed it.  Wave 0 of the workgroup reports
+// Totals over the requests that pass load_seq (work items - batches above 64
+// requests only -, key rows, query rows), and whether any request failed it.  Wave 0 of the workgroup reports
 // invalid requests.
 struct BatchTotals {
     int64_t items, kv_sum, q_sum;
@@ -198,13 +227,13 @@ struct BatchTotals {
 };
 
 // Adds the 64 requests b0 + lane (lane holding request b, ok when it passed
-// load_seq) to the totals.
-__device__ __forceinline__ void add_totals(BatchTotals &r, const AttnArgs &a, int b, bool ok, const Seq &t) {
-    r.items += wave_sum(ok ? items_of(a, t) : 0);
+// load_seq) to the row totals.
+__device__ __forceinline__ void add_totals(BatchTotals &r, const AttnArgs &a, int b, bool ok, const Seq &t,
+                                           bool unordered) {
     r.kv_sum += wave_sum(ok ? t.T : 0);
     r.q_sum += wave_sum(ok ? t.P : 0);
     r.bad |= __ballot(b < a.batch && !ok) != 0;
-    r.unordered |= __ballot(b < a.batch && a.cu_q[b + 1] < a.cu_q[b]) != 0;
+    r.unordered |= __ballot(b < a.batch && unordered) != 0;
 }
 
 __device__ BatchTotals batch_totals(const AttnArgs &a) {
@@ -213,8 +242,10 @@ __device__ BatchTotals batch_totals(const AttnArgs &a) {
     for (int b0 = 0; b0 < a.batch; b0 += 64) {
         const int b = b0 + lane;
         Seq t{};
-        const bool ok = b < a.batch && load_seq(a, b, t, threadIdx.x < 64);
-        add_totals(r, a, b, ok, t);
+        bool unordered = false;
+        const bool ok = b < a.batch && load_seq(a, b, t, threadIdx.x < 64, unordered);
+        r.items += wave_sum(ok ? items_of(a, t) : 0);
+        add_totals(r, a, b, ok, t, unordered);
     }
     return r;
 }
@@ -280,7 +311,8 @@ __device__ bool find_request(const AttnArgs &a, int64_t w, bool by_token, Seq &s
     for (int b0 = 0; b0 < a.batch; b0 += 64) {
         const int b = b0 + lane;
         Seq t{};
-        const bool ok = b < a.batch && load_seq(a, b, t, false);
+        bool unordered;
+        const bool ok = b < a.batch && load_seq(a, b, t, false, unordered);
         const int n = ok ? items_of(a, t) : 0;
         const int pp = ok && t.ns > 1 ? sat32((int64_t)t.ns * t.P) : 0;
         const int n_in = wave_scan(n), p_in = wave_scan(pp);
@@ -329,41 +361,44 @@ __device__ bool locate_sorted(const AttnArgs &a, int64_t x, const Seq &t, bool l
     // partial-row offsets stay in batch order (the combine kernel's order)
     const int pp = ok && t.ns > 1 ? sat32((int64_t)t.ns * t.P) : 0;
     const int p_excl = wave_scan(pp) - pp;
-    // rank key: keys per group descending, then request index (all distinct)
-    const uint32_t key = ok ? ((uint32_t)((1 << 24) - 1 - t.split_len) << 6) | (uint32_t)lane : 0xffffffffu;
+    // Rank key: keys per group descending, then request index; lanes without
+    // groups behind all others (all keys distinct, so the ranks are a
+    // permutation of the lanes).  One counting pass gives every lane its rank,
+    // two cross-lane moves put the lanes in that order, and prefix sums over
+    // the sorted lanes give each request's first group and first slot.
     const int ng = ok ? a.Hkv * t.ns : 0;                 // this request's groups
-    // groups ahead of this request in longest-first order
-    int off = 0;
-    for (int j = 0; j < a.batch; ++j) {
-        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key, j);
-        const int nj = __builtin_amdgcn_readlane(ng, j);
-        off += kj < key ? nj : 0;
-    }
+    const uint32_t key = ng ? ((uint32_t)((1 << 24) - 1 - t.split_len) << 6) | (uint32_t)lane : 0xffffffc0u | (uint32_t)lane;
+    int rank = 0;
+    for (int j0 = 0; j0 < a.batch; j0 += 8)   // lanes past the batch never count: their keys are the largest
+#pragma unroll
+        for (int j = 0; j < 8; ++j) rank += (uint32_t)__builtin_amdgcn_readlane((int)key, j0 + j) < key ? 1 : 0;
+    if (lane >= a.batch) rank = lane;
+    const int src = __builtin_amdgcn_ds_permute(rank * 4, lane | t.rb << 6);
+    const int s_ng = __builtin_amdgcn_ds_permute(rank * 4, ng);
+    const int s_rb = src >> 6;
+    const int off = wave_scan(s_ng) - s_ng;   // groups ahead of this request in longest-first order
     // its groups dealt to this XCD (g in [off, off + ng), g % nx == xcd), and
     // the slots they take there
     const int nx = a.xcds;
-    const int xcd = (int)(x % nx);
-    const int k = (int)(x / nx);
-    auto on_xcd = [xcd, nx](int n) { return (n + nx - 1 - xcd) / nx; };   // #g in [0, n) with g % nx == xcd
-    const int slots = ok ? (on_xcd(off + ng) - on_xcd(off)) * t.rb : 0;
-    int start = 0;
-    for (int j = 0; j < a.batch; ++j) {
-        const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key, j);
-        const int sj = __builtin_amdgcn_readlane(slots, j);
-        start += kj < key ? sj : 0;
-    }
+    const int k = a.by_xcds.div((int)x);
+    const int xcd = (int)x - k * nx;
+    auto on_xcd = [&](int n) { return a.by_xcds.div(n + nx - 1 - xcd); };   // #g in [0, n) with g % nx == xcd
+    const int slots = s_ng ? (on_xcd(off + s_ng) - on_xcd(off)) * s_rb : 0;
+    const int start = wave_scan(slots) - slots;
     const uint64_t hit = __ballot(slots > 0 && k >= start && k < start + slots);
     if (!hit) return false;
-    const int b = __builtin_amdgcn_readfirstlane(__builtin_ctzll(hit));
+    const int pos = __builtin_amdgcn_readfirstlane(__builtin_ctzll(hit));
+    const int b = bcast(src, pos) & 63;
     s = shfl_seq(t, b);
     s.part_off = bcast(p_excl, b);
-    const int kk = k - bcast(start, b);
-    const int off_b = bcast(off, b);
-    const int g = off_b + ((xcd - off_b) % nx + nx) % nx + nx * (kk / s.rb);   // the (kk / rb)-th of its groups here
+    const int kk = k - bcast(start, pos);
+    const int off_b = bcast(off, pos);
+    const int nth = udiv(kk, s.rb);
+    const int g = xcd + nx * (on_xcd(off_b) + nth);   // the nth of its groups here
     const int local = g - off_b;
-    h = local / s.ns;
-    split = local % s.ns;
-    rblk = kk % s.rb;
+    h = udiv(local, s.ns);
+    split = local - h * s.ns;
+    rblk = kk - nth * s.rb;
     return true;
 }
 
@@ -629,9 +664,10 @@ __device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *s
         // one round of metadata loads serves the totals and the schedule
         const int lane = threadIdx.x & 63;
         Seq t{};
-        const bool ok = lane < a.batch && load_seq(a, lane, t, threadIdx.x < 64);
+        bool unordered = false;
+        const bool ok = lane < a.batch && load_seq(a, lane, t, threadIdx.x < 64, unordered);
         BatchTotals tot{0, 0, 0, false, false};
-        add_totals(tot, a, lane, ok, t);
+        add_totals(tot, a, lane, ok, t, unordered);
         if (!batch_prologue(a, tot)) return false;
         int base, cost, tiles;
         const SkPlan pl = SK ? sk_plan(a, t, ok, base, cost, tiles) : SkPlan{false, 0, 0};
@@ -743,8 +779,9 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     auto load_q = [&](const Unit &w) __attribute__((always_inline)) {
         const int r = w.rb * ROWS + wave * 32 + l32;
         const bool valid = r < w.sq.P * a.G;
-        const int tok = w.sq.q0 + (valid ? r / a.G : 0);
-        const int head = w.h * a.G + (valid ? r % a.G : 0);
+        const int ti = valid ? a.by_G.div(r) : 0;
+        const int tok = w.sq.q0 + ti;
+        const int head = w.h * a.G + (valid ? r - ti * a.G : 0);
         const uint16_t *src = qp + (int64_t)tok * a.q_tok + (int64_t)head * a.q_head + g * 8;
 #pragma unroll
         for (int ds = 0; ds < DSTEPS; ++ds)
@@ -813,8 +850,9 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     const int r = rb * ROWS + wave * 32 + l32;     // this lane's query row
     const bool active = rb * ROWS + wave * 32 < rows;
     const bool qvalid = r < rows;
-    const int qtok = sq.q0 + (qvalid ? r / a.G : 0);
-    const int qhead = h * a.G + (qvalid ? r % a.G : 0);
+    const int qi = qvalid ? a.by_G.div(r) : 0;
+    const int qtok = sq.q0 + qi;
+    const int qhead = h * a.G + (qvalid ? r - qi * a.G : 0);
     const KvView<uint16_t> kv(a.kv, sq, h);
     if (!kPrefetchNext && !first_seg) {
         load_q(wu);
@@ -1181,8 +1219,9 @@ void tree_attn_f32_kernel(AttnArgs a) {
     const int r = rb * ROWS + wave * 32 + l32;
     const bool active = rb * ROWS + wave * 32 < rows;
     const bool qvalid = r < rows;
-    const int qtok = sq.q0 + (qvalid ? r / a.G : 0);
-    const int qhead = h * a.G + (qvalid ? r % a.G : 0);
+    const int qi = qvalid ? a.by_G.div(r) : 0;
+    const int qtok = sq.q0 + qi;
+    const int qhead = h * a.G + (qvalid ? r - qi * a.G : 0);
     const KvView<float> kv(a.kv, sq, h);
 
     // Q operand: head-dim elements [DH*g, DH*g + DH) of this lane's query
@@ -1579,9 +1618,10 @@ __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnArgs a) {
         // one round of metadata loads: the totals and the request of tok
         const int lane = threadIdx.x & 63;
         Seq t{};
-        const bool ok = lane < a.batch && load_seq(a, lane, t, false);
+        bool unordered = false;
+        const bool ok = lane < a.batch && load_seq(a, lane, t, false, unordered);
         BatchTotals tot{0, 0, 0, false, false};
-        add_totals(tot, a, lane, ok, t);
+        add_totals(tot, a, lane, ok, t, unordered);
         if (rejected(tot)) return;
         const int pp = ok && t.ns > 1 ? sat32((int64_t)t.ns * t.P) : 0;
         const int p_excl = wave_scan(pp) - pp;
@@ -2114,10 +2154,15 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     a.scale_log2 = sm_scale * kLog2e;
     a.status = status;
     a.max_rows = max_rows;
+    a.xcds = device_topology().xcds;
+    a.by_xcds = fast_div((uint32_t)a.xcds);
+    a.by_G = fast_div((uint32_t)a.G);
 
     if (!mfma) {
         a.chunk = kNoSplit;
+        a.by_chunk = fast_div((uint32_t)a.chunk);
         a.rows_wg = 16;
+        a.rows_shift = 4;
         const int64_t items = (int64_t)num_kv_heads * (((int64_t)total_q * a.G + 15) / 16 + batch);
         if (!(stages & kStageAttn)) return CAST_OK;
         const bool wide = head_dim > 128;
@@ -2139,6 +2184,8 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     const int waves = waves_for(total_q, a.G, dtype, head_dim);
     a.rows_wg = waves * 32;
     a.chunk = resolve_chunk(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, dtype, kv_split);
+    a.rows_shift = __builtin_ctz((unsigned)a.rows_wg);
+    a.by_chunk = fast_div((uint32_t)a.chunk);
     const SkHost sk = sk_host(batch, total_q, a.G, head_dim, dtype, kv_split, a.chunk);
     a.sk_mode = sk.mode;
     a.sk_wgs = sk.mode ? sk.wgs : 0;
@@ -2166,7 +2213,6 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     const int64_t rbmax = (pmax * a.G + a.rows_wg - 1) / a.rows_wg;
     const int64_t nsplit = a.chunk == kNoSplit ? batch : ((int64_t)total_kv + a.chunk - 1) / a.chunk + batch;
     int64_t items = (int64_t)num_kv_heads * rbmax * nsplit;
-    a.xcds = device_topology().xcds;
     items = batch <= 64 ? sorted_slots((int64_t)num_kv_heads * nsplit, rbmax, a.xcds)
                         : (items + a.xcds - 1) / a.xcds * a.xcds;
     if (a.sk_mode && items < a.sk_wgs) items = a.sk_wgs;
