@@ -95,7 +95,10 @@ struct AttnArgs {
     int32_t D, esz;     // head dim, bytes per element of q/out
     int64_t q_tok, q_head, o_tok, o_head;
     float scale_log2;   // sm_scale * log2(e)
-    int32_t chunk;      // keys per split, multiple of 64 (kNoSplit = no split)
+    int32_t chunk;      // keys per split, multiple of 64 (kNoSplit = no split); with slots > 0 the smallest
+    int32_t slots;      // > 0: the kernels choose the split from the batch's lengths (auto_split) for this
+                        // many workgroups, the number the device holds at once
+    float hkv_per_slot; // Hkv / slots
     int32_t max_rows;   // longest key source (rows) the MFMA kernel can address
     int32_t xcds;       // XCDs of the device: workgroup x runs on XCD x % xcds
     int32_t sk_mode;    // stream-K schedule asked for (CAST_SPLIT_STREAM)
@@ -261,6 +264,48 @@ __device__ __forceinline__ bool batch_fits(const AttnArgs &a, const BatchTotals 
         return false;
     }
     return true;
+}
+
+// The split of a batch of up to 64 requests, chosen from its lengths: lane j
+// holds request j (t; ok when it passed load_seq) and gets its ns and
+// split_len.  Every workgroup of the attention and combine kernels calls it
+// (at least 4 waves; fit: LDS) and finds the same split.
+//
+// With W = sum over the requests of row blocks x 64-key tiles, L = W * Hkv /
+// slots tiles is what each of the workgroups resident at once would get of an
+// even share.  A split of c tiles gives Hkv * sum rb * ceil(tiles / c) items;
+// the smallest c of L * {8, 9, 10, 12} / 8 whose items fit the slots is taken,
+// so that all items start at once and none is longer than it need be; one item
+// too many would wait for a whole other one.  When none fits (many short
+// requests beside long ones) 10/8 L: the longest-first order then fills the
+// second round with the short ones.  Waves 0..3 try one candidate each.
+// Splits below 8 tiles only where 8 would make fewer than 192 items: a split
+// costs a prologue and a partial of the block's rows written and read again
+// (8 requests of 300 to 2k keys: 32.4 us at 4 tiles, 28.1 at 7, 29.7 at 10).
+// Measured, bf16, against one chunk from the batch's averages: 8 requests of
+// 1k to 8k keys, D = 128, 83.6 -> 70.9 us; 32 requests of 300 to 4k keys with
+// packs of 2 to 64 148.9 -> 95.2 us (with 4-wave workgroups, see waves_for);
+// 8 requests of 4k to 8k keys at D = 256 282.6 -> 224.7 us.
+__device__ void auto_split(const AttnArgs &a, Seq &t, bool ok, int *fit) {
+    const int tiles = ok && t.P > 0 ? (int)(((uint32_t)t.T + 63) >> 6) : 0;
+    const int rb = tiles ? t.rb : 0;
+    const int W = wave_sum(tiles * rb);   // the host keeps it below 2^31
+    const int64_t total = (int64_t)W * a.Hkv;
+    int L = max((int)((float)W * a.hkv_per_slot) - 1, 1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) L += (int64_t)L * a.slots < total ? 1 : 0;   // the exact ceiling
+    L = max(L, total < 8 * 192 ? max((int)total / 192, a.chunk >> 6) : 8);
+    auto cand = [&](int w) { return (L * (w < 3 ? 8 + w : 12) + 7) >> 3; };
+    const int w = threadIdx.x >> 6;
+    if (w < 4) {
+        const int c = cand(w);
+        const int n = wave_sum(tiles ? rb * udiv(tiles + c - 1, c) : 0);
+        if ((threadIdx.x & 63) == 0) fit[w] = (int64_t)n * a.Hkv <= a.slots;
+    }
+    __syncthreads();
+    const int c = cand(fit[0] ? 0 : fit[1] ? 1 : fit[2] ? 2 : fit[3] ? 3 : 2);
+    t.ns = tiles ? udiv(tiles + c - 1, c) : 0;
+    t.split_len = tiles ? udiv(tiles + t.ns - 1, t.ns) * 64 : 0;
 }
 
 __device__ bool find_request(const AttnArgs &a, int64_t w, bool by_token, Seq &s, int &local);
@@ -654,9 +699,10 @@ __device__ bool sk_next_segment(const AttnArgs &a, WorkCursor &cur, Unit &u, con
 // up to 64 requests take the stream-K lanes when the caller asked for them
 // and sk_plan accepts the batch, else the longest-first schedule; larger
 // ones take items in batch order, consecutive items (the row blocks of one
-// key split) on one XCD so that they share its L2.  skr: LDS for the stream-K table (64 entries).
+// key split) on one XCD so that they share its L2.  skr: LDS for the stream-K
+// table (64 entries); fit: LDS of auto_split (4 ints).
 template <bool SK>   // SK: the kernel instance takes the stream-K schedule when the plan asks
-__device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *skr) {
+__device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *skr, int *fit) {
     cur.sk = false;
     Seq &sq = u.sq;
     int h = 0, split = 0, rb = 0;
@@ -687,6 +733,7 @@ __device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *s
             cur.end = min(cur.p + pl.L, (int64_t)pl.C);
             return sk_next_segment(a, cur, u, skr);
         }
+        if (!SK && a.slots) auto_split(a, t, ok, fit);
         if (!locate_sorted(a, blockIdx.x, t, ok, sq, h, split, rb)) return false;
     } else {
         const BatchTotals tot = batch_totals(a);
@@ -725,10 +772,7 @@ __device__ __forceinline__ bool next_unit(const AttnArgs &a, WorkCursor &cur, Un
 // WPE: waves per SIMD the register budget is sized for.  2 (256 registers a
 // lane) for head_dim 64 and 128; 1 (512) for head_dim 256, whose O^T
 // accumulators (128 registers), Q^T operand (64), scores and staged K/V
-// tiles take about 330, and for the 2-wave head_dim-128 instance, whose 128
-// threads each stage four times the 8-wave instance's share of a K tile
-// (about 330 registers): its 72 KB of LDS allow two such workgroups per
-// CU, one wave per SIMD, either way.
+// tiles take about 330.
 // SKI: the stream-K instance (a run of segments per workgroup, the next
 // segment's first tile and Q loaded during a segment's last tile); the
 // static instances do one unit each.
@@ -756,7 +800,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t Ks[NBUF][BN * KPAD];
     __shared__ __attribute__((aligned(16))) uint16_t Vt[NBUF][D * VPAD];
     __shared__ EpiArgs epi;
-    __shared__ int pack_hi[WAVES];   // per wave: the last pack key a row of it sees
+    __shared__ int pack_hi[WAVES];   // auto_split's LDS, then per wave the last pack key a row of it sees
     // Head dim 256 (one wave per SIMD, no registers to spare) has no
     // stream-K instance.
     constexpr bool kStreamK = SKI && D <= 128;
@@ -765,7 +809,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     // ---- this workgroup's work: one unit, or a run of stream-K segments
     Unit wu;
     WorkCursor cur;
-    if (!first_unit<kStreamK>(a, cur, wu, skr)) return;
+    if (!first_unit<kStreamK>(a, cur, wu, skr, pack_hi)) return;
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
@@ -1201,12 +1245,12 @@ void tree_attn_f32_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) float Ks[2][BN * KPAD];
     __shared__ __attribute__((aligned(16))) float Vs[2][BN * KPAD];
     __shared__ EpiArgs epi;
-    __shared__ int pack_hi[WAVES];   // per wave: the last pack key a row of it sees
+    __shared__ int pack_hi[WAVES];   // auto_split's LDS, then per wave the last pack key a row of it sees
     __shared__ SkReq skr[SKI ? 64 : 1];
 
     Unit wu;
     WorkCursor cur;
-    if (!first_unit<SKI>(a, cur, wu, skr)) return;
+    if (!first_unit<SKI>(a, cur, wu, skr, pack_hi)) return;
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
@@ -1511,6 +1555,7 @@ void tree_attn_f32_kernel(AttnArgs a) {
 // per head max and sum; the stream-K instance adds each piece's partial row
 // and each head's piece count.
 struct CombineLds {
+    int fit[4];   // auto_split
     float wgt[kCombineLdsHeads * kCombineLdsSplits];
     float hm[kCombineLdsHeads], hl[kCombineLdsHeads];
 };
@@ -1623,6 +1668,7 @@ __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnArgs a) {
         BatchTotals tot{0, 0, 0, false, false};
         add_totals(tot, a, lane, ok, t, unordered);
         if (rejected(tot)) return;
+        if (!SKI && a.slots) auto_split(a, t, ok, sm.fit);
         const int pp = ok && t.ns > 1 ? sat32((int64_t)t.ns * t.P) : 0;
         const int p_excl = wave_scan(pp) - pp;
         int base = 0, cost = 0, tiles = 0;
@@ -1914,28 +1960,39 @@ static bool mfma_path(int32_t dtype, int32_t D) {
     return (dtype == CAST_BF16 || dtype == CAST_FP16) && (D == 64 || D == 128 || D == 256);
 }
 
-// Waves per workgroup (32 query rows each) for the largest possible pack.
-// (The fp32 kernel has no 2-wave instance: its staging registers would not
-// fit beside the Q and O operands.)
+// Waves per workgroup (32 query rows each).  16-bit inputs take 8 waves (256
+// rows, one workgroup per CU) when the average pack fills most of them, else 4
+// (128 rows, two workgroups per CU at head dim 128, three at 64): with few
+// rows a tile's time is the latency of one wave's QK -> softmax -> PV chain
+// (3,700 cycles for 32 KB), and two workgroups have twice the loads in
+// flight.  Best split of each, 4 against 8 waves, us: 32 requests of 132
+// rows 104 against 114, 16 of 96 rows 84 against 108, 32 of 20 rows 90
+// against 117; 8 of 256 rows 92 against 85, one of 512 rows 111 against 95.
+// 2 waves (64 rows) were slower than 4 even at 64 rows (one request, 2064
+// keys: 17.5 against 16.4): each thread stages twice as much.
+// fp32 sizes by the largest possible pack (one workgroup per CU either way).
 // Head_dim 256 always runs 4 waves, one per SIMD: fewer threads would each
 // stage more of its 32 KB tiles than the registers hold.
-static int waves_for(int32_t total_q, int32_t G, int32_t dtype, int32_t D) {
-    const int pmax = total_q < kMaxPack ? total_q : kMaxPack;
-    const int rows = pmax * G;
+static int waves_for(int32_t batch, int32_t total_q, int32_t G, int32_t dtype, int32_t D) {
     if (D == 256) return 4;
-    const int w = rows <= 64 ? 2 : rows <= 128 ? 4 : 8;
-    return dtype == CAST_FP32 && w < 4 ? 4 : w;
+    if (dtype == CAST_FP32) return (int64_t)(total_q < kMaxPack ? total_q : kMaxPack) * G <= 128 ? 4 : 8;
+    const int64_t p_avg = ((int64_t)total_q + batch - 1) / batch;
+    return (p_avg < kMaxPack ? p_avg : kMaxPack) * G <= 192 ? 4 : 8;
 }
 
+// The split-K chunk from the batch's averages: what kv_split = 0 means for
+// batches above 64 requests, and for smaller ones whether a call without
+// workspace is refused (below, the kernels choose the chunk themselves).
 static int32_t resolve_chunk(int32_t batch, int32_t total_q, int32_t total_kv, int32_t Hq, int32_t Hkv,
                              int32_t D, int32_t dtype, int32_t kv_split) {
     if (!mfma_path(dtype, D) || kv_split < 0 || batch <= 0) return kNoSplit;
     if (kv_split > 0) return ((kv_split + 63) / 64) * 64;
-    const int G = Hq / Hkv;
-    const int rows_wg = waves_for(total_q, G, dtype, D) * 32;
+    const int64_t pmax = total_q < kMaxPack ? total_q : kMaxPack;
+    const int64_t rows = pmax * (Hq / Hkv);
+    const int rows_wg = D == 256 ? 128 : rows <= 64 && dtype != CAST_FP32 ? 64 : rows <= 128 ? 128 : 256;
     const int64_t p_avg = (total_q + batch - 1) / batch;
     const int64_t p_est = p_avg < kMaxPack ? p_avg : kMaxPack;
-    const int64_t rb = (p_est * G + rows_wg - 1) / rows_wg;
+    const int64_t rb = (p_est * (Hq / Hkv) + rows_wg - 1) / rows_wg;
     const int64_t units = (int64_t)Hkv * batch * (rb > 0 ? rb : 1);
     const int64_t t_avg = (total_kv + batch - 1) / batch;
     const int cus = device_topology().cus;
@@ -1985,14 +2042,11 @@ static AttnKernel attn_kernel_of(int32_t dtype, int32_t D, int waves, bool store
     }
     const bool f16 = dtype == CAST_FP16;
     if (D == 128) {
-        if (waves == 2) return mfma_instance<128, 2, 1, SKI>(f16, store);
         return waves == 4 ? mfma_instance<128, 4, 2, SKI>(f16, store) : mfma_instance<128, 8, 2, SKI>(f16, store);
     }
-    if (waves == 2) return mfma_instance<64, 2, 2, SKI>(f16, store);
     return waves == 4 ? mfma_instance<64, 4, 2, SKI>(f16, store) : mfma_instance<64, 8, 2, SKI>(f16, store);
 }
-// Head dims 64 and 128 run 2, 4 or 8 waves (bf16 / fp16) or 4 or 8 (fp32);
-// head dim 256 runs 4 (static schedule only).  WPE (waves per
+// Head dims 64 and 128 run 4 or 8 waves; head dim 256 runs 4 (static schedule only).  WPE (waves per
 // SIMD of the register budget) as the kernels' comments give it; sk picks
 // the stream-K instance.
 static AttnKernel attn_kernel(int32_t dtype, int32_t D, int waves, bool store, bool sk) {
@@ -2032,13 +2086,12 @@ static int resident_per_cu(const AttnKernel &k) {
 struct SkHost {
     int mode, wgs, rows_wg;
 };
-static SkHost sk_host(int32_t batch, int32_t total_q, int32_t G, int32_t D, int32_t dtype, int32_t kv_split,
-                      int32_t chunk) {
+static SkHost sk_host(int32_t batch, int32_t total_q, int32_t G, int32_t D, int32_t dtype, int32_t kv_split) {
     SkHost h{0, 0, 0};
     if (!mfma_path(dtype, D) || D > 128 || batch <= 0 || batch > 64) return h;
     if (kv_split != kSplitStreamK) return h;
     h.mode = 1;
-    const int waves = waves_for(total_q, G, dtype, D);
+    const int waves = waves_for(batch, total_q, G, dtype, D);
     const Topology topo = device_topology();
     const int per = resident_per_cu(attn_kernel(dtype, D, waves, false, true));
     const int step = 2 * topo.xcds;
@@ -2053,6 +2106,72 @@ static size_t sk_bytes(const SkHost &h, int32_t D) {
     if (!h.mode) return 0;
     const size_t rows = (size_t)2 * h.wgs * h.rows_wg;
     return align256(rows * D * sizeof(float)) + align256(rows * sizeof(float));
+}
+
+// How a call splits its keys, from the host-known sizes.
+struct SplitPlan {
+    int32_t chunk;       // keys per split (the smallest one when slots > 0), or kNoSplit
+    int32_t slots;       // > 0: auto_split chooses on the device
+    bool optional;       // runs unsplit without a workspace
+    int64_t part_rows;   // partial rows the split can write
+    int64_t wg_bound;    // workgroups the split can need (0: the general bound)
+};
+
+// kv_split = 0 (or the chunk that cast_tree_attn_default_split names for it)
+// and up to 64 requests: the device chooses.  Not worth the
+// combine launch where the rows alone fill the device one and a half times
+// (the longest-first order balances those), or where the averages ask for no
+// split and prefixes are short; and with one chunk of kMinChunk keys when even
+// that cannot give more items than the device holds (single-p16).
+//
+// Bounds of auto_split's result, with c >= L = W * Hkv / slots tiles per split
+// and RB = total_q * G / rows_wg + batch >= sum rb: items = Hkv * sum rb *
+// ceil(tiles / c) <= slots + Hkv * RB; an XCD takes at most ceil(groups / nx)
+// groups of each request, so its slots are at most items / nx + RB; a request
+// in ns > 1 splits has ns - 1 < tiles / c and P <= rb * rows_wg / G, so the
+// partial rows sum to less than rows_wg * slots / Hq plus the rows of the
+// split requests, which are at most that many again.
+static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, int32_t Hq, int32_t Hkv, int32_t D,
+                            int32_t dtype, int32_t kv_split) {
+    SplitPlan p{};
+    p.chunk = resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, kv_split);
+    const bool automatic =
+        kv_split == 0 || kv_split == resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, 0);
+    if (automatic && batch > 0 && batch <= 64 && mfma_path(dtype, D) && dtype != CAST_FP32) {
+        const int64_t G = Hq / Hkv;
+        const int waves = waves_for(batch, total_q, (int32_t)G, dtype, D);
+        const int64_t rows_wg = waves * 32;
+        const Topology topo = device_topology();
+        const int64_t slots = (int64_t)topo.cus * resident_per_cu(attn_kernel(dtype, D, waves, false, false));
+        const int64_t pmax = total_q < kMaxPack ? total_q : kMaxPack;
+        const int64_t rbmax = (pmax * G + rows_wg - 1) / rows_wg;
+        const int64_t t_avg = (total_kv + batch - 1) / batch;
+        const bool full = 2 * (Hkv * total_q * G / rows_wg) >= 3 * slots || (int64_t)Hkv * batch >= 2 * slots;
+        if (full || (p.chunk == kNoSplit && t_avg <= 512) || total_kv <= kMinChunk || rbmax > 32) {
+            if (p.chunk != kNoSplit) p.part_rows = part_rows_bound(total_q, total_kv, p.chunk);
+            return p;
+        }
+        p.optional = p.chunk == kNoSplit;
+        p.chunk = kMinChunk;
+        p.part_rows = part_rows_bound(total_q, total_kv, p.chunk);
+        if ((int64_t)Hkv * rbmax * ((int64_t)total_kv / kMinChunk + batch) > slots) {
+            p.slots = (int32_t)slots;
+            const int64_t rb_sum = total_q * G / rows_wg + batch;
+            const int64_t once = (rows_wg * slots + Hq - 1) / Hq;
+            const int64_t rows = once + (once < total_q ? once : total_q);
+            if (rows < p.part_rows) p.part_rows = rows;
+            p.wg_bound = topo.xcds * ((slots + Hkv * rb_sum + topo.xcds - 1) / topo.xcds + rb_sum);
+        }
+        return p;
+    }
+    if (p.chunk != kNoSplit) p.part_rows = part_rows_bound(total_q, total_kv, p.chunk);
+    return p;
+}
+
+// Bytes of the split-K partials: O [part_rows][Hq][D], then lse [part_rows][Hq].
+static size_t split_bytes(const SplitPlan &p, int32_t Hq, int32_t D) {
+    if (p.chunk == kNoSplit) return 0;
+    return align256((size_t)p.part_rows * Hq * D * sizeof(float)) + align256((size_t)p.part_rows * Hq * sizeof(float));
 }
 
 }  // namespace cast
@@ -2071,15 +2190,9 @@ extern "C" size_t cast_tree_attn_workspace_size(int32_t batch, int32_t total_q, 
                                                 int32_t num_q_heads, int32_t num_kv_heads,
                                                 int32_t head_dim, int32_t dtype, int32_t kv_split) {
     if (batch <= 0 || total_q <= 0 || num_kv_heads <= 0 || num_q_heads % num_kv_heads) return 0;
-    const int32_t chunk = resolve_chunk(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim,
-                                        dtype, kv_split);
-    size_t bytes = 0;
-    if (chunk != kNoSplit) {
-        const int64_t rows = part_rows_bound(total_q, total_kv, chunk);
-        bytes = align256((size_t)rows * num_q_heads * head_dim * sizeof(float)) +
-                align256((size_t)rows * num_q_heads * sizeof(float));
-    }
-    const SkHost sk = sk_host(batch, total_q, num_q_heads / num_kv_heads, head_dim, dtype, kv_split, chunk);
+    const SplitPlan sp = split_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, dtype, kv_split);
+    const size_t bytes = split_bytes(sp, num_q_heads, head_dim);
+    const SkHost sk = sk_host(batch, total_q, num_q_heads / num_kv_heads, head_dim, dtype, kv_split);
     const size_t skb = sk_bytes(sk, head_dim);
     return skb > bytes ? skb : bytes;
 }
@@ -2181,23 +2294,29 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
         return hipGetLastError() == hipSuccess ? CAST_OK : CAST_ERR_HIP;
     }
 
-    const int waves = waves_for(total_q, a.G, dtype, head_dim);
+    const int waves = waves_for(batch, total_q, a.G, dtype, head_dim);
     a.rows_wg = waves * 32;
-    a.chunk = resolve_chunk(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, dtype, kv_split);
     a.rows_shift = __builtin_ctz((unsigned)a.rows_wg);
-    a.by_chunk = fast_div((uint32_t)a.chunk);
-    const SkHost sk = sk_host(batch, total_q, a.G, head_dim, dtype, kv_split, a.chunk);
+    SplitPlan sp = split_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, dtype, kv_split);
+    const SkHost sk = sk_host(batch, total_q, a.G, head_dim, dtype, kv_split);
     a.sk_mode = sk.mode;
     a.sk_wgs = sk.mode ? sk.wgs : 0;
     a.sk_min_tiles = kMinChunk / 64;
+    const size_t split_need = split_bytes(sp, num_q_heads, head_dim);
+    if (sp.optional && (!workspace || workspace_bytes < split_need || (reinterpret_cast<uintptr_t>(workspace) & 255)))
+        sp = SplitPlan{kNoSplit, 0, false, 0, 0};
+    a.chunk = sp.chunk;
+    a.by_chunk = fast_div((uint32_t)a.chunk);
+    a.slots = sp.slots;
+    a.hkv_per_slot = sp.slots ? (float)num_kv_heads / (float)sp.slots : 0.f;
     if (a.chunk != kNoSplit || sk.mode) {
-        const size_t need = cast_tree_attn_workspace_size(batch, total_q, total_kv, num_q_heads, num_kv_heads,
-                                                          head_dim, dtype, kv_split);
+        const size_t skb = sk_bytes(sk, head_dim);
+        const size_t need = skb > split_need ? skb : split_need;
         if (!workspace || workspace_bytes < need) return CAST_ERR_WORKSPACE;
         if (reinterpret_cast<uintptr_t>(workspace) & 255) return CAST_ERR_ALIGNMENT;
         a.part_o = static_cast<float *>(workspace);
         if (a.chunk != kNoSplit) {
-            a.part_rows = part_rows_bound(total_q, total_kv, a.chunk);
+            a.part_rows = sp.part_rows;
             a.part_lse = reinterpret_cast<float *>(
                 static_cast<char *>(workspace) + align256((size_t)a.part_rows * num_q_heads * head_dim * sizeof(float)));
         }
@@ -2215,6 +2334,7 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     int64_t items = (int64_t)num_kv_heads * rbmax * nsplit;
     items = batch <= 64 ? sorted_slots((int64_t)num_kv_heads * nsplit, rbmax, a.xcds)
                         : (items + a.xcds - 1) / a.xcds * a.xcds;
+    if (sp.wg_bound && sp.wg_bound < items) items = sp.wg_bound;
     if (a.sk_mode && items < a.sk_wgs) items = a.sk_wgs;
     if (items > 0x7fffffff) return CAST_ERR_SHAPE;
     if (stages & kStageAttn) {
@@ -2370,8 +2490,12 @@ extern "C" int cast_tree_attn_fwd_noalloc(const void *q, const void *k, const vo
                                           int64_t k_tok, int64_t k_head, int64_t v_tok, int64_t v_head,
                                           int64_t o_tok, int64_t o_head, int32_t dtype, float sm_scale,
                                           int32_t kv_split, int32_t *status, cast_stream_t stream) {
-    const size_t need = cast_tree_attn_workspace_size(batch, total_q, total_kv, num_q_heads, num_kv_heads,
-                                                      head_dim, dtype, kv_split);
+    // a call whose split is optional runs unsplit and leaves the array alone
+    const bool sized = batch > 0 && total_q > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0;
+    const bool optional = sized && split_plan(batch, total_q, total_kv, num_q_heads, num_kv_heads, head_dim, dtype,
+                                              kv_split).optional;
+    const size_t need = optional ? 0 : cast_tree_attn_workspace_size(batch, total_q, total_kv, num_q_heads,
+                                                                     num_kv_heads, head_dim, dtype, kv_split);
     if (need > cast::kScratchBytes) return CAST_ERR_SCRATCH_LIMIT;
     void *ws = nullptr;
     if (need) {

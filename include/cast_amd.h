@@ -99,15 +99,18 @@ int cast_tree_bitmask(const int32_t *parent, const int32_t *cu_q, int32_t batch,
  *   sm_scale  > 0 (the Python layer substitutes 1/sqrt(D) for None)
  *   kv_split  keys per split-K chunk (multiple of 64); 0 lets the library
  *             choose; CAST_SPLIT_STREAM (-2) asks for the stream-K schedule;
- *             any other negative value disables split-K.  With 0 the library
- *             cuts long prefixes into equal splits so that the work items
- *             cover the device's CUs (static schedule, longest items first).
+ *             any other negative value disables split-K.  With 0 (or the
+ *             value of cast_tree_attn_default_split) long prefixes are cut
+ *             into equal splits so that the work items cover the device once;
+ *             for batches of up to 64 requests the kernels choose the chunk
+ *             from the requests' lengths (static schedule, longest items
+ *             first).
  *             Stream-K (only when asked for): pairs of workgroups on one XCD
  *             get equal ranges of key tiles over all (request, KV head, row
  *             block) units, and a combine merges the pieces of units cut
  *             between workgroups; the pieces' cut points follow the batch
  *             order.  The static schedule sums each request's keys in an
- *             order that only depends on batch totals.
+ *             order that only depends on the batch's lengths.
  *   workspace / workspace_bytes  scratch of at least
  *             cast_tree_attn_workspace_size(...) bytes, 256-byte aligned
  *   status    int32*, nullable device status word
@@ -223,7 +226,9 @@ size_t cast_tree_attn_workspace_size(int32_t batch, int32_t total_q, int32_t tot
                                      int32_t num_q_heads, int32_t num_kv_heads,
                                      int32_t head_dim, int32_t dtype, int32_t kv_split);
 
-/* The split-K chunk (keys) the library would choose for kv_split = 0. */
+/* The split-K chunk (keys) that kv_split = 0 stands for, estimated from the
+ * batch's averages (-1: no split); passing it back as kv_split is the same
+ * as 0. */
 int32_t cast_tree_attn_default_split(int32_t batch, int32_t total_q, int32_t total_kv,
                                      int32_t num_q_heads, int32_t num_kv_heads,
                                      int32_t head_dim, int32_t dtype);
