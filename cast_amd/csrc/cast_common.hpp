@@ -49,6 +49,19 @@ struct Bf16 {
     }
     static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return pack_bf16x2(lo, hi); }
     static __device__ __forceinline__ float widen(uint16_t h) { return bf16_to_float(h); }
+    // a float pair as the sum of kTerms pairs of the format, the largest
+    // first: three truncations of 8 bits each hold all 24 bits
+    static constexpr int kTerms = 3;
+    static constexpr float kTermShift = 0.f;
+    static __device__ __forceinline__ void split2(float lo, float hi, uint32_t (&w)[3]) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            const uint32_t bl = __builtin_bit_cast(uint32_t, lo), bh = __builtin_bit_cast(uint32_t, hi);
+            w[t] = __builtin_amdgcn_perm(bh, bl, 0x07060302u);
+            lo -= __builtin_bit_cast(float, bl & 0xffff0000u);
+            hi -= __builtin_bit_cast(float, bh & 0xffff0000u);
+        }
+    }
 };
 struct Fp16 {
     using vec8 = f16x8;
@@ -57,6 +70,15 @@ struct Fp16 {
     }
     static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return pack_f16x2(lo, hi); }
     static __device__ __forceinline__ float widen(uint16_t h) { return f16_to_float(h); }
+    // two roundings of 11 bits each leave 2^-24 of the value, as float does,
+    // while the second term is a normal half: values of about 1 are scaled by
+    // 2^kTermShift first
+    static constexpr int kTerms = 2;
+    static constexpr float kTermShift = 7.f;
+    static __device__ __forceinline__ void split2(float lo, float hi, uint32_t (&w)[2]) {
+        w[0] = pack_f16x2(lo, hi);
+        w[1] = pack_f16x2(lo - f16_to_float((uint16_t)w[0]), hi - f16_to_float((uint16_t)(w[0] >> 16)));
+    }
 };
 
 __device__ __forceinline__ void raise_flag(int32_t *status, int32_t bit) {

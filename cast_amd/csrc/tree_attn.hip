@@ -18,9 +18,10 @@
 //   S^T accumulator registers (a lane's 16 score values are exactly the 8+8
 //   k-slots it must supply), V^T read from a transposed LDS copy.  fp32
 //   inputs with head_dim 64/128/256 run the same structure on
-//   v_mfma_f32_32x32x2_f32 (tree_attn_f32_kernel); other head dims (up to
-//   256) take a scalar kernel.  Head_dim 256 runs one wave per SIMD (512
-//   registers a lane).
+//   v_mfma_f32_32x32x2_f32 (tree_attn_f32_kernel).  Other head dims
+//   (multiples of 8 up to 256) take padded instances of both, or a scalar
+//   kernel where bases, strides or sizes do not allow those.  Head_dim 256
+//   runs one wave per SIMD (512 registers a lane).
 // K/V tiles of 64 keys (32 for fp32 at head_dim 256) are double-buffered
 // through LDS with 16-byte loads; the ancestor words are only consulted on
 // the tile(s) holding pack keys, and pack tiles past the last key any row
@@ -518,6 +519,56 @@ __device__ __forceinline__ bool block_live(uint64_t w0, uint64_t w1, int j0, int
     return __any(vis != 0u);
 }
 
+template <typename T, typename E>
+__device__ __forceinline__ float load_elem(const T *p) {
+    if constexpr (sizeof(T) == 2)
+        return E::widen(*p);
+    else
+        return *p;
+}
+
+// One query row against keys [k_begin, k_end) in plain fp32, by one wave: the
+// (unnormalised) output element lane + 64 j in acc[j], and the row's running
+// max (base 2) and sum.  For rows whose split products met an infinity or a
+// NaN: a term that is zero there makes a NaN of what a float product keeps.
+template <typename T, typename E>
+__device__ void exact_row(const KvView<T> &kv, int S, int k_begin, int k_end, const T *q, int D, uint64_t w0,
+                          uint64_t w1, float c, float (&acc)[4], float &m, float &l) {
+    const int lane = threadIdx.x & 63;
+    m = -INFINITY;
+    l = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = 0.f;
+    for (int k0 = k_begin; k0 < k_end; k0 += 64) {
+        const int kk = k0 + lane;
+        float s = -INFINITY;
+        if (kk < k_end && (kk < S || pack_bit(kk - S, w0, w1))) {
+            const T *kp = kv.key(kk, S);
+            float dot = 0.f;
+            for (int d = 0; d < D; ++d) dot = fmaf(load_elem<T, E>(q + d), load_elem<T, E>(kp + d), dot);
+            s = dot * c;
+        }
+        float mx = s;
+        for (int off = 32; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+        const float mn = fmaxf(m, mx);
+        const float alpha = mn == -INFINITY ? 1.f : exp2f(m - mn);
+        const float p = exp2f(s - (mn == -INFINITY ? 0.f : mn));
+        float ps = p;
+        for (int off = 32; off; off >>= 1) ps += __shfl_xor(ps, off);
+        l = l * alpha + ps;
+        m = mn;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] *= alpha;
+        for (int i = 0; i < 64 && k0 + i < k_end; ++i) {
+            const float pi = __shfl(p, i);
+            const T *vp = kv.val(k0 + i, S);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (lane + 64 * j < D) acc[j] = fmaf(pi, load_elem<T, E>(vp + lane + 64 * j), acc[j]);
+        }
+    }
+}
+
 // What the MFMA kernel's epilogue needs, parked in LDS during the key loop
 // so that it holds no scalar registers there.
 struct EpiArgs {
@@ -776,10 +827,22 @@ __device__ __forceinline__ bool next_unit(const AttnArgs &a, WorkCursor &cur, Un
 // SKI: the stream-K instance (a run of segments per workgroup, the next
 // segment's first tile and Q loaded during a segment's last tile); the
 // static instances do one unit each.
-template <int D, int WAVES, bool STORE, typename E, int WPE = 2, bool SKI = false>
+// PAD: head dims the instances do not name (multiples of 8 below D): the
+// missing elements of K, V and Q are zeros, and P, which the scalar kernel
+// that ran these dims kept in fp32, goes into the value product as E::kTerms
+// 16-bit terms that add up to it (each V^T operand read then feeds kTerms
+// MFMAs).  A row whose result is not finite is computed again in plain fp32.
+// B = 4, S of 500 to 2000, P of 16 to 64, 32 / 8 heads of 96, fp16: 549 us on
+// the scalar kernel (no split-K, no matrix cores, each key row read by every
+// 16 query rows), 26.4 us here.
+template <int D, int WAVES, bool STORE, typename E, int WPE = 2, bool SKI = false, bool PAD = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void tree_attn_mfma_kernel(AttnArgs a) {
     using vec8 = typename E::vec8;
+    constexpr int PT = PAD ? E::kTerms : 1;            // 16-bit terms of P
+    constexpr float kShift = PAD ? E::kTermShift : 0.f;   // P is scaled by 2^kShift
+    constexpr uint32_t kNowhere = 0x7ffffff0u;         // byte offset past every source: loads as zeros
+    const int dr = PAD ? a.D : D;                      // the call's head dim
     constexpr int NT = WAVES * 64;
     constexpr int BN = 64;                 // keys per tile: two 32-key MFMA blocks
     constexpr int ROWS = WAVES * 32;       // query rows per workgroup
@@ -829,7 +892,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
         const uint16_t *src = qp + (int64_t)tok * a.q_tok + (int64_t)head * a.q_head + g * 8;
 #pragma unroll
         for (int ds = 0; ds < DSTEPS; ++ds)
-            qreg[ds] = valid ? *reinterpret_cast<const vec8 *>(src + ds * 16) : vec8{};
+            qreg[ds] = valid && (!PAD || ds * 16 + g * 8 < dr) ? *reinterpret_cast<const vec8 *>(src + ds * 16) : vec8{};
     };
 
     // ---- global -> register staging of one tile.  Each key source of a
@@ -844,14 +907,15 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     // the tile's first row within that source
     auto fetch_from = [&](const uint16_t *kb, const uint16_t *vb, int rows, uint32_t ksb, uint32_t vsb,
                           uint32_t row0) __attribute__((always_inline)) {
-        const __amdgpu_buffer_rsrc_t krs = seg_rsrc(kb, rows, ksb, D * 2);
-        const __amdgpu_buffer_rsrc_t vrs = seg_rsrc(vb, rows, vsb, D * 2);
+        const __amdgpu_buffer_rsrc_t krs = seg_rsrc(kb, rows, ksb, dr * 2);
+        const __amdgpu_buffer_rsrc_t vrs = seg_rsrc(vb, rows, vsb, dr * 2);
 #pragma unroll
         for (int it = 0; it < K_PER_T; ++it) {
             const int cidx = tid + it * NT;
             if (cidx >= KCH) break;
             const int key = cidx / (D / 8), dch = cidx % (D / 8);
-            kst[it] = load16(krs, __umul24(row0 + key, ksb) + dch * 16);
+            const uint32_t off = __umul24(row0 + key, ksb) + dch * 16;
+            kst[it] = load16(krs, PAD && dch * 8 >= dr ? kNowhere : off);
         }
 #pragma unroll
         for (int it = 0; it < V_PER_T; ++it) {
@@ -862,7 +926,9 @@ void tree_attn_mfma_kernel(AttnArgs a) {
             const uint32_t v0 = row0 + 16 * (oc >> 1) + 4 * (oc & 1);
 #pragma unroll
             for (int i = 0; i < 8; ++i)
-                vst[it][i] = load16(vrs, __umul24(v0 + 8 * (i >> 2) + (i & 3), vsb) + dch * 16);
+                vst[it][i] = load16(vrs, PAD && dch * 8 >= dr
+                                             ? kNowhere
+                                             : __umul24(v0 + 8 * (i >> 2) + (i & 3), vsb) + dch * 16);
         }
     };
     // the tile of keys [t0, t0 + 64) of (request q, head view v): its source
@@ -1015,7 +1081,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
         __builtin_amdgcn_sched_group_barrier(0x008, kQkAhead, 0);
     };
     // visibility, the online softmax in base 2 and the P^T operand of tile t
-    auto softmax = [&](int t, floatx16 (&s)[2], vec8 (&pb)[2][2]) __attribute__((always_inline)) {
+    auto softmax = [&](int t, floatx16 (&s)[2], vec8 (&pb)[PT][2][2]) __attribute__((always_inline)) {
         // visibility (pack tiles and partial tiles only).  Element e of
         // lane (l32, g) in block kb is key t0 + 32*kb + 4*g + off(e),
         // off(e) = 8*(e/4) + e%4; in a pack tile that is pack key t0 - S + ...
@@ -1053,7 +1119,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
 #pragma unroll
             for (int db = 0; db < DB; ++db) o[db] *= alpha;
             m = mn;
-            msafe = m == -INFINITY ? 0.f : m;
+            msafe = m == -INFINITY ? 0.f : m - kShift;
         }
         float acc = 0.f;
 #pragma unroll
@@ -1066,10 +1132,21 @@ void tree_attn_mfma_kernel(AttnArgs a) {
             }
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
-                u32x4 w;
+                u32x4 w[PT];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) w[e] = E::pack2(p[hf * 8 + 2 * e], p[hf * 8 + 2 * e + 1]);
-                pb[kb][hf] = __builtin_bit_cast(vec8, w);
+                for (int e = 0; e < 4; ++e) {
+                    const float p0 = p[hf * 8 + 2 * e], p1 = p[hf * 8 + 2 * e + 1];
+                    if constexpr (PAD) {
+                        uint32_t x[PT];
+                        E::split2(p0, p1, x);
+#pragma unroll
+                        for (int i = 0; i < PT; ++i) w[i][e] = x[i];
+                    } else {
+                        w[0][e] = E::pack2(p0, p1);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < PT; ++i) pb[i][kb][hf] = __builtin_bit_cast(vec8, w[i]);
             }
         }
         lsum += acc;
@@ -1077,7 +1154,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     // O^T += V^T P^T over four 16-key slices.  Slot j of lane group g in
     // slice (kb, hf) is key 32*kb + 16*hf + 8*(j/4) + 4*g + j%4, stored at
     // column 32*kb + 16*hf + 8*g + j.
-    auto pv = [&](int buf, const vec8 (&pb)[2][2]) __attribute__((always_inline)) {
+    auto pv = [&](int buf, const vec8 (&pb)[PT][2][2]) __attribute__((always_inline)) {
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
@@ -1086,22 +1163,23 @@ void tree_attn_mfma_kernel(AttnArgs a) {
                 for (int db = 0; db < DB; ++db) {
                     const vec8 va = *reinterpret_cast<const vec8 *>(
                         &Vt[buf][(db * 32 + l32) * VPAD + kb * 32 + hf * 16 + g * 8]);
-                    o[db] = E::mma(va, pb[kb][hf], o[db]);
+#pragma unroll
+                    for (int i = PT - 1; i >= 0; --i) o[db] = E::mma(va, pb[i][kb][hf], o[db]);
                 }
         // the same for the V^T operand reads of the PV product; the
         // exponentials stay free to fill the gaps
         __builtin_amdgcn_sched_group_barrier(0x100, kQkAhead, 1);
 #pragma unroll
         for (int i = 0; i < 4 * DB - kQkAhead; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+            __builtin_amdgcn_sched_group_barrier(0x008, PT, 1);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, kQkAhead, 1);
+        __builtin_amdgcn_sched_group_barrier(0x008, kQkAhead * PT, 1);
     };
 
     auto tile_body = [&](int t, int buf) __attribute__((always_inline)) {
         floatx16 s[2];
-        vec8 pb[2][2];
+        vec8 pb[PT][2][2];
         qk(buf, s);
         softmax(t, s, pb);
         pv(buf, pb);
@@ -1160,32 +1238,77 @@ void tree_attn_mfma_kernel(AttnArgs a) {
         const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
         const float lse2 = ltot > 0.f ? msafe + log2f(ltot) : -INFINITY;
         const EpiArgs e = epi;
-        if (qvalid && e.final_out) {
+        // static split: row (token, head) of the partial rows; stream-K:
+        // row wave * 32 + l32 of the workgroup's slot
+        const int64_t prow = e.slot >= 0 ? (int64_t)e.slot * ROWS + wave * 32 + l32 : e.prow0 + qtok;
+        bool store_row = qvalid;
+        if constexpr (PAD) {
+            // NaN as soon as one of the row's sums is not finite
+            float z = ltot * 0.f;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
+            const uint64_t bad = __ballot(qvalid && !(z == 0.f));
+            const uint32_t redo = (uint32_t)bad | (uint32_t)(bad >> 32);
+            store_row = qvalid && !(redo >> l32 & 1);
+            for (uint32_t left = redo; left; left &= left - 1) {
+                const int i = __builtin_ctz(left);
+                const int tok = bcast(qtok, i), head = bcast(qhead, i);
+                const int64_t row = bcast64(prow, i);
+                const uint64_t w0 = (uint64_t)bcast64((int64_t)mw0, i), w1 = (uint64_t)bcast64((int64_t)mw1, i);
+                float acc[4], mr, lr;
+                exact_row<uint16_t, E>(kv, sq.S, k_begin, k_end, qp + (int64_t)tok * a.q_tok + (int64_t)head * a.q_head,
+                                       dr, w0, w1, c, acc, mr, lr);
+                const float ir = lr > 0.f ? 1.f / lr : 0.f;
+                const float l2 = lr > 0.f ? (mr == -INFINITY ? 0.f : mr) + log2f(lr) : -INFINITY;
+                if (!e.final_out && row >= e.part_rows) {
+                    raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
+                    continue;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int d = lane + 64 * j;
+                    if (d >= dr) break;
+                    if (e.final_out)
+                        static_cast<uint16_t *>(e.out)[(int64_t)tok * e.o_tok + (int64_t)head * e.o_head + d] =
+                            (uint16_t)E::pack2(acc[j] * ir, 0.f);
+                    else
+                        e.part_o[(row * e.Hq + head) * dr + d] = acc[j] * ir;
+                }
+                if (lane == 0) {
+                    if (!e.final_out)
+                        e.part_lse[row * e.Hq + head] = l2;
+                    else if (e.lse)
+                        e.lse[(int64_t)tok * e.Hq + head] = l2 * kLn2;
+                }
+            }
+        }
+        if (store_row && e.final_out) {
             uint16_t *op = static_cast<uint16_t *>(e.out) + (int64_t)qtok * e.o_tok + (int64_t)qhead * e.o_head;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
                     const int d = db * 32 + 8 * r4 + 4 * g;
+                    if (PAD && db * 32 + 8 * r4 >= dr) continue;
                     const u32x2 w = {E::pack2(o[db][4 * r4] * inv, o[db][4 * r4 + 1] * inv),
                                      E::pack2(o[db][4 * r4 + 2] * inv, o[db][4 * r4 + 3] * inv)};
                     *reinterpret_cast<u32x2 *>(op + d) = w;
                 }
             if (e.lse && g == 0) e.lse[(int64_t)qtok * e.Hq + qhead] = lse2 * kLn2;
-        } else if (qvalid) {
-            // static split: row (token, head) of the partial rows; stream-K:
-            // row wave * 32 + l32 of the workgroup's slot
-            const int64_t prow = e.slot >= 0 ? (int64_t)e.slot * ROWS + wave * 32 + l32 : e.prow0 + qtok;
+        } else if (store_row) {
             if (prow >= e.part_rows) {
                 raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
             } else {
                 const int64_t orow = e.slot >= 0 ? prow : prow * e.Hq + qhead;
-                float *pp = e.part_o + orow * D;
+                float *pp = e.part_o + orow * dr;
 #pragma unroll
                 for (int db = 0; db < DB; ++db)
 #pragma unroll
                     for (int r4 = 0; r4 < 4; ++r4) {
                         const int d = db * 32 + 8 * r4 + 4 * g;
+                        if (PAD && db * 32 + 8 * r4 >= dr) continue;
                         const floatx4 w = {o[db][4 * r4] * inv, o[db][4 * r4 + 1] * inv, o[db][4 * r4 + 2] * inv,
                                            o[db][4 * r4 + 3] * inv};
                         *reinterpret_cast<floatx4 *>(pp + d) = w;
@@ -1226,9 +1349,13 @@ void tree_attn_mfma_kernel(AttnArgs a) {
 // stage twice the 8-wave instance's share of a tile, the latter holds 128
 // registers of Q and 128 of O per lane; their 133-135 KB of LDS leave room
 // for one workgroup (one wave per SIMD) per CU anyway.
-template <int D, int WAVES, bool STORE, int WPE = 2, bool SKI = false>
+// PAD: head dims the instances do not name (multiples of 8 below D), the
+// missing elements zeros.
+template <int D, int WAVES, bool STORE, int WPE = 2, bool SKI = false, bool PAD = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void tree_attn_f32_kernel(AttnArgs a) {
+    constexpr uint32_t kNowhere = 0x7ffffff0u;   // byte offset past every source: loads as zeros
+    const int dr = PAD ? a.D : D;                // the call's head dim
     constexpr int NT = WAVES * 64;
     constexpr int BN = D <= 128 ? 64 : 32;  // keys per tile
     constexpr int NKB = BN / 32;           // 32-key MFMA blocks per tile
@@ -1275,7 +1402,8 @@ void tree_attn_f32_kernel(AttnArgs a) {
                            DH * g;
 #pragma unroll
         for (int i = 0; i < DH / 4; ++i) {
-            const floatx4 x = qvalid ? *reinterpret_cast<const floatx4 *>(src + 4 * i) : floatx4{};
+            const floatx4 x = qvalid && (!PAD || DH * g + 4 * i < dr) ? *reinterpret_cast<const floatx4 *>(src + 4 * i)
+                                                                      : floatx4{};
 #pragma unroll
             for (int j = 0; j < 4; ++j) qf[4 * i + j] = x[j];
         }
@@ -1303,10 +1431,10 @@ void tree_attn_f32_kernel(AttnArgs a) {
     const uint32_t ksb_pre = (uint32_t)kv.kpre_t * 4u, vsb_pre = (uint32_t)kv.vpre_t * 4u;
     const uint32_t ksb_pack = (uint32_t)kv.kpack_t * 4u, vsb_pack = (uint32_t)kv.vpack_t * 4u;
     const int rows_pre = STORE ? sq.S : sq.T;
-    const __amdgpu_buffer_rsrc_t kr_pre = seg_rsrc(kv.kpre, rows_pre, ksb_pre, D * 4);
-    const __amdgpu_buffer_rsrc_t vr_pre = seg_rsrc(kv.vpre, rows_pre, vsb_pre, D * 4);
-    const __amdgpu_buffer_rsrc_t kr_pack = seg_rsrc(kv.kpack, STORE ? sq.P : 0, ksb_pack, D * 4);
-    const __amdgpu_buffer_rsrc_t vr_pack = seg_rsrc(kv.vpack, STORE ? sq.P : 0, vsb_pack, D * 4);
+    const __amdgpu_buffer_rsrc_t kr_pre = seg_rsrc(kv.kpre, rows_pre, ksb_pre, dr * 4);
+    const __amdgpu_buffer_rsrc_t vr_pre = seg_rsrc(kv.vpre, rows_pre, vsb_pre, dr * 4);
+    const __amdgpu_buffer_rsrc_t kr_pack = seg_rsrc(kv.kpack, STORE ? sq.P : 0, ksb_pack, dr * 4);
+    const __amdgpu_buffer_rsrc_t vr_pack = seg_rsrc(kv.vpack, STORE ? sq.P : 0, vsb_pack, dr * 4);
     u32x4 kst[K_PER_T];
     u32x4 vst[V_PER_T][DB];
     auto fetch = [&](int t) __attribute__((always_inline)) {
@@ -1322,7 +1450,8 @@ void tree_attn_f32_kernel(AttnArgs a) {
             const int cidx = tid + it * NT;
             if (cidx >= KCH) break;
             const int key = cidx / (D / 4), dch = cidx % (D / 4);
-            kst[it] = load16(krs, __umul24(row0 + key, ksb) + dch * 16);
+            const uint32_t off = __umul24(row0 + key, ksb) + dch * 16;
+            kst[it] = load16(krs, PAD && dch * 4 >= dr ? kNowhere : off);
         }
 #pragma unroll
         for (int it = 0; it < V_PER_T; ++it) {
@@ -1331,7 +1460,8 @@ void tree_attn_f32_kernel(AttnArgs a) {
             const int key = u >> 3, lg = u & 7;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
-                vst[it][db] = load16(vrs, __umul24(row0 + key, vsb) + db * 128 + lg * 16);
+                vst[it][db] = load16(vrs, PAD && db * 32 + lg * 4 >= dr ? kNowhere
+                                                                        : __umul24(row0 + key, vsb) + db * 128 + lg * 16);
         }
     };
     // register -> LDS: K as is; V with d = 32*db + l stored at vpos(l)*DB + db
@@ -1520,7 +1650,7 @@ void tree_attn_f32_kernel(AttnArgs a) {
                 raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
             } else {
                 const int64_t orow = e.slot >= 0 ? prow : prow * e.Hq + qhead;
-                dst = e.part_o + orow * D;
+                dst = e.part_o + orow * dr;
                 if (g == 0) (e.slot >= 0 ? e.sk_lse : e.part_lse)[orow] = lse2;
             }
         }
@@ -1530,6 +1660,7 @@ void tree_attn_f32_kernel(AttnArgs a) {
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
                     const int d = db * 32 + 8 * r4 + 4 * g;
+                    if (PAD && db * 32 + 8 * r4 >= dr) continue;
                     const floatx4 w = {o[db][4 * r4] * inv, o[db][4 * r4 + 1] * inv, o[db][4 * r4 + 2] * inv,
                                        o[db][4 * r4 + 3] * inv};
                     *reinterpret_cast<floatx4 *>(dst + d) = w;
@@ -1646,10 +1777,12 @@ __device__ void combine_stream_k(const AttnArgs &a, const SkPlan &pl, const Seq 
     }
 }
 
-// E: the 16-bit format when OutT is 2 bytes; SKI: merges stream-K pieces
-template <typename OutT, int D, typename E, bool SKI = false>
+// E: the 16-bit format when OutT is 2 bytes; SKI: merges stream-K pieces;
+// DT: the head dim, or 0 to read it from the arguments
+template <typename OutT, int DT, typename E, bool SKI = false>
 __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnArgs a) {
-    constexpr int C = D / 4;
+    const int D = DT ? DT : a.D;
+    const int C = D / 4;
     __shared__ typename std::conditional<SKI, CombineLdsSk, CombineLds>::type sm;
     const int groups = a.comb_groups;
     const int tok = blockIdx.x / groups;
@@ -1681,7 +1814,7 @@ __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnArgs a) {
         i = tok - sq.q0;
         if constexpr (SKI) {
             if (pl.use) {
-                combine_stream_k<OutT, D, E>(a, pl, sq, i, tok, h0, min(a.Hq, h0 + hpg), bcast(base, src),
+                combine_stream_k<OutT, DT, E>(a, pl, sq, i, tok, h0, min(a.Hq, h0 + hpg), bcast(base, src),
                                              bcast(tiles, src), sm);
                 return;
             }
@@ -1819,19 +1952,12 @@ __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnArgs a) {
 }
 
 // --------------------------------------------------------------------------
-// Generic kernel: fp32, bf16 or fp16 inputs, any head_dim <= 256 (multiple of 8),
-// scalar FMA.  One workgroup = 16 query rows of one (request, KV head).
+// Generic kernel, for head dims without an instance of their own whose bases
+// or strides are not 16-byte aligned or whose sources exceed the MFMA kernels'
+// row addressing: fp32, bf16 or fp16, any multiple of 8 up to 256, scalar FMA.  One workgroup = 16 query rows of one (request, KV head).
 // DMAX sizes the LDS tiles: 128 (42 KB) for head_dim <= 128, 256 (83 KB)
 // above, as the reference kernel takes any power-of-two head_dim.
 // --------------------------------------------------------------------------
-template <typename T, typename E>
-__device__ __forceinline__ float load_elem(const T *p) {
-    if constexpr (sizeof(T) == 2)
-        return E::widen(*p);
-    else
-        return *p;
-}
-
 // T: float or uint16_t; E: the 16-bit format when T is 2 bytes
 template <typename T, int DMAX, typename E>
 __global__ __launch_bounds__(256) void tree_attn_generic_kernel(AttnArgs a, int D) {
@@ -1955,9 +2081,13 @@ static Topology device_topology() {
     return t;
 }
 
-static bool mfma_path(int32_t dtype, int32_t D) {
-    if (dtype == CAST_FP32) return D == 64 || D == 128 || D == 256;
-    return (dtype == CAST_BF16 || dtype == CAST_FP16) && (D == 64 || D == 128 || D == 256);
+static bool mfma_path(int32_t, int32_t D) { return D == 64 || D == 128 || D == 256; }
+
+// The padded MFMA instance of another head dim: its D, or 0.
+static int padded_dim(int32_t dtype, int32_t D) {
+    if (mfma_path(dtype, D) || D <= 0 || D > 256 || D % 8) return 0;
+    if (dtype == CAST_FP32) return D < 64 ? 64 : D < 128 ? 128 : 256;
+    return D < 64 ? 64 : D <= 96 ? 96 : D < 128 ? 128 : D <= 192 ? 192 : 256;
 }
 
 // Waves per workgroup (32 query rows each).  16-bit inputs take 8 waves (256
@@ -1974,7 +2104,9 @@ static bool mfma_path(int32_t dtype, int32_t D) {
 // Head_dim 256 always runs 4 waves, one per SIMD: fewer threads would each
 // stage more of its 32 KB tiles than the registers hold.
 static int waves_for(int32_t batch, int32_t total_q, int32_t G, int32_t dtype, int32_t D) {
-    if (D == 256) return 4;
+    // the padded 16-bit instances have 4 waves only
+    const int dp = padded_dim(dtype, D);
+    if (D == 256 || dp == 256 || (dp && dtype != CAST_FP32)) return 4;
     if (dtype == CAST_FP32) return (int64_t)(total_q < kMaxPack ? total_q : kMaxPack) * G <= 128 ? 4 : 8;
     const int64_t p_avg = ((int64_t)total_q + batch - 1) / batch;
     return (p_avg < kMaxPack ? p_avg : kMaxPack) * G <= 192 ? 4 : 8;
@@ -2019,19 +2151,19 @@ struct AttnKernel {
     const void *fn;
     int threads;
 };
-template <int DD, int W, int WPE, bool SKI>
+template <int DD, int W, int WPE, bool SKI, bool PAD = false>
 static AttnKernel mfma_instance(bool f16, bool store) {
     const void *fn =
-        f16 ? (store ? reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, true, Fp16, WPE, SKI>)
-                     : reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, false, Fp16, WPE, SKI>))
-            : (store ? reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, true, Bf16, WPE, SKI>)
-                     : reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, false, Bf16, WPE, SKI>));
+        f16 ? (store ? reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, true, Fp16, WPE, SKI, PAD>)
+                     : reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, false, Fp16, WPE, SKI, PAD>))
+            : (store ? reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, true, Bf16, WPE, SKI, PAD>)
+                     : reinterpret_cast<const void *>(&tree_attn_mfma_kernel<DD, W, false, Bf16, WPE, SKI, PAD>));
     return {fn, W * 64};
 }
-template <int DD, int W, int WPE, bool SKI>
+template <int DD, int W, int WPE, bool SKI, bool PAD = false>
 static AttnKernel f32_instance(bool store) {
-    const void *fn = store ? reinterpret_cast<const void *>(&tree_attn_f32_kernel<DD, W, true, WPE, SKI>)
-                           : reinterpret_cast<const void *>(&tree_attn_f32_kernel<DD, W, false, WPE, SKI>);
+    const void *fn = store ? reinterpret_cast<const void *>(&tree_attn_f32_kernel<DD, W, true, WPE, SKI, PAD>)
+                           : reinterpret_cast<const void *>(&tree_attn_f32_kernel<DD, W, false, WPE, SKI, PAD>);
     return {fn, W * 64};
 }
 template <bool SKI>
@@ -2050,9 +2182,21 @@ static AttnKernel attn_kernel_of(int32_t dtype, int32_t D, int waves, bool store
 // SIMD of the register budget) as the kernels' comments give it; sk picks
 // the stream-K instance.
 static AttnKernel attn_kernel(int32_t dtype, int32_t D, int waves, bool store, bool sk) {
+    const bool f16 = dtype == CAST_FP16;
+    switch (dtype == CAST_FP32 ? -padded_dim(dtype, D) : padded_dim(dtype, D)) {
+        case 64: return mfma_instance<64, 4, 2, false, true>(f16, store);
+        case 96: return mfma_instance<96, 4, 2, false, true>(f16, store);
+        case 128: return mfma_instance<128, 4, 2, false, true>(f16, store);
+        case 192: return mfma_instance<192, 4, 1, false, true>(f16, store);
+        case 256: return mfma_instance<256, 4, 1, false, true>(f16, store);
+        case -64: return waves == 4 ? f32_instance<64, 4, 2, false, true>(store) : f32_instance<64, 8, 2, false, true>(store);
+        case -128: return waves == 4 ? f32_instance<128, 4, 1, false, true>(store) : f32_instance<128, 8, 2, false, true>(store);
+        case -256: return f32_instance<256, 4, 1, false, true>(store);
+        default: break;
+    }
     if (D == 256)
         return dtype == CAST_FP32 ? f32_instance<256, 4, 1, false>(store)
-                                  : mfma_instance<256, 4, 1, false>(dtype == CAST_FP16, store);
+                                  : mfma_instance<256, 4, 1, false>(f16, store);
     return sk ? attn_kernel_of<true>(dtype, D, waves, store) : attn_kernel_of<false>(dtype, D, waves, store);
 }
 
@@ -2137,7 +2281,8 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
     p.chunk = resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, kv_split);
     const bool automatic =
         kv_split == 0 || kv_split == resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, 0);
-    if (automatic && batch > 0 && batch <= 64 && mfma_path(dtype, D) && dtype != CAST_FP32) {
+    const bool padded = padded_dim(dtype, D) != 0;
+    if (automatic && batch > 0 && batch <= 64 && ((mfma_path(dtype, D) && dtype != CAST_FP32) || padded)) {
         const int64_t G = Hq / Hkv;
         const int waves = waves_for(batch, total_q, (int32_t)G, dtype, D);
         const int64_t rows_wg = waves * 32;
@@ -2215,31 +2360,45 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     if (!q || !kv.k_pre || !kv.v_pre || !kv.k_pack || !kv.v_pack || !out || !cu_q || !prefix_len || !pack_len ||
         !mask || (!kv.store && !cu_kv))
         return CAST_ERR_NULL_POINTER;
-    const bool mfma = mfma_path(dtype, head_dim);
-    if (!mfma && (head_dim > 256 || head_dim % 8)) return CAST_ERR_HEAD_DIM;
+    bool mfma = mfma_path(dtype, head_dim);
+    const bool padded = padded_dim(dtype, head_dim) != 0;
+    if (!mfma && !padded) return CAST_ERR_HEAD_DIM;
     const int64_t esz = dtype == CAST_FP32 ? 4 : 2;
     int32_t max_rows = INT32_MAX;
     auto a16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    if (mfma) {
-        if (!a16(q) || !a16(kv.k_pre) || !a16(kv.v_pre) || !a16(kv.k_pack) || !a16(kv.v_pack) || !a16(out))
-            return CAST_ERR_ALIGNMENT;
-        const int64_t strides[14] = {q_tok,     q_head,    kv.kpre_b,  kv.kpre_h,  kv.kpre_t,
-                                     kv.vpre_b, kv.vpre_h, kv.vpre_t,  kv.kpack_h, kv.kpack_t,
-                                     kv.vpack_h, kv.vpack_t, o_tok,    o_head};
-        for (int64_t s : strides)
-            if ((s * esz) % 16) return CAST_ERR_ALIGNMENT;
-        // key rows are addressed by 24-bit row index x 24-bit byte stride,
-        // within 2^31 bytes of their source's first row
+    // 16-byte bases and strides; key rows are addressed by 24-bit row index x
+    // 24-bit byte stride, within 2^31 bytes of their source's first row.  The
+    // padded instances leave what breaks these to the scalar kernel, which
+    // always took it.
+    int limit = CAST_OK;
+    if (!a16(q) || !a16(kv.k_pre) || !a16(kv.v_pre) || !a16(kv.k_pack) || !a16(kv.v_pack) || !a16(out))
+        limit = CAST_ERR_ALIGNMENT;
+    const int64_t strides[14] = {q_tok,     q_head,    kv.kpre_b,  kv.kpre_h,  kv.kpre_t,
+                                 kv.vpre_b, kv.vpre_h, kv.vpre_t,  kv.kpack_h, kv.kpack_t,
+                                 kv.vpack_h, kv.vpack_t, o_tok,    o_head};
+    for (int64_t s : strides)
+        if ((s * esz) % 16) limit = CAST_ERR_ALIGNMENT;
+    if (limit == CAST_OK) {
         const int64_t rows[4] = {kv.kpre_t, kv.vpre_t, kv.kpack_t, kv.vpack_t};
         int64_t rb = 0;
         for (int64_t r : rows) {
-            if (r < 0 || r * esz >= (int64_t)1 << 24) return CAST_ERR_SHAPE;
+            if (r < 0 || r * esz >= (int64_t)1 << 24) limit = CAST_ERR_SHAPE;
             rb = r * esz > rb ? r * esz : rb;
         }
         const int64_t by_bytes = rb ? (((int64_t)1 << 31) - 1 - head_dim * esz) / rb : INT32_MAX;
         const int64_t by_index = ((int64_t)1 << 24) - 64;
-        max_rows = (int32_t)(by_bytes < by_index ? by_bytes : by_index);
+        const int64_t most = by_bytes < by_index ? by_bytes : by_index;
+        if (mfma) {
+            max_rows = (int32_t)most;
+        } else if (limit == CAST_OK && most > 0) {
+            const int64_t longest = kv.store ? (kv.cap > total_q ? kv.cap : total_q) : total_kv;
+            if (longest <= most) {
+                mfma = true;
+                max_rows = (int32_t)most;
+            }
+        }
     }
+    if (mfma && limit != CAST_OK) return limit;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     AttnArgs a{};
     a.q = q;
@@ -2357,7 +2516,11 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
 #define CAST_COMBINE(OT, DD, E)                                                         \
     (a.sk_mode ? tree_attn_combine_kernel<OT, DD, E, true><<<cg, 256, 0, st>>>(a) \
                : tree_attn_combine_kernel<OT, DD, E, false><<<cg, 256, 0, st>>>(a))
-        if (dtype == CAST_FP32) {
+        if (padded) {
+            if (dtype == CAST_FP32) tree_attn_combine_kernel<float, 0, Bf16><<<cg, 256, 0, st>>>(a);
+            else if (dtype == CAST_FP16) tree_attn_combine_kernel<uint16_t, 0, Fp16><<<cg, 256, 0, st>>>(a);
+            else tree_attn_combine_kernel<uint16_t, 0, Bf16><<<cg, 256, 0, st>>>(a);
+        } else if (dtype == CAST_FP32) {
             if (head_dim == 256) tree_attn_combine_kernel<float, 256, Bf16, false><<<cg, 256, 0, st>>>(a);
             else if (head_dim == 128) CAST_COMBINE(float, 128, Bf16);
             else CAST_COMBINE(float, 64, Bf16);

@@ -1,0 +1,125 @@
+"""Head dims without an instance of their own (multiples of 8 up to 256) on
+the padded MFMA kernels: against float64, against the scalar kernel (which
+takes what the padded kernels cannot: here an output that is not 16-byte
+aligned), and rows that hold infinities."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from cast_amd import scenarios as SC
+from cast_amd import varlen_tree_attention
+from cast_amd.tree import TreeNode
+from cast_amd.tree_attn import store_tree_attention
+from oracle import bitmask as OB
+
+pytestmark = pytest.mark.gpu
+
+# the spacing just above 1 (8, 11 and 24 significant bits): rounding is within half of it, relatively
+EPS = {"bf16": 2.0 ** -7, "fp16": 2.0 ** -10, "fp32": 2.0 ** -23}
+
+
+def _case(gpu, D, dtype, seed, prefix, packs, Hq=8, Hkv=2):
+    rng = np.random.default_rng(seed)
+    trees = [[TreeNode(i, 1, int(rng.integers(-1, i)) if i else -1, 0.0) for i in range(p - 1)] for p in packs]
+    wl = SC._make(f"d{D}", trees, prefix, dict(Hq=Hq, Hkv=Hkv, D=D, vocab=100), dtype, seed, 0.5)
+    q, k, v = wl.qkv(device=gpu)
+    words = OB.chain_walk_words(wl.packed.parent, wl.cu_q)
+    return wl, q, k, v, wl.meta_tensors(gpu), torch.from_numpy(words.view(np.int64).copy()).to(gpu), words
+
+
+def _exact(wl, q, k, v, words):
+    """out, lse in float64 (the visibility bits unpacked to a dense mask)."""
+    G = wl.Hq // wl.Hkv
+    out = torch.zeros(q.shape, dtype=torch.float64)
+    lse = torch.zeros(q.shape[:2], dtype=torch.float64)
+    q, k, v = (x.double().cpu() for x in (q, k, v))
+    for b in range(wl.B):
+        r0, r1, S = int(wl.cu_q[b]), int(wl.cu_q[b + 1]), int(wl.prefix_len[b])
+        kb, vb = (x[int(wl.cu_kv[b]):int(wl.cu_kv[b + 1])].repeat_interleave(G, dim=1) for x in (k, v))
+        bits = np.unpackbits(words[r0:r1].view(np.uint8), axis=1, bitorder="little")[:, :r1 - r0].astype(bool)
+        vis = torch.cat([torch.ones(r1 - r0, S, dtype=torch.bool), torch.from_numpy(bits)], dim=1)
+        s = torch.matmul(q[r0:r1].transpose(0, 1), kb.permute(1, 2, 0).contiguous()) / math.sqrt(wl.D)
+        s = s.masked_fill(~vis[None], -math.inf)
+        lse[r0:r1] = torch.logsumexp(s, -1).T
+        out[r0:r1] = torch.matmul(torch.softmax(s, -1), vb.transpose(0, 1).contiguous()).transpose(0, 1)
+    return out, lse
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("D", [8, 56, 72, 80, 96, 104, 120, 136, 192, 200, 248])
+def test_padded_head_dims(gpu, D, dtype):
+    # 700 keys split by the automatic choice; packs around the 32-row block
+    wl, q, k, v, meta, mask, words = _case(gpu, D, dtype, D, [700, 0, 65], [64, 9, 33])
+    print(f"case padded D={D} {dtype}", flush=True)
+    want, want_l = _exact(wl, q, k, v, words)
+    for split in (0, -1):
+        out, lse = varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"],
+                                         mask, return_lse=True, kv_split=split, check=True)
+        # P and every sum are fp32: what is left is the output's own rounding
+        # (EPS / 2), twice where a split's fp32 partial rounds first, and fp32
+        # sums of up to 764 terms (2^-24 * sqrt(764) * 8 < 2e-5 of the rows' scale)
+        err = (out.double().cpu() - want).abs()
+        assert (err <= 0.51 * EPS[dtype] * want.abs() + 2e-5).all(), f"{err.max()}"
+        assert ((lse.double().cpu() - want_l).abs() <= 2e-5).all()
+
+
+@pytest.mark.parametrize("D", [80, 192])
+def test_padded_store_layout_and_scalar_fallback(gpu, D):
+    wl, q, k, v, meta, mask, _ = _case(gpu, D, "bf16", 1, [300, 129], [20, 64])
+    print(f"case padded-store D={D}", flush=True)
+    cap = 320
+    ks = torch.zeros((wl.B, wl.Hkv, cap, D), dtype=q.dtype, device=gpu)
+    vs, kp = torch.zeros_like(ks), torch.empty((wl.Hkv, wl.total_q, D), dtype=q.dtype, device=gpu)
+    vp = torch.empty_like(kp)
+    for b in range(wl.B):
+        a, S, e = int(wl.cu_kv[b]), int(wl.prefix_len[b]), int(wl.cu_kv[b + 1])
+        r = slice(int(wl.cu_q[b]), int(wl.cu_q[b + 1]))
+        for src, st, pk in ((k, ks, kp), (v, vs, vp)):
+            st[b, :, :S] = src[a:a + S].transpose(0, 1)
+            pk[:, r] = src[a + S:e].transpose(0, 1)
+    args = (meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask)
+    o1, l1 = varlen_tree_attention(q, k, v, *args, return_lse=True, check=True)
+    o2, l2 = store_tree_attention(q, ks, vs, kp, vp, meta["cu_q"], meta["prefix_len"], meta["pack_len"], mask,
+                                  total_kv=wl.total_kv, return_lse=True, check=True)
+    assert torch.equal(o1, o2) and torch.equal(l1, l2)
+    # an output 8 bytes off: the scalar kernel, as before; both are the fp32
+    # result rounded once, so at most a rounding apart
+    buf = torch.empty(q.numel() + 4, dtype=q.dtype, device=gpu)
+    o3, l3 = varlen_tree_attention(q, k, v, *args, return_lse=True, check=True, out=buf[4:].view(q.shape))
+    assert ((o3.float() - o1.float()).abs() <= EPS["bf16"] * o1.float().abs() + 2e-5).all()
+    assert ((l3 - l1).abs() <= 2e-5).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("what", ["v-inf", "k-minus-inf", "k-nan", "q-inf", "score-overflow"])
+def test_padded_rows_with_infinities(gpu, dtype, what):
+    # rows whose products meet an infinity or a NaN come out as the scalar
+    # kernel gives them; all others keep their bits
+    wl, q, k, v, meta, mask, _ = _case(gpu, 96, dtype, 2, [200, 90], [10, 40])
+    print(f"case padded-nonfinite {what} {dtype}", flush=True)
+    args = (meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask)
+    clean = varlen_tree_attention(q, k, v, *args)
+    q, k, v = q.clone(), k.clone(), v.clone()
+    if what == "v-inf":
+        v[5, 0, 17] = math.inf
+    elif what == "k-minus-inf":
+        k[70, 1, 3] = -math.inf
+    elif what == "k-nan":
+        k[12, 0, 95] = math.nan
+    elif what == "q-inf":
+        q[3, 2, 40] = math.inf
+    else:
+        q[4] *= 1e4
+        k[:200, 0] *= 1e4
+    got, lse = varlen_tree_attention(q, k, v, *args, return_lse=True, check=True)
+    buf = torch.empty(q.numel() + 4, dtype=q.dtype, device=gpu)
+    ref, ref_l = varlen_tree_attention(q, k, v, *args, return_lse=True, out=buf[4:].view(q.shape))
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isnan(lse), torch.isnan(ref_l))
+    fin = torch.isfinite(ref)
+    assert torch.equal(got[~fin & ~torch.isnan(ref)], ref[~fin & ~torch.isnan(ref)])
+    if what != "score-overflow":
+        assert not fin.all()
+        assert ((got.float() - ref.float()).abs()[fin] <= EPS[dtype] * ref.float().abs()[fin] + 2e-5).all()
+        assert torch.equal(got[10:], clean[10:]) or what == "k-minus-inf"
