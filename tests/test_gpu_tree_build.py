@@ -1,0 +1,53 @@
+"""The workgroup-wide tree build against the host's heap (cast_amd.tree
+build_tree in float64), node for node: pool sizes, ties and budgets at the
+edges of its tables."""
+import numpy as np
+import pytest
+import torch
+
+from cast_amd import build_trees
+from cast_amd.tree import build_tree
+
+pytestmark = pytest.mark.gpu
+
+
+def _lp(kind, rng, B, L, k):
+    if kind == "gaps":          # drafter-like
+        lp = -np.cumsum(rng.exponential(1.0, size=(B, L, k)), axis=2)
+    elif kind == "coarse":      # many equal path scores at several depths
+        lp = -np.sort(rng.integers(0, 6, size=(B, L, k)), axis=2) / 4.0
+    elif kind == "zeros":       # every score equal: the pool outgrows its tables
+        lp = np.zeros((B, L, k))
+    elif kind == "flat":        # children nearly as good as their parents
+        lp = -np.sort(rng.random((B, L, k)) * 1e-3, axis=2)
+    elif kind == "positive":    # scores that grow along a path: not for the bulk path
+        lp = 0.5 - np.cumsum(rng.exponential(0.3, size=(B, L, k)), axis=2)
+    else:                       # "masked": candidates of log-probability -inf
+        lp = -np.cumsum(rng.exponential(1.0, size=(B, L, k)), axis=2)
+        lp[..., max(1, k // 2):] = -np.inf
+    return lp
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("kind", ["gaps", "coarse", "zeros", "flat", "positive", "masked"])
+@pytest.mark.parametrize("L,k", [(15, 8), (15, 16), (15, 10), (2, 4), (40, 2), (3, 1), (255, 3)])
+def test_trees_match_the_heap(gpu, L, k, kind, dtype):
+    rng = np.random.default_rng(L * 100 + k)
+    budgets = [127, 64, 41, 40, 39, 1, 0]
+    B = len(budgets)
+    print(f"case trees L={L} k={k} {kind} {dtype}", flush=True)
+    lp = torch.from_numpy(_lp(kind, rng, B, L, k)).to(dtype)
+    idx = torch.from_numpy(rng.integers(0, 1000, size=(B, L, k)))
+    token, depth, parent, score, n = (x.cpu().numpy() for x in build_trees(
+        idx.to(gpu), lp.to(gpu), torch.tensor(budgets, dtype=torch.int32), check=True))
+    for b, want in enumerate(budgets):
+        if kind == "masked":    # the host heap adds infinities; stop it at the finite nodes
+            ref = [x for x in build_tree(idx[b].numpy(), lp[b].double().numpy(), want, k) if np.isfinite(x.score)]
+        else:
+            ref = build_tree(idx[b].numpy(), lp[b].double().numpy(), want, k)
+        m = len(ref)
+        assert n[b] == m or (kind == "masked" and n[b] >= m)
+        assert token[b, :m].tolist() == [x.token for x in ref]
+        assert depth[b, :m].tolist() == [x.depth for x in ref]
+        assert parent[b, :m].tolist() == [x.parent for x in ref]
+        assert score[b, :m].tolist() == [x.score for x in ref]
