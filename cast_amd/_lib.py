@@ -52,6 +52,7 @@ SIGNATURES = {
                           [_I32, _P, _P], ctypes.c_int),
     "cast_draft_topk": ([_P, _I64, _I32, _I32, _I32, _I32, _P, _P, _I32, _P, _SZ, _P], ctypes.c_int),
     "cast_draft_topk_workspace_size": ([_I32, _I32, _I32, _I32, _I32], _SZ),
+    "cast_build_trees_uniform": ([_P, _P, _I32, _I32, _I32, _I32, _I32] + [_P] * 7, ctypes.c_int),
     "cast_build_trees": ([_P, _P, _I32, _I32, _I32, _I32] + [_P] * 8, ctypes.c_int),
     "cast_greedy_accept": ([_P, _I64, _I32, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _P], ctypes.c_int),
 }
@@ -106,8 +107,8 @@ def stream_of(tensor):
     import torch
     raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
     if raw is None:
-        return ctypes.c_void_p(torch.cuda.current_stream(tensor.device).cuda_stream)
-    return ctypes.c_void_p(raw(tensor.device.index))
+        return torch.cuda.current_stream(tensor.device).cuda_stream
+    return raw(tensor.get_device())
 
 
 _NO_SWITCH = contextlib.nullcontext()
@@ -117,11 +118,14 @@ def on_device(dev):
     """A context that makes dev the current HIP device for the launches inside
     it, switching only when another device is current."""
     import torch
-    return _NO_SWITCH if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+    get = getattr(torch._C, "_cuda_getDevice", None)
+    current = torch.cuda.current_device() if get is None or not torch.cuda.is_initialized() else get()
+    return _NO_SWITCH if current == dev.index else torch.cuda.device(dev)
 
 
 def ptr(tensor):
-    return ctypes.c_void_p(tensor.data_ptr()) if tensor is not None else ctypes.c_void_p(0)
+    """A tensor's device address as ctypes takes it (None: a null pointer)."""
+    return tensor.data_ptr() if tensor is not None else None
 
 
 def raise_device_flags(flags, what):

@@ -713,7 +713,8 @@ __device__ int build_bulk(TreeLds &m, int L, int k, int want) {
 template <typename LP>
 __global__ __launch_bounds__(kBulkThreads) void build_trees_kernel(const int64_t *__restrict__ top_idx,
                                                          const LP *__restrict__ top_lp, int32_t L, int32_t k,
-                                                         const int32_t *__restrict__ budget, int64_t *token,
+                                                         const int32_t *__restrict__ budget, int32_t uniform,
+                                                         int64_t *token,
                                                          int32_t *depth, int32_t *parent, double *score,
                                                          int32_t *n_nodes, int32_t *status) {
     __shared__ TreeLds m;
@@ -722,7 +723,7 @@ __global__ __launch_bounds__(kBulkThreads) void build_trees_kernel(const int64_t
     const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     const int64_t *ti = top_idx + (size_t)b * L * k;
     const LP *tl = top_lp + (size_t)b * L * k;
-    int want = budget[b];
+    int want = budget ? budget[b] : uniform;
     if (want < 0 || want > kMaxPack - 1) {
         if (tid == 0) raise_flag(status, CAST_FLAG_BAD_PACK);
         want = want < 0 ? 0 : kMaxPack - 1;
@@ -917,21 +918,41 @@ extern "C" int cast_draft_topk(const void *logits, int64_t logits_ld, int32_t ro
     return hipGetLastError() == hipSuccess ? CAST_OK : CAST_ERR_HIP;
 }
 
+// budget: per-request node counts, or null for `uniform` in every tree
+static int build_trees_run(const int64_t *top_idx, const void *top_lp, int32_t lp_dtype, int32_t batch, int32_t L,
+                           int32_t k, const int32_t *budget, int32_t uniform, int64_t *token, int32_t *depth,
+                           int32_t *parent, double *score, int32_t *n_nodes, int32_t *status, cast_stream_t stream) {
+    if (batch < 0 || L < 1 || L > kLMax || k < 1 || k > kTopKMax) return CAST_ERR_SHAPE;
+    if (lp_dtype != CAST_FP32 && lp_dtype != CAST_FP64) return CAST_ERR_DTYPE;
+    if (batch == 0) return CAST_OK;
+    if (!top_idx || !top_lp || !token || !depth || !parent || !score || !n_nodes) return CAST_ERR_NULL_POINTER;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (lp_dtype == CAST_FP32)
+        build_trees_kernel<float><<<batch, kBulkThreads, 0, s>>>(top_idx, static_cast<const float *>(top_lp), L, k,
+                                                                 budget, uniform, token, depth, parent, score, n_nodes,
+                                                                 status);
+    else
+        build_trees_kernel<double><<<batch, kBulkThreads, 0, s>>>(top_idx, static_cast<const double *>(top_lp), L, k,
+                                                                  budget, uniform, token, depth, parent, score,
+                                                                  n_nodes, status);
+    return hipGetLastError() == hipSuccess ? CAST_OK : CAST_ERR_HIP;
+}
+
 extern "C" int cast_build_trees(const int64_t *top_idx, const void *top_lp, int32_t lp_dtype, int32_t batch,
                                 int32_t L, int32_t k, const int32_t *budget, int64_t *token, int32_t *depth,
                                 int32_t *parent, double *score, int32_t *n_nodes, int32_t *status,
                                 cast_stream_t stream) {
-    if (batch < 0 || L < 1 || L > kLMax || k < 1 || k > kTopKMax) return CAST_ERR_SHAPE;
-    if (lp_dtype != CAST_FP32 && lp_dtype != CAST_FP64) return CAST_ERR_DTYPE;
-    if (batch == 0) return CAST_OK;
-    if (!top_idx || !top_lp || !budget || !token || !depth || !parent || !score || !n_nodes)
+    if (batch > 0 && L >= 1 && L <= kLMax && k >= 1 && k <= kTopKMax &&
+        (lp_dtype == CAST_FP32 || lp_dtype == CAST_FP64) && !budget)
         return CAST_ERR_NULL_POINTER;
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (lp_dtype == CAST_FP32)
-        build_trees_kernel<float><<<batch, kBulkThreads, 0, s>>>(top_idx, static_cast<const float *>(top_lp), L, k, budget,
-                                                       token, depth, parent, score, n_nodes, status);
-    else
-        build_trees_kernel<double><<<batch, kBulkThreads, 0, s>>>(top_idx, static_cast<const double *>(top_lp), L, k,
-                                                        budget, token, depth, parent, score, n_nodes, status);
-    return hipGetLastError() == hipSuccess ? CAST_OK : CAST_ERR_HIP;
+    return build_trees_run(top_idx, top_lp, lp_dtype, batch, L, k, budget, 0, token, depth, parent, score, n_nodes,
+                           status, stream);
+}
+
+extern "C" int cast_build_trees_uniform(const int64_t *top_idx, const void *top_lp, int32_t lp_dtype, int32_t batch,
+                                        int32_t L, int32_t k, int32_t nodes, int64_t *token, int32_t *depth,
+                                        int32_t *parent, double *score, int32_t *n_nodes, int32_t *status,
+                                        cast_stream_t stream) {
+    return build_trees_run(top_idx, top_lp, lp_dtype, batch, L, k, nullptr, nodes, token, depth, parent, score,
+                           n_nodes, status, stream);
 }

@@ -68,7 +68,10 @@ def build_trees(top_idx, top_lp, budget, k=None, *, check=False):
         top_idx, top_lp = top_idx[None], top_lp[None]
     if top_idx.dim() != 3 or top_lp.shape != top_idx.shape:
         raise ValueError("top_idx and top_lp must both be [B, L, k] (or [L, k])")
-    if isinstance(budget, int) or not (isinstance(budget, torch.Tensor) and budget.is_cuda):
+    if isinstance(budget, int):
+        if not 0 <= budget <= MAX_PACK - 1:
+            raise ValueError(f"budget must be in [0, {MAX_PACK - 1}] nodes per tree (packs of up to {MAX_PACK} tokens)")
+    elif not (isinstance(budget, torch.Tensor) and budget.is_cuda):
         # budgets known on the host are checked here; a device tensor above 127
         # is clamped by the kernel and flagged in the status word
         b_host = np.asarray(budget.cpu() if isinstance(budget, torch.Tensor) else budget).reshape(-1)
@@ -81,28 +84,30 @@ def build_trees(top_idx, top_lp, budget, k=None, *, check=False):
     if L < 1 or L > 255 or k < 1 or k > 16:
         raise ValueError("build_trees needs 1 <= L <= 255 future positions and 1 <= k <= 16 candidates")
     dev = top_idx.device
-    ti = top_idx[..., :k].to(torch.int64).contiguous()
-    tl = top_lp[..., :k]
+    if k < kk:
+        top_idx, top_lp = top_idx[..., :k], top_lp[..., :k]
+    ti = top_idx.to(torch.int64).contiguous()
+    tl = top_lp
     if tl.dtype != torch.float64:
         tl = tl.to(torch.float32)
     tl = tl.contiguous()
-    if isinstance(budget, int):
-        budget = torch.full((B,), budget, dtype=torch.int32, device=dev)
-    budget = torch.as_tensor(budget, device=dev).to(torch.int32).contiguous()
-    if budget.shape != (B,):
-        raise ValueError(f"budget must be an int or [{B}] per-request node counts")
+    uniform = isinstance(budget, int)   # one count for all: a kernel argument, no tensor to fill
+    if not uniform:
+        budget = torch.as_tensor(budget, device=dev).to(torch.int32).contiguous()
+        if budget.shape != (B,):
+            raise ValueError(f"budget must be an int or [{B}] per-request node counts")
     n = MAX_PACK - 1
-    token = torch.empty((B, n), dtype=torch.int64, device=dev)
-    depth = torch.empty((B, n), dtype=torch.int32, device=dev)
-    parent = torch.empty((B, n), dtype=torch.int32, device=dev)
-    score = torch.empty((B, n), dtype=torch.float64, device=dev)
-    n_nodes = torch.empty(B, dtype=torch.int32, device=dev)
+    token = ti.new_empty((B, n))
+    depth = ti.new_empty((B, n), dtype=torch.int32)
+    parent = torch.empty_like(depth)
+    score = ti.new_empty((B, n), dtype=torch.float64)
+    n_nodes = ti.new_empty(B, dtype=torch.int32)
     status = torch.zeros(1, dtype=torch.int32, device=dev) if check else None
+    build = lib.cast_build_trees_uniform if uniform else lib.cast_build_trees
     with _lib.on_device(dev):
-        st = lib.cast_build_trees(_lib.ptr(ti), _lib.ptr(tl), _lib.FP64 if tl.dtype == torch.float64 else _lib.FP32,
-                                  B, L, k, _lib.ptr(budget), _lib.ptr(token),
-                                  _lib.ptr(depth), _lib.ptr(parent), _lib.ptr(score), _lib.ptr(n_nodes),
-                                  _lib.ptr(status), _lib.stream_of(ti))
+        st = build(_lib.ptr(ti), _lib.ptr(tl), _lib.FP64 if tl.dtype == torch.float64 else _lib.FP32, B, L, k,
+                   budget if uniform else _lib.ptr(budget), _lib.ptr(token), _lib.ptr(depth), _lib.ptr(parent),
+                   _lib.ptr(score), _lib.ptr(n_nodes), _lib.ptr(status), _lib.stream_of(ti))
     _lib.check(st, "cast_build_trees")
     if check:
         _lib.raise_device_flags(status.item(), "build_trees")

@@ -27,6 +27,7 @@ Unlike the reference, the call needs no device-to-host copy of cu_q
 """
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
 
@@ -41,6 +42,8 @@ SPLIT_STREAM = -2
 
 
 def _as_i32(x, device):
+    if isinstance(x, torch.Tensor) and x.dtype is torch.int32 and x.get_device() == device.index and x.is_contiguous():
+        return x
     t = torch.as_tensor(x, device=device)
     if t.dtype != torch.int32:
         t = t.to(torch.int32)
@@ -48,11 +51,13 @@ def _as_i32(x, device):
 
 
 def _mask_words(mask, total_q, device):
-    m = torch.as_tensor(mask, device=device)
-    if m.dtype == torch.uint64:
-        m = m.view(torch.int64)
-    if m.dtype != torch.int64:
-        m = m.to(torch.int64)
+    m = mask
+    if not (isinstance(m, torch.Tensor) and m.dtype is torch.int64 and m.get_device() == device.index):
+        m = torch.as_tensor(mask, device=device)
+        if m.dtype == torch.uint64:
+            m = m.view(torch.int64)
+        if m.dtype != torch.int64:
+            m = m.to(torch.int64)
     if m.dim() == 1:
         words = 1
     elif m.dim() == 2 and m.shape[1] in (1, 2):
@@ -64,9 +69,19 @@ def _mask_words(mask, total_q, device):
     return m.contiguous(), words
 
 
-def _host_side(x):
-    """Metadata the caller holds on the host (list, tuple, numpy, CPU tensor)."""
-    return not (isinstance(x, torch.Tensor) and x.is_cuda)
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(device_index, *sizes):
+    """cast_tree_attn_workspace_size of one call's sizes (a function of them
+    and the device alone: asked once per size, not once per layer)."""
+    return _lib.load().cast_tree_attn_workspace_size(*sizes)
+
+
+def _host_side(*metadata):
+    """Whether the caller holds any of it on the host (list, tuple, numpy, CPU tensor)."""
+    for x in metadata:
+        if not (isinstance(x, torch.Tensor) and x.is_cuda):
+            return True
+    return False
 
 
 def check_host_metadata(cu_q, prefix_len, pack_len, total_q, total_kv, words, cu_kv=None, cap=None):
@@ -108,16 +123,19 @@ def check_host_metadata(cu_q, prefix_len, pack_len, total_q, total_kv, words, cu
 def _require_on(dev, **tensors):
     """Every given tensor (None skipped) on q's device: the kernels take raw
     device pointers, so a host or other-GPU tensor is refused here."""
+    di = dev.index
     for name, t in tensors.items():
-        if t is not None and t.device != dev:
+        if t is not None and t.get_device() != di:
             raise ValueError(f"{name} is on {t.device}, q on {dev}: all tensors must be on one GPU")
 
 
 def _ready(x, esz):
     """Last dim contiguous, 16-byte aligned base and strides."""
-    if x.stride(-1) != 1 or x.data_ptr() % 16 or any((s * esz) % 16 for s in x.stride()[:-1]):
-        return x.contiguous()
-    return x
+    st = x.stride()
+    low = x.data_ptr()
+    for s in st[:-1]:
+        low |= s * esz
+    return x if st[-1] == 1 and not low & 15 else x.contiguous()
 
 
 @dataclass
@@ -161,10 +179,12 @@ def varlen_tree_attention(q, k, v, cu_q, cu_kv, prefix_len, pack_len, ancestor_m
         raise ValueError("k and v must both be [total_kv, H_kv, D] with the head dim of q")
     esz = q.element_size()
     dev = q.device
-    _require_on(dev, k=k, v=v, out=out, workspace=workspace)
+    di = dev.index
+    if k.get_device() != di or v.get_device() != di or out is not None or workspace is not None:
+        _require_on(dev, k=k, v=v, out=out, workspace=workspace)
     q, k, v = _ready(q, esz), _ready(k, esz), _ready(v, esz)
     mask, words = _mask_words(ancestor_mask, total_q, dev)
-    if any(_host_side(x) for x in (cu_q, cu_kv, prefix_len, pack_len)):
+    if _host_side(cu_q, cu_kv, prefix_len, pack_len):
         check_host_metadata(cu_q, prefix_len, pack_len, total_q, total_kv, words, cu_kv=cu_kv)
     cu_q = _as_i32(cu_q, dev)
     cu_kv = _as_i32(cu_kv, dev)
@@ -174,20 +194,19 @@ def varlen_tree_attention(q, k, v, cu_q, cu_kv, prefix_len, pack_len, ancestor_m
     if cu_q.shape[0] != B + 1 or cu_kv.shape[0] != B + 1 or prefix_len.shape[0] != B:
         raise ValueError("cu_q / cu_kv need B+1 entries and prefix_len / pack_len B entries")
     if out is None:
-        out = torch.empty((total_q, H_q, D), dtype=q.dtype, device=dev)
+        out = q.new_empty((total_q, H_q, D))
     elif out.shape != q.shape or out.dtype != q.dtype or out.stride(-1) != 1:
         raise ValueError("out must match q's shape and dtype with a contiguous head dim")
-    lse = torch.empty((total_q, H_q), dtype=torch.float32, device=dev) if return_lse else None
+    lse = q.new_empty((total_q, H_q), dtype=torch.float32) if return_lse else None
     dt = _DTYPES[q.dtype]
-    ws_bytes = lib.cast_tree_attn_workspace_size(B, total_q, total_kv, H_q, H_kv, D, dt, kv_split)
+    ws_bytes = _workspace_bytes(dev.index, B, total_q, total_kv, H_q, H_kv, D, dt, kv_split)
     if ws_bytes and (workspace is None or workspace.numel() * workspace.element_size() < ws_bytes):
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        workspace = q.new_empty(ws_bytes, dtype=torch.uint8)
     status = torch.zeros(1, dtype=torch.int32, device=dev) if check else None
-    args = (_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(out), _lib.ptr(lse),
-            _lib.ptr(cu_q), _lib.ptr(cu_kv), _lib.ptr(prefix_len), _lib.ptr(pack_len), _lib.ptr(mask), words,
+    args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _lib.ptr(lse), cu_q.data_ptr(), cu_kv.data_ptr(),
+            prefix_len.data_ptr(), pack_len.data_ptr(), mask.data_ptr(), words,
             B, total_q, total_kv, H_q, H_kv, D,
-            q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
-            out.stride(0), out.stride(1), dt, float(sm_scale), int(kv_split),
+            *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], dt, float(sm_scale), int(kv_split),
             _lib.ptr(workspace) if ws_bytes else None, ws_bytes, _lib.ptr(status), _lib.stream_of(q))
     with _lib.on_device(dev):
         if _stage_hook is None:
@@ -251,7 +270,7 @@ def store_tree_attention(q, k_store, v_store, k_pack, v_pack, cu_q, prefix_len, 
         total_kv = B * cap + total_q
     total_kv = int(total_kv)
     mask, words = _mask_words(ancestor_mask, total_q, dev)
-    if any(_host_side(x) for x in (cu_q, prefix_len, pack_len)):
+    if _host_side(cu_q, prefix_len, pack_len):
         check_host_metadata(cu_q, prefix_len, pack_len, total_q, total_kv, words, cap=cap)
     cu_q = _as_i32(cu_q, dev)
     prefix_len = _as_i32(prefix_len, dev)
@@ -259,23 +278,21 @@ def store_tree_attention(q, k_store, v_store, k_pack, v_pack, cu_q, prefix_len, 
     if cu_q.shape[0] != B + 1 or prefix_len.shape[0] != B or pack_len.shape[0] != B:
         raise ValueError("cu_q needs B+1 entries and prefix_len / pack_len B entries (B = store batch)")
     if out is None:
-        out = torch.empty((total_q, H_q, D), dtype=q.dtype, device=dev)
+        out = q.new_empty((total_q, H_q, D))
     elif tuple(out.shape) != tuple(q.shape) or out.dtype != q.dtype or out.stride(-1) != 1:
         raise ValueError("out must match q's shape and dtype with a contiguous head dim")
-    lse = torch.empty((total_q, H_q), dtype=torch.float32, device=dev) if return_lse else None
+    lse = q.new_empty((total_q, H_q), dtype=torch.float32) if return_lse else None
     dt = _DTYPES[q.dtype]
-    ws_bytes = lib.cast_tree_attn_workspace_size(B, total_q, total_kv, H_q, H_kv, D, dt, kv_split)
+    ws_bytes = _workspace_bytes(dev.index, B, total_q, total_kv, H_q, H_kv, D, dt, kv_split)
     if ws_bytes and (workspace is None or workspace.numel() * workspace.element_size() < ws_bytes):
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        workspace = q.new_empty(ws_bytes, dtype=torch.uint8)
     status = torch.zeros(1, dtype=torch.int32, device=dev) if check else None
     with _lib.on_device(dev):
         st = lib.cast_tree_attn_store_fwd(
-            _lib.ptr(q), _lib.ptr(k_store), _lib.ptr(v_store), _lib.ptr(k_pack), _lib.ptr(v_pack), _lib.ptr(out),
-            _lib.ptr(lse), _lib.ptr(cu_q), _lib.ptr(prefix_len), _lib.ptr(pack_len), _lib.ptr(mask), words,
-            B, total_q, total_kv, cap, H_q, H_kv, D, q.stride(0), q.stride(1),
-            k_store.stride(0), k_store.stride(1), k_store.stride(2), v_store.stride(0), v_store.stride(1),
-            v_store.stride(2), k_pack.stride(1), k_pack.stride(0), v_pack.stride(1), v_pack.stride(0),
-            out.stride(0), out.stride(1), dt, float(sm_scale), int(kv_split),
+            q.data_ptr(), k_store.data_ptr(), v_store.data_ptr(), k_pack.data_ptr(), v_pack.data_ptr(), out.data_ptr(),
+            _lib.ptr(lse), cu_q.data_ptr(), prefix_len.data_ptr(), pack_len.data_ptr(), mask.data_ptr(), words,
+            B, total_q, total_kv, cap, H_q, H_kv, D, *q.stride()[:2], *k_store.stride()[:3], *v_store.stride()[:3],
+            *k_pack.stride()[1::-1], *v_pack.stride()[1::-1], *out.stride()[:2], dt, float(sm_scale), int(kv_split),
             _lib.ptr(workspace) if ws_bytes else None, ws_bytes, _lib.ptr(status), _lib.stream_of(q))
     _lib.check(st, "cast_tree_attn_store_fwd")
     if check:

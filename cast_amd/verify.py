@@ -82,8 +82,8 @@ def greedy_accept(logits, cu_q, parent, token, *, check=False):
     if logits.stride(1) != 1:
         logits = logits.contiguous()
     total_q, V = logits.shape
-    cu_q = torch.as_tensor(cu_q, device=dev).to(torch.int32).contiguous()
-    parent = torch.as_tensor(parent, device=dev).to(torch.int32).contiguous()
+    cu_q = _i32_on(cu_q, dev)
+    parent = _i32_on(parent, dev)
     token = torch.as_tensor(token, device=dev).to(torch.int64).contiguous()
     if parent.shape[0] != total_q or token.shape[0] != total_q:
         raise ValueError("parent and token need one entry per logits row")

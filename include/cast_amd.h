@@ -326,8 +326,9 @@ int cast_store_append(const void *const *k_pack, const void *const *v_pack, void
  *   score double: [batch][127] nodes in pop order;  n_nodes int32 [batch]
  *   1 <= L <= 255, 1 <= k <= 16.  Log-probs must not be NaN or +inf (the
  *   reference's heap has no defined order then).  Positions whose log-probs
- *   are non-increasing in rank (top-k output) take a sorted-frontier search;
- *   others a scan of every pushed candidate; both pop the heap's order.
+ *   are non-increasing in rank (top-k output) are built depth by depth or by
+ *   a sorted-frontier search, others by a scan of every pushed candidate; all
+ *   give the heap's order.
  * ------------------------------------------------------------------- */
 int cast_draft_topk(const void *logits, int64_t logits_ld, int32_t rows, int32_t vocab,
                     int32_t dtype, int32_t k, int64_t *top_idx, float *top_lp, int32_t splits,
@@ -338,6 +339,12 @@ int cast_build_trees(const int64_t *top_idx, const void *top_lp, int32_t lp_dtyp
                      int32_t L, int32_t k, const int32_t *budget, int64_t *token, int32_t *depth,
                      int32_t *parent, double *score, int32_t *n_nodes, int32_t *status,
                      cast_stream_t stream);
+/* cast_build_trees with one node count for every tree instead of a budget
+ * array (no tensor to fill and no launch to fill it). */
+int cast_build_trees_uniform(const int64_t *top_idx, const void *top_lp, int32_t lp_dtype,
+                             int32_t batch, int32_t L, int32_t k, int32_t nodes, int64_t *token,
+                             int32_t *depth, int32_t *parent, double *score, int32_t *n_nodes,
+                             int32_t *status, cast_stream_t stream);
 
 
 #ifdef __cplusplus
