@@ -63,6 +63,19 @@ struct Bf16 {
         }
     }
 };
+// A float pair as the sum of three bf16 pairs, each the rounding of what the
+// ones before it leave: 8 bits a term and signed remainders hold all 24 bits
+// (of values that do not round to infinity).
+__device__ __forceinline__ void split_bf16x3(float lo, float hi, uint32_t &w0, uint32_t &w1, uint32_t &w2) {
+    w0 = pack_bf16x2(lo, hi);
+    lo -= __builtin_bit_cast(float, w0 << 16);
+    hi -= __builtin_bit_cast(float, w0 & 0xffff0000u);
+    w1 = pack_bf16x2(lo, hi);
+    lo -= __builtin_bit_cast(float, w1 << 16);
+    hi -= __builtin_bit_cast(float, w1 & 0xffff0000u);
+    w2 = pack_bf16x2(lo, hi);
+}
+
 struct Fp16 {
     using vec8 = f16x8;
     static __device__ __forceinline__ floatx16 mma(vec8 a, vec8 b, floatx16 c) {

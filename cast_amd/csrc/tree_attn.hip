@@ -17,13 +17,13 @@
 //   O^T += V^T P^T with the same instruction, P^T taken straight from the
 //   S^T accumulator registers (a lane's 16 score values are exactly the 8+8
 //   k-slots it must supply), V^T read from a transposed LDS copy.  fp32
-//   inputs with head_dim 64/128/256 run the same structure on
-//   v_mfma_f32_32x32x2_f32 (tree_attn_f32_kernel).  Other head dims
+//   inputs run the same structure with every operand as three bf16 terms
+//   (tree_attn_f32_kernel).  Other head dims
 //   (multiples of 8 up to 256) take padded instances of both, or a scalar
 //   kernel where bases, strides or sizes do not allow those.  Head_dim 256
 //   runs one wave per SIMD (512 registers a lane).
-// K/V tiles of 64 keys (32 for fp32 at head_dim 256) are double-buffered
-// through LDS with 16-byte loads; the ancestor words are only consulted on
+// K/V tiles of 64 keys (32 for fp32) go through LDS, double-buffered where
+// two fit; the ancestor words are only consulted on
 // the tile(s) holding pack keys, and pack tiles past the last key any row
 // of a workgroup sees are skipped.
 // The online softmax works in base 2 with a lazy rescale: the running max
@@ -283,6 +283,8 @@ __device__ __forceinline__ bool batch_fits(const AttnArgs &a, const BatchTotals 
 // Splits below 8 tiles only where 8 would make fewer than 192 items: a split
 // costs a prologue and a partial of the block's rows written and read again
 // (8 requests of 300 to 2k keys: 32.4 us at 4 tiles, 28.1 at 7, 29.7 at 10).
+// An fp32 tile takes about three times as long beside the same overhead, so
+// there the limits are 4 tiles and one item per slot.
 // Measured, bf16, against one chunk from the batch's averages: 8 requests of
 // 1k to 8k keys, D = 128, 83.6 -> 70.9 us; 32 requests of 300 to 4k keys with
 // packs of 2 to 64 148.9 -> 95.2 us (with 4-wave workgroups, see waves_for);
@@ -295,7 +297,8 @@ __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok, int *fit) {
     int L = max((int)((float)W * a.hkv_per_slot) - 1, 1);
 #pragma unroll
     for (int i = 0; i < 3; ++i) L += (int64_t)L * a.slots < total ? 1 : 0;   // the exact ceiling
-    L = max(L, total < 8 * 192 ? max((int)total / 192, a.chunk >> 6) : 8);
+    const int few = a.esz == 4 ? a.slots : 192, least = a.esz == 4 ? 4 : 8;
+    L = max(L, total < (int64_t)least * few ? max(udiv((int)total, few), a.chunk >> 6) : least);
     auto cand = [&](int w) { return (L * (w < 3 ? 8 + w : 12) + 7) >> 3; };
     const int w = threadIdx.x >> 6;
     if (w < 4) {
@@ -1324,31 +1327,31 @@ void tree_attn_mfma_kernel(AttnArgs a) {
 }
 // --------------------------------------------------------------------------
 // MFMA kernel for fp32 inputs: head_dim D in {64, 128, 256}, WAVES waves x
-// 32 query rows, v_mfma_f32_32x32x2_f32.  The reference hook runs its kernel on
-// fp32 copies of q/k/v (cast_trees/serving.py:68-71), where p stays fp32
-// for the value product (tree_attn.py:66,87 cast p to the input dtype):
-// so does this kernel.  Same structure as the bf16 kernel: S^T = K Q^T with
-// each lane owning one query column, P^T straight from the S^T
-// accumulators, O^T += V^T P^T.  A 32x32x2 step takes one value per lane
-// per operand: in the QK product lane (l32, g) supplies head-dim element
-// (D/2)*g + step of its key and of its query, so a lane's K operands for
-// four steps are one 16-byte LDS read; in the PV product it supplies the
-// value of key 8*(e/4) + 4*g + e%4 at step e, which is exactly its own
-// accumulator element e.  V sits in LDS as V'[key][vpos(l)*DB + db] =
-// V[key][32*db + l], so one read gives lane l the operands of all DB
-// output blocks; vpos(l) = 8*(l%4) + l/4 (a 4x8 transpose of the group
-// index) puts the eight groups of a key that one staging store covers
-// (l = 4*lg + i, lg = 0..7) side by side, on distinct banks; the reads
-// take a permutation of the same row.  The product is MFMA-bound (16 x the
-// bf16 cycles per flop): staging and softmax are small beside it.
+// 32 query rows.  The reference hook runs its kernel on fp32 copies of q/k/v
+// (cast_trees/serving.py:68-71), where p stays fp32 for the value product
+// (tree_attn.py:66,87 cast p to the input dtype): so does this kernel.
+//
+// Structure of the bf16 kernel, with every operand as three bf16 terms that
+// add up to the float (8 bits a term, h + m + l) and six of the nine products
+// of the terms: l h, h l, m m, m h, h m, h h, the smallest first.  The three
+// left out are below 2^-26 of the product.  v_mfma_f32_32x32x2_f32, which ran
+// here before, takes 16 times the bf16 cycles per product and rounds its sum
+// every 2 products; six bf16 steps of 16 products take 6 / 16 of that and
+// round at most as often, so the error against 64 bits is no larger
+// (relative 2-norm, 8 requests of 1k to 4k keys at D = 128: 4.2e-7 against
+// 6.1e-7; with scores six times as wide 5.9e-7 against 1.5e-6).  A row that meets an infinity or a NaN, where a
+// remainder is no number, is computed again in plain fp32 (exact_row).
+//
+// K and V are split once per tile while they are staged, Q once, P per tile
+// in registers.  Tiles of 32 keys: K [term][key][d] and V^T [term][d][key']
+// (keys permuted as in the bf16 kernel) take 57 KB at D = 128.  8 waves
+// double-buffer them, one workgroup per CU; 4 waves take one buffer and two
+// barriers a tile, two workgroups per CU; D = 256 takes one buffer of 112 KB
+// and one wave per SIMD.  Bound by the MFMA pipe and the splitting beside it:
+// 8 requests of 1k to 4k keys, packs of 2 to 64, D = 128 169.2 -> 98.1 us; 8 of
+// 2000 keys, packs of 128 295 -> 202 us; D = 64 130 -> 86 us; D = 256 (whose
+// one wave per SIMD spills 60 registers) 590 -> 508 us.
 // --------------------------------------------------------------------------
-// Key tiles hold 64 keys (two 32-key blocks), or 32 at head dim 256, where
-// two double-buffered 64-key K and V' tiles would not fit in LDS.
-// WPE: waves per SIMD the register budget is sized for: 2, except the
-// 4-wave head-dim-128 and -256 instances (1): the former's threads each
-// stage twice the 8-wave instance's share of a tile, the latter holds 128
-// registers of Q and 128 of O per lane; their 133-135 KB of LDS leave room
-// for one workgroup (one wave per SIMD) per CU anyway.
 // PAD: head dims the instances do not name (multiples of 8 below D), the
 // missing elements zeros.
 template <int D, int WAVES, bool STORE, int WPE = 2, bool SKI = false, bool PAD = false>
@@ -1357,20 +1360,20 @@ void tree_attn_f32_kernel(AttnArgs a) {
     constexpr uint32_t kNowhere = 0x7ffffff0u;   // byte offset past every source: loads as zeros
     const int dr = PAD ? a.D : D;                // the call's head dim
     constexpr int NT = WAVES * 64;
-    constexpr int BN = D <= 128 ? 64 : 32;  // keys per tile
-    constexpr int NKB = BN / 32;           // 32-key MFMA blocks per tile
+    constexpr int BN = 32;                 // keys per tile
     constexpr int ROWS = WAVES * 32;       // query rows per workgroup
-    constexpr int DH = D / 2;              // k-steps per 32-key block (2 head-dim values each)
+    constexpr int DSTEPS = D / 16;         // MFMA k-steps over the head dim
     constexpr int DB = D / 32;             // 32-row blocks of O^T
-    constexpr int KPAD = D + 4;            // LDS row stride (floats)
-    constexpr int KCH = BN * D / 4;        // 16-byte K chunks per tile
-    constexpr int K_PER_T = (KCH + NT - 1) / NT;
-    constexpr int VUNITS = BN * 8;         // (key, group of 4 l) staging units of V
-    constexpr int V_PER_T = (VUNITS + NT - 1) / NT;
-    typedef float floatxDB __attribute__((ext_vector_type(DB)));
+    constexpr int NBUF = WAVES == 8 ? 2 : 1;
+    constexpr int KPAD = D + 8;            // K row stride in LDS (elements)
+    constexpr int VPAD = BN + 8;           // V^T row stride in LDS (elements)
+    constexpr int KU = BN * D / 8;         // (key, 8 d) staging units of K
+    constexpr int K_PER_T = (KU + NT - 1) / NT;
+    constexpr int VU = BN / 8 * D;         // (8 keys, d) staging units of V
+    constexpr int V_PER_T = (VU + NT - 1) / NT;
 
-    __shared__ __attribute__((aligned(16))) float Ks[2][BN * KPAD];
-    __shared__ __attribute__((aligned(16))) float Vs[2][BN * KPAD];
+    __shared__ __attribute__((aligned(16))) uint16_t Ks[NBUF][3][BN * KPAD];
+    __shared__ __attribute__((aligned(16))) uint16_t Vt[NBUF][3][D * VPAD];
     __shared__ EpiArgs epi;
     __shared__ int pack_hi[WAVES];   // auto_split's LDS, then per wave the last pack key a row of it sees
     __shared__ SkReq skr[SKI ? 64 : 1];
@@ -1394,18 +1397,114 @@ void tree_attn_f32_kernel(AttnArgs a) {
     const int qtok = sq.q0 + qi;
     const int qhead = h * a.G + (qvalid ? r - qi * a.G : 0);
     const KvView<float> kv(a.kv, sq, h);
+    const float *qp = static_cast<const float *>(a.q);
 
-    // Q operand: head-dim elements [DH*g, DH*g + DH) of this lane's query
-    float qf[DH];
+    const int pre_end = min(k_end, sq.S);
+    const int n_pre = k_begin < pre_end ? (pre_end - k_begin + BN - 1) / BN : 0;
+    const int pk_begin = max(k_begin, sq.S);
+    const int n_pack = k_end > pk_begin ? (k_end - pk_begin + BN - 1) / BN : 0;
+    auto tile_t0 = [&](int t) __attribute__((always_inline)) { return t < n_pre ? k_begin + t * BN : pk_begin + (t - n_pre) * BN; };
+    auto tile_valid = [&](int t) __attribute__((always_inline)) { return min(BN, (t < n_pre ? pre_end : k_end) - tile_t0(t)); };
+
+    u32x4 kst[K_PER_T][2];
+    uint32_t vst[V_PER_T][8];
+    auto fetch_from = [&](const float *kb, const float *vb, int nrows, uint32_t ksb, uint32_t vsb,
+                          uint32_t row0) __attribute__((always_inline)) {
+        const __amdgpu_buffer_rsrc_t krs = seg_rsrc(kb, nrows, ksb, dr * 4);
+        const __amdgpu_buffer_rsrc_t vrs = seg_rsrc(vb, nrows, vsb, dr * 4);
+#pragma unroll
+        for (int it = 0; it < K_PER_T; ++it) {
+            const int u = tid + it * NT;
+            if (u >= KU) break;
+            const int key = u / (D / 8), dch = u % (D / 8);
+            const uint32_t off = PAD && dch * 8 >= dr ? kNowhere - 16 : __umul24(row0 + key, ksb) + dch * 32;
+            kst[it][0] = load16(krs, off);
+            kst[it][1] = load16(krs, off + 16);
+        }
+#pragma unroll
+        for (int it = 0; it < V_PER_T; ++it) {
+            const int u = tid + it * NT;
+            if (u >= VU) break;
+            const int d = u % D, oc = u / D;
+            // key i of stored group oc: 16*(oc/2) + 4*(oc%2) + 8*(i/4) + i%4
+            const uint32_t v0 = row0 + 16 * (oc >> 1) + 4 * (oc & 1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t off = PAD && d >= dr ? kNowhere : __umul24(v0 + 8 * (i >> 2) + (i & 3), vsb) + d * 4;
+                vst[it][i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(vrs, (int)off, 0, 0);
+            }
+        }
+    };
+    auto fetch = [&](int t) __attribute__((always_inline)) {
+        const int t0 = tile_t0(t);
+        if (!STORE || t < n_pre)
+            fetch_from(kv.kpre, kv.vpre, STORE ? sq.S : sq.T, (uint32_t)kv.kpre_t * 4u, (uint32_t)kv.vpre_t * 4u,
+                       (uint32_t)t0);
+        else
+            fetch_from(kv.kpack, kv.vpack, sq.P, (uint32_t)kv.kpack_t * 4u, (uint32_t)kv.vpack_t * 4u,
+                       (uint32_t)(t0 - sq.S));
+    };
+    // eight floats into the three terms' 16-byte rows
+    auto split8 = [](const float (&x)[8], u32x4 (&w)[3]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t w0, w1, w2;
+            split_bf16x3(x[2 * e], x[2 * e + 1], w0, w1, w2);
+            w[0][e] = w0;
+            w[1][e] = w1;
+            w[2][e] = w2;
+        }
+    };
+    auto publish = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int it = 0; it < K_PER_T; ++it) {
+            const int u = tid + it * NT;
+            if (u >= KU) break;
+            const int key = u / (D / 8), dch = u % (D / 8);
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t bits = kst[it][e >> 2][e & 3];
+                x[e] = __builtin_bit_cast(float, bits);
+            }
+            u32x4 w[3];
+            split8(x, w);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4 *>(&Ks[buf][i][key * KPAD + dch * 8]) = w[i];
+        }
+#pragma unroll
+        for (int it = 0; it < V_PER_T; ++it) {
+            const int u = tid + it * NT;
+            if (u >= VU) break;
+            const int d = u % D, oc = u / D;
+            float x[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = __builtin_bit_cast(float, vst[it][e]);
+            u32x4 w[3];
+            split8(x, w);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x4 *>(&Vt[buf][i][d * VPAD + oc * 8]) = w[i];
+        }
+    };
+
+    // Q^T operand: head-dim elements [ds*16 + g*8, +8) of this lane's query
+    bf16x8 qf[3][DSTEPS];
     {
-        const float *src = static_cast<const float *>(a.q) + (int64_t)qtok * a.q_tok + (int64_t)qhead * a.q_head +
-                           DH * g;
+        const float *src = qp + (int64_t)qtok * a.q_tok + (int64_t)qhead * a.q_head + g * 8;
 #pragma unroll
-        for (int i = 0; i < DH / 4; ++i) {
-            const floatx4 x = qvalid && (!PAD || DH * g + 4 * i < dr) ? *reinterpret_cast<const floatx4 *>(src + 4 * i)
-                                                                      : floatx4{};
+        for (int ds = 0; ds < DSTEPS; ++ds) {
+            float x[8];
+            const bool in = qvalid && (!PAD || ds * 16 + g * 8 < dr);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) qf[4 * i + j] = x[j];
+            for (int i = 0; i < 2; ++i) {
+                const floatx4 y = in ? *reinterpret_cast<const floatx4 *>(src + ds * 16 + 4 * i) : floatx4{};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * i + e] = y[e];
+            }
+            u32x4 w[3];
+            split8(x, w);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) qf[i][ds] = __builtin_bit_cast(bf16x8, w[i]);
         }
     }
     uint64_t mw0 = 0, mw1 = 0;
@@ -1420,79 +1519,6 @@ void tree_attn_f32_kernel(AttnArgs a) {
     for (int db = 0; db < DB; ++db) o[db] = floatx16{};
     float m = -INFINITY, msafe = 0.f, lsum = 0.f;
     const float c = a.scale_log2;
-
-    const int pre_end = min(k_end, sq.S);
-    const int n_pre = k_begin < pre_end ? (pre_end - k_begin + BN - 1) / BN : 0;
-    const int pk_begin = max(k_begin, sq.S);
-    const int n_pack = k_end > pk_begin ? (k_end - pk_begin + BN - 1) / BN : 0;
-    auto tile_t0 = [&](int t) __attribute__((always_inline)) { return t < n_pre ? k_begin + t * BN : pk_begin + (t - n_pre) * BN; };
-    auto tile_valid = [&](int t) __attribute__((always_inline)) { return min(BN, (t < n_pre ? pre_end : k_end) - tile_t0(t)); };
-
-    const uint32_t ksb_pre = (uint32_t)kv.kpre_t * 4u, vsb_pre = (uint32_t)kv.vpre_t * 4u;
-    const uint32_t ksb_pack = (uint32_t)kv.kpack_t * 4u, vsb_pack = (uint32_t)kv.vpack_t * 4u;
-    const int rows_pre = STORE ? sq.S : sq.T;
-    const __amdgpu_buffer_rsrc_t kr_pre = seg_rsrc(kv.kpre, rows_pre, ksb_pre, dr * 4);
-    const __amdgpu_buffer_rsrc_t vr_pre = seg_rsrc(kv.vpre, rows_pre, vsb_pre, dr * 4);
-    const __amdgpu_buffer_rsrc_t kr_pack = seg_rsrc(kv.kpack, STORE ? sq.P : 0, ksb_pack, dr * 4);
-    const __amdgpu_buffer_rsrc_t vr_pack = seg_rsrc(kv.vpack, STORE ? sq.P : 0, vsb_pack, dr * 4);
-    u32x4 kst[K_PER_T];
-    u32x4 vst[V_PER_T][DB];
-    auto fetch = [&](int t) __attribute__((always_inline)) {
-        const bool pre = !STORE || t < n_pre;
-        const int t0 = tile_t0(t);
-        const uint32_t row0 = (uint32_t)(pre ? t0 : t0 - sq.S);
-        const __amdgpu_buffer_rsrc_t krs = pre ? kr_pre : kr_pack;
-        const __amdgpu_buffer_rsrc_t vrs = pre ? vr_pre : vr_pack;
-        const uint32_t ksb = pre ? ksb_pre : ksb_pack;
-        const uint32_t vsb = pre ? vsb_pre : vsb_pack;
-#pragma unroll
-        for (int it = 0; it < K_PER_T; ++it) {
-            const int cidx = tid + it * NT;
-            if (cidx >= KCH) break;
-            const int key = cidx / (D / 4), dch = cidx % (D / 4);
-            const uint32_t off = __umul24(row0 + key, ksb) + dch * 16;
-            kst[it] = load16(krs, PAD && dch * 4 >= dr ? kNowhere : off);
-        }
-#pragma unroll
-        for (int it = 0; it < V_PER_T; ++it) {
-            const int u = tid + it * NT;
-            if (u >= VUNITS) break;
-            const int key = u >> 3, lg = u & 7;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-                vst[it][db] = load16(vrs, PAD && db * 32 + lg * 4 >= dr ? kNowhere
-                                                                        : __umul24(row0 + key, vsb) + db * 128 + lg * 16);
-        }
-    };
-    // register -> LDS: K as is; V with d = 32*db + l stored at vpos(l)*DB + db
-    auto vpos = [](int l) __attribute__((always_inline)) { return 8 * (l & 3) + (l >> 2); };
-    auto publish = [&](int buf) __attribute__((always_inline)) {
-#pragma unroll
-        for (int it = 0; it < K_PER_T; ++it) {
-            const int cidx = tid + it * NT;
-            if (cidx >= KCH) break;
-            const int key = cidx / (D / 4), dch = cidx % (D / 4);
-            *reinterpret_cast<u32x4 *>(&Ks[buf][key * KPAD + dch * 4]) = kst[it];
-        }
-#pragma unroll
-        for (int it = 0; it < V_PER_T; ++it) {
-            const int u = tid + it * NT;
-            if (u >= VUNITS) break;
-            const int key = u >> 3, lg = u & 7;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                floatxDB w;
-#pragma unroll
-                for (int db = 0; db < DB; ++db) {
-                    // element i through a scalar: hipcc (ROCm 7.2) reads element 0
-                    // for every i of __builtin_bit_cast(float, vec[db][i])
-                    const uint32_t bits = vst[it][db][i];
-                    w[db] = __builtin_bit_cast(float, bits);
-                }
-                *reinterpret_cast<floatxDB *>(&Vs[buf][key * KPAD + vpos(4 * lg + i) * DB]) = w;
-            }
-        }
-    };
 
     // pack tiles past the last pack key any row of the workgroup sees are
     // skipped (a one-unit workgroup; the stream-K segments keep their tiles)
@@ -1527,78 +1553,48 @@ void tree_attn_f32_kernel(AttnArgs a) {
     // (read from LDS, so held in a vector register: made scalar again)
     const int ntiles = __builtin_amdgcn_readfirstlane(n_pre + n_pack_live);
 
-    if (ntiles > 0) fetch(0);
-    for (int t = 0; t < ntiles; ++t) {
-        const int buf = t & 1;
-        publish(buf);
-        __syncthreads();
-        if (t + 1 < ntiles) fetch(t + 1);
-        if (!active) continue;
+    auto tile_body = [&](int t, int buf) __attribute__((always_inline)) {
         const int t0 = tile_t0(t);
         const int valid = tile_valid(t);
         const bool pack_tile = t >= n_pre;
-        // in a pack tile, the 32-key blocks no row of the wave sees are
-        // skipped: scores -inf, no PV product
-        bool live[NKB];
+        // a pack tile no row of the wave sees adds nothing
+        if (!SKI && pack_tile && !block_live(mw0, mw1, t0 - sq.S, valid)) return;
+        // S^T = K Q^T: the small products and the leading ones in a sum each
+        // (one sum at D = 256, which has no registers for two)
+        constexpr bool kTwoSums = D <= 128;
+        floatx16 sm = floatx16{}, s = floatx16{};
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-            live[kb] = SKI || !pack_tile || block_live(mw0, mw1, t0 - sq.S + 32 * kb, valid - 32 * kb);
-        // S^T = K Q^T, the two 32-key blocks' chains interleaved
-        floatx16 s[NKB];
+        for (int ds = 0; ds < DSTEPS; ++ds) {
+            bf16x8 k[3];
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) s[kb] = floatx16{};
-        if (NKB == 2 && live[0] && live[NKB - 1]) {
-#pragma unroll
-            for (int i = 0; i < DH / 4; ++i) {
-                const floatx4 k0 = *reinterpret_cast<const floatx4 *>(&Ks[buf][l32 * KPAD + DH * g + 4 * i]);
-                const floatx4 k1 =
-                    *reinterpret_cast<const floatx4 *>(&Ks[buf][((NKB - 1) * 32 + l32) * KPAD + DH * g + 4 * i]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(k0[j], qf[4 * i + j], s[0], 0, 0, 0);
-                    s[NKB - 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(k1[j], qf[4 * i + j], s[NKB - 1], 0, 0, 0);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                if (!live[kb]) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) s[kb][e] = -INFINITY;
-                    continue;
-                }
-#pragma unroll
-                for (int i = 0; i < DH / 4; ++i) {
-                    const floatx4 kk =
-                        *reinterpret_cast<const floatx4 *>(&Ks[buf][(kb * 32 + l32) * KPAD + DH * g + 4 * i]);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        s[kb] = __builtin_amdgcn_mfma_f32_32x32x2f32(kk[j], qf[4 * i + j], s[kb], 0, 0, 0);
-                }
-            }
+            for (int i = 0; i < 3; ++i)
+                k[i] = *reinterpret_cast<const bf16x8 *>(&Ks[buf][i][l32 * KPAD + ds * 16 + g * 8]);
+            sm = Bf16::mma(k[2], qf[0][ds], sm);
+            sm = Bf16::mma(k[0], qf[2][ds], sm);
+            sm = Bf16::mma(k[1], qf[1][ds], sm);
+            sm = Bf16::mma(k[1], qf[0][ds], sm);
+            sm = Bf16::mma(k[0], qf[1][ds], sm);
+            if constexpr (kTwoSums)
+                s = Bf16::mma(k[0], qf[0][ds], s);
+            else
+                sm = Bf16::mma(k[0], qf[0][ds], sm);
         }
+        s = kTwoSums ? s + sm : sm;
         // visibility on pack tiles and partial tiles (as in the bf16 kernel)
         if (pack_tile || valid < BN) {
+            const int k0 = 4 * g;
+            const int lim = valid - k0;
+            uint32_t vis = pack_tile ? vis_window(mw0, mw1, t0 - sq.S + k0) : ~0u;
+            vis &= lim >= 32 ? ~0u : (lim <= 0 ? 0u : ((1u << lim) - 1u));
 #pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                const int k0 = kb * 32 + 4 * g;
-                const int lim = valid - k0;
-                uint32_t vis = pack_tile ? vis_window(mw0, mw1, t0 - sq.S + k0) : ~0u;
-                vis &= lim >= 32 ? ~0u : (lim <= 0 ? 0u : ((1u << lim) - 1u));
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int off = 8 * (e >> 2) + (e & 3);
-                    s[kb][e] = (vis >> off) & 1u ? s[kb][e] : -INFINITY;
-                }
+            for (int e = 0; e < 16; ++e) {
+                const int off = 8 * (e >> 2) + (e & 3);
+                s[e] = (vis >> off) & 1u ? s[e] : -INFINITY;
             }
         }
-        float lmax = s[0][0];
+        float lmax = s[0];
 #pragma unroll
-        for (int e = 1; e < 16; ++e) lmax = fmaxf(lmax, s[0][e]);
-#pragma unroll
-        for (int kb = 1; kb < NKB; ++kb)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) lmax = fmaxf(lmax, s[kb][e]);
+        for (int e = 1; e < 16; ++e) lmax = fmaxf(lmax, s[e]);
         if (__any(lmax * c > m + kRescaleSlack)) {
             const float mx = fmaxf(lmax, partner32(lmax)) * c;
             const float mn = fmaxf(m, mx);
@@ -1610,51 +1606,83 @@ void tree_attn_f32_kernel(AttnArgs a) {
             msafe = m == -INFINITY ? 0.f : m;
         }
         float acc = 0.f;
+        bf16x8 pb[2][3];
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
+        for (int hf = 0; hf < 2; ++hf) {
+            u32x4 w[3];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                s[kb][e] = __builtin_amdgcn_exp2f(fmaf(s[kb][e], c, -msafe));
-                acc += s[kb][e];
+            for (int e = 0; e < 4; ++e) {
+                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[8 * hf + 2 * e], c, -msafe));
+                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[8 * hf + 2 * e + 1], c, -msafe));
+                acc += p0;
+                acc += p1;
+                uint32_t x[3];
+                Bf16::split2(p0, p1, x);
+#pragma unroll
+                for (int i = 0; i < 3; ++i) w[i][e] = x[i];
             }
+#pragma unroll
+            for (int i = 0; i < 3; ++i) pb[hf][i] = __builtin_bit_cast(bf16x8, w[i]);
+        }
         lsum += acc;
-        // O^T += V^T P^T: step e of block kb is key 32*kb + 8*(e/4) + 4*g + e%4
+        // O^T += V^T P^T over two 16-key slices
 #pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) {
-            if (!live[kb]) continue;
+        for (int hf = 0; hf < 2; ++hf) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int key = kb * 32 + 8 * (e >> 2) + 4 * g + (e & 3);
-                const floatxDB vv = *reinterpret_cast<const floatxDB *>(&Vs[buf][key * KPAD + vpos(l32) * DB]);
+            for (int db = 0; db < DB; ++db) {
+                bf16x8 v[3];
 #pragma unroll
-                for (int db = 0; db < DB; ++db)
-                    o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv[db], s[kb][e], o[db], 0, 0, 0);
+                for (int i = 0; i < 3; ++i)
+                    v[i] = *reinterpret_cast<const bf16x8 *>(&Vt[buf][i][(db * 32 + l32) * VPAD + hf * 16 + g * 8]);
+                o[db] = Bf16::mma(v[2], pb[hf][0], o[db]);
+                o[db] = Bf16::mma(v[0], pb[hf][2], o[db]);
+                o[db] = Bf16::mma(v[1], pb[hf][1], o[db]);
+                o[db] = Bf16::mma(v[1], pb[hf][0], o[db]);
+                o[db] = Bf16::mma(v[0], pb[hf][1], o[db]);
+                o[db] = Bf16::mma(v[0], pb[hf][0], o[db]);
             }
         }
+    };
+
+    if (ntiles > 0) fetch(0);
+    for (int t = 0; t < ntiles; ++t) {
+        const int buf = NBUF == 2 ? t & 1 : 0;
+        publish(buf);
+        __syncthreads();
+        if (t + 1 < ntiles) fetch(t + 1);
+        if (active) tile_body(t, buf);
+        if (NBUF == 1 && t + 1 < ntiles) __syncthreads();
     }
 
-    if (active && qvalid) {
+    if (active) {
         const float ltot = lsum + partner32(lsum);
         const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
         const float lse2 = ltot > 0.f ? msafe + log2f(ltot) : -INFINITY;
         const EpiArgs e = epi;
-        float *dst = nullptr;
-        if (e.final_out) {
-            dst = static_cast<float *>(e.out) + (int64_t)qtok * e.o_tok + (int64_t)qhead * e.o_head;
-            if (e.lse && g == 0) e.lse[(int64_t)qtok * e.Hq + qhead] = lse2 * kLn2;
-        } else {
-            // static split: row (token, head) of the partial rows; stream-K:
-            // row wave * 32 + l32 of the workgroup's slot
-            const int64_t prow = e.slot >= 0 ? (int64_t)e.slot * ROWS + wave * 32 + l32 : e.prow0 + qtok;
-            if (prow >= e.part_rows) {
-                raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
-            } else {
-                const int64_t orow = e.slot >= 0 ? prow : prow * e.Hq + qhead;
-                dst = e.part_o + orow * dr;
-                if (g == 0) (e.slot >= 0 ? e.sk_lse : e.part_lse)[orow] = lse2;
-            }
-        }
-        if (dst) {
+        // static split: row (token, head) of the partial rows; stream-K:
+        // row wave * 32 + l32 of the workgroup's slot
+        const int64_t prow = e.slot >= 0 ? (int64_t)e.slot * ROWS + wave * 32 + l32 : e.prow0 + qtok;
+        const int64_t orow = e.slot >= 0 ? prow : prow * e.Hq + qhead;
+        const bool fits = e.final_out || prow < e.part_rows;
+        if (qvalid && !fits) raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
+        float *dst = !fits           ? nullptr
+                     : e.final_out ? static_cast<float *>(e.out) + (int64_t)qtok * e.o_tok + (int64_t)qhead * e.o_head
+                                   : e.part_o + orow * dr;
+        float *lse_dst = !fits           ? nullptr
+                         : !e.final_out ? (e.slot >= 0 ? e.sk_lse : e.part_lse) + orow
+                         : e.lse        ? e.lse + (int64_t)qtok * e.Hq + qhead
+                                        : nullptr;
+        const float lse_unit = e.final_out ? kLn2 : 1.f;
+        // NaN as soon as one of the row's sums is not finite
+        float z = ltot * 0.f;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
+        const uint64_t bad = __ballot(qvalid && !(z == 0.f));
+        const uint32_t redo = (uint32_t)bad | (uint32_t)(bad >> 32);
+        if (qvalid && fits && !(redo >> l32 & 1)) {
+            if (lse_dst && g == 0) *lse_dst = lse2 * lse_unit;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -1665,6 +1693,23 @@ void tree_attn_f32_kernel(AttnArgs a) {
                                        o[db][4 * r4 + 3] * inv};
                     *reinterpret_cast<floatx4 *>(dst + d) = w;
                 }
+        }
+        for (uint32_t left = redo; left; left &= left - 1) {
+            const int i = __builtin_ctz(left);
+            float *const row = reinterpret_cast<float *>(bcast64(reinterpret_cast<int64_t>(dst), i));
+            float *const row_lse = reinterpret_cast<float *>(bcast64(reinterpret_cast<int64_t>(lse_dst), i));
+            if (!row) continue;
+            float acc[4], mr, lr;
+            exact_row<float, Bf16>(kv, sq.S, k_begin, k_end,
+                                   qp + (int64_t)bcast(qtok, i) * a.q_tok + (int64_t)bcast(qhead, i) * a.q_head, dr,
+                                   (uint64_t)bcast64((int64_t)mw0, i), (uint64_t)bcast64((int64_t)mw1, i), c, acc, mr,
+                                   lr);
+            const float ir = lr > 0.f ? 1.f / lr : 0.f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (lane + 64 * j < dr) row[lane + 64 * j] = acc[j] * ir;
+            if (row_lse && lane == 0)
+                *row_lse = (lr > 0.f ? (mr == -INFINITY ? 0.f : mr) + log2f(lr) : -INFINITY) * lse_unit;
         }
     }
     } while (SKI && next_unit(a, cur, wu, skr));
@@ -2090,7 +2135,7 @@ static int padded_dim(int32_t dtype, int32_t D) {
     return D < 64 ? 64 : D <= 96 ? 96 : D < 128 ? 128 : D <= 192 ? 192 : 256;
 }
 
-// Waves per workgroup (32 query rows each).  16-bit inputs take 8 waves (256
+// Waves per workgroup (32 query rows each): 8 (256
 // rows, one workgroup per CU) when the average pack fills most of them, else 4
 // (128 rows, two workgroups per CU at head dim 128, three at 64): with few
 // rows a tile's time is the latency of one wave's QK -> softmax -> PV chain
@@ -2100,14 +2145,12 @@ static int padded_dim(int32_t dtype, int32_t D) {
 // against 117; 8 of 256 rows 92 against 85, one of 512 rows 111 against 95.
 // 2 waves (64 rows) were slower than 4 even at 64 rows (one request, 2064
 // keys: 17.5 against 16.4): each thread stages twice as much.
-// fp32 sizes by the largest possible pack (one workgroup per CU either way).
 // Head_dim 256 always runs 4 waves, one per SIMD: fewer threads would each
 // stage more of its 32 KB tiles than the registers hold.
 static int waves_for(int32_t batch, int32_t total_q, int32_t G, int32_t dtype, int32_t D) {
     // the padded 16-bit instances have 4 waves only
     const int dp = padded_dim(dtype, D);
     if (D == 256 || dp == 256 || (dp && dtype != CAST_FP32)) return 4;
-    if (dtype == CAST_FP32) return (int64_t)(total_q < kMaxPack ? total_q : kMaxPack) * G <= 128 ? 4 : 8;
     const int64_t p_avg = ((int64_t)total_q + batch - 1) / batch;
     return (p_avg < kMaxPack ? p_avg : kMaxPack) * G <= 192 ? 4 : 8;
 }
@@ -2169,7 +2212,7 @@ static AttnKernel f32_instance(bool store) {
 template <bool SKI>
 static AttnKernel attn_kernel_of(int32_t dtype, int32_t D, int waves, bool store) {
     if (dtype == CAST_FP32) {
-        if (D == 128) return waves == 4 ? f32_instance<128, 4, 1, SKI>(store) : f32_instance<128, 8, 2, SKI>(store);
+        if (D == 128) return waves == 4 ? f32_instance<128, 4, 2, SKI>(store) : f32_instance<128, 8, 2, SKI>(store);
         return waves == 4 ? f32_instance<64, 4, 2, SKI>(store) : f32_instance<64, 8, 2, SKI>(store);
     }
     const bool f16 = dtype == CAST_FP16;
@@ -2190,7 +2233,7 @@ static AttnKernel attn_kernel(int32_t dtype, int32_t D, int waves, bool store, b
         case 192: return mfma_instance<192, 4, 1, false, true>(f16, store);
         case 256: return mfma_instance<256, 4, 1, false, true>(f16, store);
         case -64: return waves == 4 ? f32_instance<64, 4, 2, false, true>(store) : f32_instance<64, 8, 2, false, true>(store);
-        case -128: return waves == 4 ? f32_instance<128, 4, 1, false, true>(store) : f32_instance<128, 8, 2, false, true>(store);
+        case -128: return waves == 4 ? f32_instance<128, 4, 2, false, true>(store) : f32_instance<128, 8, 2, false, true>(store);
         case -256: return f32_instance<256, 4, 1, false, true>(store);
         default: break;
     }
@@ -2281,8 +2324,7 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
     p.chunk = resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, kv_split);
     const bool automatic =
         kv_split == 0 || kv_split == resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, 0);
-    const bool padded = padded_dim(dtype, D) != 0;
-    if (automatic && batch > 0 && batch <= 64 && ((mfma_path(dtype, D) && dtype != CAST_FP32) || padded)) {
+    if (automatic && batch > 0 && batch <= 64 && (mfma_path(dtype, D) || padded_dim(dtype, D))) {
         const int64_t G = Hq / Hkv;
         const int waves = waves_for(batch, total_q, (int32_t)G, dtype, D);
         const int64_t rows_wg = waves * 32;

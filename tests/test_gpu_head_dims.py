@@ -123,3 +123,53 @@ def test_padded_rows_with_infinities(gpu, dtype, what):
         assert not fin.all()
         assert ((got.float() - ref.float()).abs()[fin] <= EPS[dtype] * ref.float().abs()[fin] + 2e-5).all()
         assert torch.equal(got[10:], clean[10:]) or what == "k-minus-inf"
+
+
+@pytest.mark.parametrize("what", ["v-inf", "k-minus-inf", "k-nan", "q-inf", "huge", "scaled"])
+@pytest.mark.parametrize("D,packs", [(128, [10, 40]), (128, [120, 90]), (64, [10, 40]), (256, [10, 40])])
+def test_fp32_terms_keep_floats(gpu, D, packs, what):
+    # fp32 operands enter the products as three bf16 terms: infinities, NaN
+    # and floats next to the largest (whose leading term rounds to infinity)
+    # give what float products give, and powers of two pass through exactly
+    wl, q, k, v, meta, mask, words = _case(gpu, D, "fp32", 2, [200, 90], packs)
+    print(f"case fp32-terms D={D} packs={packs} {what}", flush=True)
+    args = (meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask)
+    clean = varlen_tree_attention(q, k, v, *args, kv_split=-1)
+    q, k, v = q.clone(), k.clone(), v.clone()
+    if what == "v-inf":
+        v[5, 0, 17] = math.inf
+    elif what == "k-minus-inf":
+        k[70, 1, 3] = -math.inf
+    elif what == "k-nan":
+        k[12, 0, D - 1] = math.nan
+    elif what == "q-inf":
+        q[3, 2, 40] = math.inf
+    elif what == "huge":
+        v[7, 1, 5] = 3.4e38      # rounds to infinity in bf16
+    else:
+        v *= 2.0 ** -90
+    out, lse = varlen_tree_attention(q, k, v, *args, return_lse=True, kv_split=-1, check=True)
+    if what == "scaled":
+        assert torch.equal(out, clean * 2.0 ** -90)
+        return
+    assert torch.equal(out[packs[0]:], clean[packs[0]:])       # request 1 is untouched
+    want, want_l = _exact(wl, q, k, v, words)
+    hot = {"v-inf": (slice(None), slice(0, 4)), "k-minus-inf": (slice(None), slice(4, 8)),
+           "k-nan": (slice(None), slice(0, 4)), "q-inf": (slice(3, 4), slice(2, 3)),
+           "huge": (slice(None), slice(4, 8))}[what]
+    rows = torch.zeros(out.shape[:2], dtype=torch.bool)
+    rows[:packs[0]][hot] = True
+    got = out.cpu()
+    assert torch.equal(got[~rows], clean.cpu()[~rows])
+    if what == "v-inf":
+        assert torch.isposinf(got[:packs[0], :4, 17]).all()
+        keep = [d for d in range(D) if d != 17]
+        assert torch.isfinite(got[:packs[0], :4, keep]).all()
+    elif what in ("k-nan", "q-inf"):
+        assert torch.isnan(got[rows]).any(dim=-1).all()
+    elif what == "huge":
+        assert ((got.double() - want).abs()[rows] <= 2e-5 * want.abs()[rows].clamp(min=1.0)).all()
+    else:                        # a score of -inf (q > 0) is a key that is not there; one of +inf makes NaN
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        fin = rows[..., None] & torch.isfinite(want)
+        assert fin.any() and ((got.double() - want).abs()[fin] <= 2e-5).all()
