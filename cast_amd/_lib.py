@@ -54,6 +54,9 @@ SIGNATURES = {
     "cast_draft_topk_workspace_size": ([_I32, _I32, _I32, _I32, _I32], _SZ),
     "cast_build_trees_uniform": ([_P, _P, _I32, _I32, _I32, _I32, _I32] + [_P] * 7, ctypes.c_int),
     "cast_build_trees": ([_P, _P, _I32, _I32, _I32, _I32] + [_P] * 8, ctypes.c_int),
+    "cast_greedy_accept_split": ([_P, _I64, _I32, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _P, _SZ, _P],
+                                 ctypes.c_int),
+    "cast_greedy_accept_workspace_size": ([_I32, _I32, _I32], _SZ),
     "cast_greedy_accept": ([_P, _I64, _I32, _I32, _P, _P, _P, _I32, _I32, _P, _P, _P, _P, _P, _P], ctypes.c_int),
 }
 

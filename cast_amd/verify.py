@@ -88,16 +88,19 @@ def greedy_accept(logits, cu_q, parent, token, *, check=False):
     if parent.shape[0] != total_q or token.shape[0] != total_q:
         raise ValueError("parent and token need one entry per logits row")
     B = int(cu_q.shape[0]) - 1
-    path = torch.empty((B, MAX_PACK), dtype=torch.int32, device=dev)
-    path_len = torch.empty(B, dtype=torch.int32, device=dev)
-    bonus = torch.empty(B, dtype=torch.int64, device=dev)
-    argmax = torch.empty(total_q, dtype=torch.int32, device=dev)
+    path = cu_q.new_empty((B, MAX_PACK))
+    path_len = cu_q.new_empty(B)
+    bonus = token.new_empty(B)
+    argmax = cu_q.new_empty(total_q)
     status = torch.zeros(1, dtype=torch.int32, device=dev) if check else None
     dt = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16}.get(logits.dtype, _lib.FP32)
+    ws_bytes = lib.cast_greedy_accept_workspace_size(total_q, V, dt)
+    ws = logits.new_empty(ws_bytes, dtype=torch.uint8) if ws_bytes else None
     with _lib.on_device(dev):
-        st = lib.cast_greedy_accept(_lib.ptr(logits), logits.stride(0), V, dt, _lib.ptr(cu_q), _lib.ptr(parent),
-                                    _lib.ptr(token), B, total_q, _lib.ptr(argmax), _lib.ptr(path),
-                                    _lib.ptr(path_len), _lib.ptr(bonus), _lib.ptr(status), _lib.stream_of(logits))
+        st = lib.cast_greedy_accept_split(_lib.ptr(logits), logits.stride(0), V, dt, _lib.ptr(cu_q), _lib.ptr(parent),
+                                          _lib.ptr(token), B, total_q, _lib.ptr(argmax), _lib.ptr(path),
+                                          _lib.ptr(path_len), _lib.ptr(bonus), _lib.ptr(status), _lib.ptr(ws),
+                                          ws_bytes, _lib.stream_of(logits))
     _lib.check(st, "cast_greedy_accept")
     if check:
         _lib.raise_device_flags(status.item(), "greedy_accept")

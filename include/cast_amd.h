@@ -255,6 +255,16 @@ int cast_greedy_accept(const void *logits, int64_t logits_ld, int32_t vocab, int
                        int32_t batch, int32_t total_q, int32_t *argmax, int32_t *path,
                        int32_t *path_len, int64_t *bonus, int32_t *status,
                        cast_stream_t stream);
+/* The same with a workspace (8-byte aligned) of at least
+ * cast_greedy_accept_workspace_size(...) bytes: few rows are then cut into
+ * segments that several workgroups scan.  Same results; a smaller or NULL
+ * workspace runs as cast_greedy_accept does. */
+int cast_greedy_accept_split(const void *logits, int64_t logits_ld, int32_t vocab, int32_t dtype,
+                             const int32_t *cu_q, const int32_t *parent, const int64_t *token,
+                             int32_t batch, int32_t total_q, int32_t *argmax, int32_t *path,
+                             int32_t *path_len, int64_t *bonus, int32_t *status,
+                             void *workspace, size_t workspace_bytes, cast_stream_t stream);
+size_t cast_greedy_accept_workspace_size(int32_t total_q, int32_t vocab, int32_t dtype);
 
 /* ---------------------------------------------------------------------
  * K4: accepted-path KV append into the per-request store, every layer in
