@@ -46,8 +46,10 @@ __device__ int argmax_exact(const char *__restrict__ base, int32_t vocab) {
     const int tid = threadIdx.x;
     float best = -INFINITY;
     int bi = INT_MAX;
-    const bool vec = ((reinterpret_cast<uintptr_t>(base) & 15) == 0);
-    const int nch = vec ? vocab / EPC : 0;
+    // the elements up to a 16-byte boundary come one by one, before the chunks
+    const int head = min(vocab, (int)(-reinterpret_cast<uintptr_t>(base) & 15) / (16 / EPC));
+    base += head * (16 / EPC);
+    const int nch = (vocab - head) / EPC;
     // A thread visits its elements in increasing index order, so an element
     // replaces the running best iff it is the first, strictly greater, or the
     // first NaN: ties keep the earlier index and a NaN best is never replaced.
@@ -70,18 +72,32 @@ __device__ int argmax_exact(const char *__restrict__ base, int32_t vocab) {
                 v = __builtin_bit_cast(float, bits);
             if (first && e == 0) {   // the thread's first element seeds the running best
                 best = v;
-                bi = c * EPC;
+                bi = head + c * EPC;
             } else {
-                take(v, c * EPC + e);
+                take(v, head + c * EPC + e);
             }
         }
     };
     // UNR independent 16-byte loads in flight per thread, then the compares
     // (in increasing index order per thread, as the tie rule needs)
     constexpr int UNR = 8;
+    auto element = [&](int i) {   // i < 0: in the head
+        float v;
+        if constexpr (BF16)
+            v = F::widen(reinterpret_cast<const uint16_t *>(base)[i]);
+        else
+            v = reinterpret_cast<const float *>(base)[i];
+        if (bi == INT_MAX) {     // the thread's first element
+            best = v;
+            bi = head + i;
+        } else {
+            take(v, head + i);
+        }
+    };
+    if (tid < head) element(tid - head);
     int c = tid;
     if (c < nch) {
-        scan_chunk(*reinterpret_cast<const u32x4 *>(base + (size_t)c * 16), c, true);
+        scan_chunk(*reinterpret_cast<const u32x4 *>(base + (size_t)c * 16), c, bi == INT_MAX);
         c += NT;
     }
     for (; c + (UNR - 1) * NT < nch; c += UNR * NT) {
@@ -92,19 +108,7 @@ __device__ int argmax_exact(const char *__restrict__ base, int32_t vocab) {
         for (int u = 0; u < UNR; ++u) scan_chunk(w[u], c + u * NT, false);
     }
     for (; c < nch; c += NT) scan_chunk(*reinterpret_cast<const u32x4 *>(base + (size_t)c * 16), c, false);
-    for (int i = nch * EPC + tid; i < vocab; i += NT) {
-        float v;
-        if constexpr (BF16)
-            v = F::widen(reinterpret_cast<const uint16_t *>(base)[i]);
-        else
-            v = reinterpret_cast<const float *>(base)[i];
-        if (bi == INT_MAX) {     // no vector chunk seeded this thread
-            best = v;
-            bi = i;
-        } else {
-            take(v, i);
-        }
-    }
+    for (int i = nch * EPC + tid; i < vocab - head; i += NT) element(i);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const float ov = __shfl_xor(best, off);
@@ -216,8 +220,12 @@ __global__ __launch_bounds__(256) void row_argmax_bf16_kernel(const void *__rest
     const int vocab = seg.n;
     const int tid = threadIdx.x;
     const char *base = static_cast<const char *>(logits) + ((size_t)blockIdx.x * (size_t)ld + (size_t)seg.first) * 2;
-    const bool vec = ((reinterpret_cast<uintptr_t>(base) & 15) == 0);
-    const int nch = vec ? vocab / EPC : 0;
+    // the elements up to a 16-byte boundary come one by one (rows of an odd
+    // length, as 50257, went one by one whole)
+    const char *const row_base = base;
+    const int head = min(vocab, (int)(-reinterpret_cast<uintptr_t>(base) & 15) / 2);
+    base += head * 2;
+    const int nch = (vocab - head) / EPC;
     int bk = INT_MIN, bc = -1;          // best chunk key, first chunk holding it
     u16x2 magmax = {0, 0};
     auto chunk_key = [&](const u32x4 &w) {
@@ -256,13 +264,22 @@ __global__ __launch_bounds__(256) void row_argmax_bf16_kernel(const void *__rest
 #pragma unroll
         for (int e = EPC - 1; e >= 0; --e) {
             const uint32_t bits = w[e >> 1];
-            if (bf16_key((uint16_t)(bits >> ((e & 1) * 16))) == bk) bi = bc * EPC + e;
+            if (bf16_key((uint16_t)(bits >> ((e & 1) * 16))) == bk) bi = head + bc * EPC + e;
         }
     }
-    // elements past the last whole chunk (or all of an unaligned row): their
-    // indices follow every chunk's, so they win only on a larger key
-    for (int i = nch * EPC + tid; i < vocab; i += NT) {
-        const uint16_t bits = reinterpret_cast<const uint16_t *>(base)[i];
+    if (tid < head) {   // smaller indices than any chunk's: a tie wins
+        const uint16_t bits = reinterpret_cast<const uint16_t *>(row_base)[tid];
+        magmax[0] = max(magmax[0], (unsigned short)(bits & 0x7fff));
+        const int k = bf16_key(bits);
+        if (k >= bk) {
+            bk = k;
+            bi = tid;
+        }
+    }
+    // elements past the last whole chunk: their indices follow every chunk's,
+    // so they win only on a larger key
+    for (int i = head + nch * EPC + tid; i < vocab; i += NT) {
+        const uint16_t bits = reinterpret_cast<const uint16_t *>(row_base)[i];
         const int m = bits & 0x7fff;
         magmax[0] = max(magmax[0], (unsigned short)m);
         const int k = bf16_key(bits);
@@ -273,8 +290,8 @@ __global__ __launch_bounds__(256) void row_argmax_bf16_kernel(const void *__rest
     }
     const bool nan = max(magmax[0], magmax[1]) > kInfMag;
     if (__syncthreads_or(nan)) {
-        const int exact = argmax_exact<F>(base, vocab);
-        if (tid == 0) write_best<F>(base, seg, exact, argmax, part);
+        const int exact = argmax_exact<F>(row_base, vocab);
+        if (tid == 0) write_best<F>(row_base, seg, exact, argmax, part);
         return;
     }
     // (key desc, index asc) over the workgroup
@@ -300,7 +317,7 @@ __global__ __launch_bounds__(256) void row_argmax_bf16_kernel(const void *__rest
                 bk = sk[w];
                 bi = si[w];
             }
-        write_best<F>(base, seg, bi, argmax, part);
+        write_best<F>(row_base, seg, bi, argmax, part);
     }
 }
 

@@ -14,6 +14,8 @@
 // the reference's Python floats are.
 #include <float.h>
 
+#include <type_traits>
+
 #include "cast_common.hpp"
 
 namespace cast {
@@ -143,7 +145,9 @@ __global__ __launch_bounds__(64) void draft_topk_combine_kernel(const TopkPart *
 //
 // Each thread keeps its best K rank keys (K >= k) in a fully unrolled sorted
 // list.  Only elements whose key is at least a threshold key enter the lists.
-// The threshold comes from the first batch (8 chunks per thread): the k-th
+// The threshold comes from the first batch (8 chunks per thread, or what a
+// shorter slice has: without one every element of a 32000-entry row went
+// through the lists: 120 rows of fp16, k = 8, 56.7 us against 10.3): the k-th
 // largest of the NW * R best thread keys, R per wave (2 for k <= 8, 4 for
 // k > 8), a bound no final top-k element of the slice falls below since at
 // least k distinct elements are at or above it.  At k = 8 two per wave were
@@ -154,11 +158,15 @@ __global__ __launch_bounds__(64) void draft_topk_combine_kernel(const TopkPart *
 // into LDS and ranked by counting (k rounds over the list heads when more
 // than kTopkNT entries survive).
 //
+// Register limits: 168 for the 16-bit rows (one workgroup a CU either way; a
+// larger budget made the fp16 instance 5 % slower), 128 for fp32 (two
+// workgroups a CU: 400 rows of 151936 54 us against 63 at 210 registers).
+//
 // Log-sum-exp: a running max per thread; a chunk's exp terms are summed
 // pairwise in float onto the thread's float sum, which is rescaled only when
 // the running max moves.  Workgroup and split sums are combined in double.
 template <bool BF16, int K, typename E = Bf16>
-__global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restrict__ logits, int64_t ld,
+__global__ __launch_bounds__(kTopkNT) __attribute__((amdgpu_waves_per_eu(BF16 ? 3 : 4))) void draft_topk_kernel(const void *__restrict__ logits, int64_t ld,
                                                              int32_t vocab, int32_t k, int32_t per_e,
                                                              TopkPart *__restrict__ part,
                                                              int64_t *__restrict__ top_idx,
@@ -168,11 +176,16 @@ __global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restr
     constexpr int EPC = BF16 ? 8 : 4;
     const int row = blockIdx.x, split = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const char *base = static_cast<const char *>(logits) + (size_t)row * (size_t)ld * (BF16 ? 2 : 4);
+    // the row's first `head` elements, up to a 16-byte boundary, come one by
+    // one; element positions below count from there (rows of an odd length,
+    // as 50257, went one by one whole: 120 rows of bf16, k = 8, 60.9 us
+    // against 11.7)
+    const int head = min(vocab, (int)(-reinterpret_cast<uintptr_t>(base) & 15) / (BF16 ? 2 : 4));
+    base += head * (BF16 ? 2 : 4);
     const int e0 = split * per_e;
-    const int e1 = max(e0, min(vocab, e0 + per_e));   // an empty last split stays empty
-    const bool vec = (reinterpret_cast<uintptr_t>(base) & 15) == 0;
-    const int cb = vec ? e0 / EPC : 0, ce = vec ? e1 / EPC : 0;   // this split's whole chunks
-    const int tail0 = vec ? ce * EPC : e0;                         // then elements [tail0, e1)
+    const int e1 = max(e0, min(vocab - head, e0 + per_e));   // an empty last split stays empty
+    const int cb = e0 / EPC, ce = e1 / EPC;                   // this split's whole chunks
+    const int tail0 = ce * EPC;                               // then elements [tail0, e1)
 
     uint64_t tk[K];   // descending; 0 = empty
 #pragma unroll
@@ -249,7 +262,7 @@ __global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restr
                 float ve = v[0];
 #pragma unroll
                 for (int e2 = 1; e2 < EPC; ++e2) ve = e == e2 ? v[e2] : ve;
-                const uint64_t key = rank_key(ve, c * EPC + e);
+                const uint64_t key = rank_key(ve, head + c * EPC + e);
                 if (key >= thr) insert(key);
             }
         }
@@ -271,13 +284,23 @@ __global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restr
     __shared__ uint64_t thr_pick;
     int c = cb + tid;
     u32x4 nxt[NB];
-    if (ce - cb >= NB * NT) {   // first batch: the threshold, then the batch through it
+    // first batch (of a short slice the only one, partly filled): the
+    // threshold, then the batch through it
+    auto first_batch = [&](auto whole) __attribute__((always_inline)) {
+        constexpr bool full = decltype(whole)::value;
         u32x4 w[NB];
-        load_batch(w, c);
-        if (c + NB * NT + (NB - 1) * NT < ce) load_batch(nxt, c + NB * NT);
+        if constexpr (full) {
+            load_batch(w, c);
+            if (c + NB * NT + (NB - 1) * NT < ce) load_batch(nxt, c + NB * NT);
+        } else {
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+                if (c + u * NT < ce) w[u] = *reinterpret_cast<const u32x4 *>(base + (size_t)(c + u * NT) * 16);
+        }
         uint64_t best = 0;
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
+            if (!full && c + u * NT >= ce) break;
             float v[EPC];
             unpack(w[u], v);
             const float m = chunk_max(v);
@@ -285,7 +308,7 @@ __global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restr
             int fi = EPC - 1;   // the chunk's first element equal to its max
 #pragma unroll
             for (int e = EPC - 2; e >= 0; --e) fi = v[e] == m ? e : fi;
-            const uint64_t key = rank_key(m, (c + u * NT) * EPC + fi);
+            const uint64_t key = rank_key(m, head + (c + u * NT) * EPC + fi);
             best = key > best ? key : best;
         }
 #pragma unroll
@@ -313,14 +336,17 @@ __global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restr
         }
 #pragma unroll
         for (int u = 0; u < NB; ++u) {
+            if (!full && c + u * NT >= ce) break;
             float v[EPC];
             unpack(w[u], v);
             filter(v, chunk_max(v), c + u * NT);
         }
         c += NB * NT;
-    } else if (c + (NB - 1) * NT < ce) {
-        load_batch(nxt, c);
-    }
+    };
+    if (ce - cb >= NB * NT)
+        first_batch(std::true_type{});
+    else if (ce - cb >= NT)
+        first_batch(std::false_type{});
     // the rest in batches, the next batch loading while this one is consumed
     for (; c + (NB - 1) * NT < ce; c += NB * NT) {
         u32x4 w[NB];
@@ -339,12 +365,14 @@ __global__ __launch_bounds__(kTopkNT) void draft_topk_kernel(const void *__restr
         for (int u = 0; u < NB - 1; ++u)
             if (c + u * NT < ce) chunk(w[u], c + u * NT);
     }
-    for (int i = tail0 + tid; i < e1; i += NT) {
+    auto single = [&](int i) {   // i < 0: in the head
         const float v[1] = {logit_at<BF16, E>(base, i)};
         lse_add(v, v[0]);
-        const uint64_t key = rank_key(v[0], i);
+        const uint64_t key = rank_key(v[0], head + i);
         if (key >= thr) insert(key);
-    }
+    };
+    for (int i = tail0 + tid; i < e1; i += NT) single(i);
+    if (split == 0 && tid < head) single(tid - head);
 
     // ---- the slice's log-sum-exp: max, then the sums rescaled to it
     __shared__ float red[NW];
