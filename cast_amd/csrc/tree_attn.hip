@@ -100,6 +100,7 @@ struct AttnArgs {
     int32_t slots;      // > 0: the kernels choose the split from the batch's lengths (auto_split) for this
                         // many workgroups, the number the device holds at once
     float hkv_per_slot; // Hkv / slots
+    int32_t *split_tiles;   // slots > 0: the attention kernel's choice (tiles per split), for the combine
     int32_t max_rows;   // longest key source (rows) the MFMA kernel can address
     int32_t xcds;       // XCDs of the device: workgroup x runs on XCD x % xcds
     int32_t sk_mode;    // stream-K schedule asked for (CAST_SPLIT_STREAM)
@@ -269,8 +270,9 @@ __device__ __forceinline__ bool batch_fits(const AttnArgs &a, const BatchTotals 
 
 // The split of a batch of up to 64 requests, chosen from its lengths: lane j
 // holds request j (t; ok when it passed load_seq) and gets its ns and
-// split_len.  Every workgroup of the attention and combine kernels calls it
-// (at least 4 waves; fit: LDS) and finds the same split.
+// split_len.  Every workgroup of the attention kernel calls it (at least 4
+// waves; fit: LDS) and finds the same split; the first leaves it for the
+// combine kernel, which then need not look for it again (0.5 us a call).
 //
 // With W = sum over the requests of row blocks x 64-key tiles, L = W * Hkv /
 // slots tiles is what each of the workgroups resident at once would get of an
@@ -308,6 +310,7 @@ __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok, int *fit) {
     }
     __syncthreads();
     const int c = cand(fit[0] ? 0 : fit[1] ? 1 : fit[2] ? 2 : fit[3] ? 3 : 2);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.split_tiles = c;
     t.ns = tiles ? udiv(tiles + c - 1, c) : 0;
     t.split_len = tiles ? udiv(tiles + t.ns - 1, t.ns) * 64 : 0;
 }
@@ -1731,7 +1734,6 @@ void tree_attn_f32_kernel(AttnArgs a) {
 // per head max and sum; the stream-K instance adds each piece's partial row
 // and each head's piece count.
 struct CombineLds {
-    int fit[4];   // auto_split
     float wgt[kCombineLdsHeads * kCombineLdsSplits];
     float hm[kCombineLdsHeads], hl[kCombineLdsHeads];
 };
@@ -1840,13 +1842,17 @@ __global__ __launch_bounds__(256) void tree_attn_combine_kernel(AttnArgs a) {
     if (a.batch <= 64) {
         // one round of metadata loads: the totals and the request of tok
         const int lane = threadIdx.x & 63;
+        const int chosen = !SKI && a.slots ? *a.split_tiles : 0;   // (loaded beside the metadata)
         Seq t{};
         bool unordered = false;
         const bool ok = lane < a.batch && load_seq(a, lane, t, false, unordered);
         BatchTotals tot{0, 0, 0, false, false};
         add_totals(tot, a, lane, ok, t, unordered);
         if (rejected(tot)) return;
-        if (!SKI && a.slots) auto_split(a, t, ok, sm.fit);
+        if (!SKI && a.slots) {
+            const int tiles = ok && t.P > 0 ? (int)(((uint32_t)t.T + 63) >> 6) : 0;
+            t.ns = tiles ? udiv(tiles + chosen - 1, chosen) : 0;
+        }
         const int pp = ok && t.ns > 1 ? sat32((int64_t)t.ns * t.P) : 0;
         const int p_excl = wave_scan(pp) - pp;
         int base = 0, cost = 0, tiles = 0;
@@ -2312,9 +2318,12 @@ struct SplitPlan {
 // that cannot give more items than the device holds (single-p16).
 //
 // Bounds of auto_split's result, with c >= L = W * Hkv / slots tiles per split
-// and RB = total_q * G / rows_wg + batch >= sum rb: items = Hkv * sum rb *
-// ceil(tiles / c) <= slots + Hkv * RB; an XCD takes at most ceil(groups / nx)
-// groups of each request, so its slots are at most items / nx + RB; a request
+// and RB = min(total_q * G / rows_wg + batch, batch * rbmax) >= sum rb: the
+// items fit the slots, or c >= 10/8 L and they are Hkv * sum rb * ceil(tiles / c)
+// <= 8/10 slots + Hkv * RB; an XCD takes at most ceil(groups / nx) groups of
+// each request, so its slots are at most items / nx, plus RB where Hkv is no
+// multiple of nx (workgroups past the last item cost their prologue at the end
+// of the call: 2 us at the headline with a bound of 640 for 256); a request
 // in ns > 1 splits has ns - 1 < tiles / c and P <= rb * rows_wg / G, so the
 // partial rows sum to less than rows_wg * slots / Hq plus the rows of the
 // split requests, which are at most that many again.
@@ -2343,11 +2352,14 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
         p.part_rows = part_rows_bound(total_q, total_kv, p.chunk);
         if ((int64_t)Hkv * rbmax * ((int64_t)total_kv / kMinChunk + batch) > slots) {
             p.slots = (int32_t)slots;
-            const int64_t rb_sum = total_q * G / rows_wg + batch;
+            const int64_t by_rows = total_q * G / rows_wg + batch, by_pack = batch * rbmax;
+            const int64_t rb_sum = by_rows < by_pack ? by_rows : by_pack;
             const int64_t once = (rows_wg * slots + Hq - 1) / Hq;
             const int64_t rows = once + (once < total_q ? once : total_q);
             if (rows < p.part_rows) p.part_rows = rows;
-            p.wg_bound = topo.xcds * ((slots + Hkv * rb_sum + topo.xcds - 1) / topo.xcds + rb_sum);
+            const int64_t second = (slots * 8 + 9) / 10 + Hkv * rb_sum;
+            const int64_t most = second > slots ? second : slots;
+            p.wg_bound = topo.xcds * ((most + topo.xcds - 1) / topo.xcds + (Hkv % topo.xcds ? rb_sum : 0));
         }
         return p;
     }
@@ -2355,10 +2367,12 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
     return p;
 }
 
-// Bytes of the split-K partials: O [part_rows][Hq][D], then lse [part_rows][Hq].
+// Bytes of the split-K partials: O [part_rows][Hq][D], then lse [part_rows][Hq],
+// then the chosen split where the device chooses.
 static size_t split_bytes(const SplitPlan &p, int32_t Hq, int32_t D) {
     if (p.chunk == kNoSplit) return 0;
-    return align256((size_t)p.part_rows * Hq * D * sizeof(float)) + align256((size_t)p.part_rows * Hq * sizeof(float));
+    return align256((size_t)p.part_rows * Hq * D * sizeof(float)) +
+           align256((size_t)p.part_rows * Hq * sizeof(float)) + (p.slots ? align256(sizeof(int32_t)) : 0);
 }
 
 }  // namespace cast
@@ -2510,6 +2524,8 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     a.by_chunk = fast_div((uint32_t)a.chunk);
     a.slots = sp.slots;
     a.hkv_per_slot = sp.slots ? (float)num_kv_heads / (float)sp.slots : 0.f;
+    if (sp.slots)
+        a.split_tiles = reinterpret_cast<int32_t *>(static_cast<char *>(workspace) + split_need - align256(sizeof(int32_t)));
     if (a.chunk != kNoSplit || sk.mode) {
         const size_t skb = sk_bytes(sk, head_dim);
         const size_t need = skb > split_need ? skb : split_need;
