@@ -37,7 +37,7 @@ sys.path.insert(0, str(ROOT))
 METRIC = "tree-verify attn µs/call + % HBM roofline, Qwen3-8B shape, N=128, ctx 8k, B=8"
 PEAK_HBM = 8.0e12          # B/s, MI355X HBM3E
 PEAK_MFMA_BF16 = 2.5e15    # FLOP/s, dense bf16
-PEAK_MFMA_FP32 = 157.3e12  # FLOP/s, dense fp32
+PEAK_MFMA_FP32 = PEAK_MFMA_BF16 / 6   # fp32 as six products of bf16 terms (the fp32 instruction: 157.3e12)
 TRAFFIC_FILE = ROOT / "profiles" / "traffic.json"
 BENCH_LIB = ROOT / "cast_amd" / "libcast_bench.so"
 _bench_lib = None
