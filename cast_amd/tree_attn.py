@@ -73,7 +73,8 @@ def _mask_words(mask, total_q, device):
 def _workspace_bytes(device_index, *sizes):
     """cast_tree_attn_workspace_size of one call's sizes (a function of them
     and the device alone: asked once per size, not once per layer)."""
-    return _lib.load().cast_tree_attn_workspace_size(*sizes)
+    with _lib.on_device(torch.device("cuda", device_index)):
+        return _lib.load().cast_tree_attn_workspace_size(*sizes)
 
 
 def _host_side(*metadata):
