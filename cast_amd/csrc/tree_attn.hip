@@ -270,9 +270,11 @@ __device__ __forceinline__ bool batch_fits(const AttnArgs &a, const BatchTotals 
 
 // The split of a batch of up to 64 requests, chosen from its lengths: lane j
 // holds request j (t; ok when it passed load_seq) and gets its ns and
-// split_len.  Every workgroup of the attention kernel calls it (at least 4
-// waves; fit: LDS) and finds the same split; the first leaves it for the
-// combine kernel, which then need not look for it again (0.5 us a call).
+// split_len.  Every workgroup of the attention kernel calls it once (at least
+// 4 waves) and finds the same split; the first leaves it for the combine
+// kernel, which then need not look for it again (0.5 us a call).  The waves'
+// answers lie in LDS words that nothing else writes: its one barrier orders
+// their writes before the reads, and no barrier follows the reads.
 //
 // With W = sum over the requests of row blocks x 64-key tiles, L = W * Hkv /
 // slots tiles is what each of the workgroups resident at once would get of an
@@ -291,7 +293,8 @@ __device__ __forceinline__ bool batch_fits(const AttnArgs &a, const BatchTotals 
 // 1k to 8k keys, D = 128, 83.6 -> 70.9 us; 32 requests of 300 to 4k keys with
 // packs of 2 to 64 148.9 -> 95.2 us (with 4-wave workgroups, see waves_for);
 // 8 requests of 4k to 8k keys at D = 256 282.6 -> 224.7 us.
-__device__ void auto_split(const AttnArgs &a, Seq &t, bool ok, int *fit) {
+__device__ void auto_split(const AttnArgs &a, Seq &t, bool ok) {
+    __shared__ __attribute__((aligned(16))) int fit[4];
     const int tiles = ok && t.P > 0 ? (int)(((uint32_t)t.T + 63) >> 6) : 0;
     const int rb = tiles ? t.rb : 0;
     const int W = wave_sum(tiles * rb);   // the host keeps it below 2^31
@@ -309,7 +312,8 @@ __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok, int *fit) {
         if ((threadIdx.x & 63) == 0) fit[w] = (int64_t)n * a.Hkv <= a.slots;
     }
     __syncthreads();
-    const int c = cand(fit[0] ? 0 : fit[1] ? 1 : fit[2] ? 2 : fit[3] ? 3 : 2);
+    const int4 f = *reinterpret_cast<const int4 *>(fit);   // one read
+    const int c = cand(f.x ? 0 : f.y ? 1 : f.z ? 2 : f.w ? 3 : 2);
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.split_tiles = c;
     t.ns = tiles ? udiv(tiles + c - 1, c) : 0;
     t.split_len = tiles ? udiv(tiles + t.ns - 1, t.ns) * 64 : 0;
@@ -757,9 +761,9 @@ __device__ bool sk_next_segment(const AttnArgs &a, WorkCursor &cur, Unit &u, con
 // and sk_plan accepts the batch, else the longest-first schedule; larger
 // ones take items in batch order, consecutive items (the row blocks of one
 // key split) on one XCD so that they share its L2.  skr: LDS for the stream-K
-// table (64 entries); fit: LDS of auto_split (4 ints).
+// table (64 entries).
 template <bool SK>   // SK: the kernel instance takes the stream-K schedule when the plan asks
-__device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *skr, int *fit) {
+__device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *skr) {
     cur.sk = false;
     Seq &sq = u.sq;
     int h = 0, split = 0, rb = 0;
@@ -790,7 +794,7 @@ __device__ bool first_unit(const AttnArgs &a, WorkCursor &cur, Unit &u, SkReq *s
             cur.end = min(cur.p + pl.L, (int64_t)pl.C);
             return sk_next_segment(a, cur, u, skr);
         }
-        if (!SK && a.slots) auto_split(a, t, ok, fit);
+        if (!SK && a.slots) auto_split(a, t, ok);
         if (!locate_sorted(a, blockIdx.x, t, ok, sq, h, split, rb)) return false;
     } else {
         const BatchTotals tot = batch_totals(a);
@@ -869,7 +873,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t Ks[NBUF][BN * KPAD];
     __shared__ __attribute__((aligned(16))) uint16_t Vt[NBUF][D * VPAD];
     __shared__ EpiArgs epi;
-    __shared__ int pack_hi[WAVES];   // auto_split's LDS, then per wave the last pack key a row of it sees
+    __shared__ int pack_hi[WAVES];   // per wave: the last pack key a row of it sees
     // Head dim 256 (one wave per SIMD, no registers to spare) has no
     // stream-K instance.
     constexpr bool kStreamK = SKI && D <= 128;
@@ -878,7 +882,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     // ---- this workgroup's work: one unit, or a run of stream-K segments
     Unit wu;
     WorkCursor cur;
-    if (!first_unit<kStreamK>(a, cur, wu, skr, pack_hi)) return;
+    if (!first_unit<kStreamK>(a, cur, wu, skr)) return;
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
@@ -1378,12 +1382,12 @@ void tree_attn_f32_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) uint16_t Ks[NBUF][3][BN * KPAD];
     __shared__ __attribute__((aligned(16))) uint16_t Vt[NBUF][3][D * VPAD];
     __shared__ EpiArgs epi;
-    __shared__ int pack_hi[WAVES];   // auto_split's LDS, then per wave the last pack key a row of it sees
+    __shared__ int pack_hi[WAVES];   // per wave: the last pack key a row of it sees
     __shared__ SkReq skr[SKI ? 64 : 1];
 
     Unit wu;
     WorkCursor cur;
-    if (!first_unit<SKI>(a, cur, wu, skr, pack_hi)) return;
+    if (!first_unit<SKI>(a, cur, wu, skr)) return;
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
     const int lane = tid & 63;
