@@ -2314,8 +2314,8 @@ struct SplitPlan {
     int64_t wg_bound;    // workgroups the split can need (0: the general bound)
 };
 
-// kv_split = 0 (or the chunk that cast_tree_attn_default_split names for it)
-// and up to 64 requests: the device chooses.  Not worth the
+// kv_split = 0 and up to 64 requests: the device chooses (a chunk the caller
+// names is taken as it is).  Not worth the
 // combine launch where the rows alone fill the device one and a half times
 // (the longest-first order balances those), or where the averages ask for no
 // split and prefixes are short; and with one chunk of kMinChunk keys when even
@@ -2335,9 +2335,7 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
                             int32_t dtype, int32_t kv_split) {
     SplitPlan p{};
     p.chunk = resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, kv_split);
-    const bool automatic =
-        kv_split == 0 || kv_split == resolve_chunk(batch, total_q, total_kv, Hq, Hkv, D, dtype, 0);
-    if (automatic && batch > 0 && batch <= 64 && (mfma_path(dtype, D) || padded_dim(dtype, D))) {
+    if (kv_split == 0 && batch > 0 && batch <= 64 && (mfma_path(dtype, D) || padded_dim(dtype, D))) {
         const int64_t G = Hq / Hkv;
         const int waves = waves_for(batch, total_q, (int32_t)G, dtype, D);
         const int64_t rows_wg = waves * 32;

@@ -5,8 +5,9 @@ positional signature, argument meaning and result, with these additions
 (keyword-only, all optional):
 
   return_lse  also return the natural-log log-sum-exp [total_q, Hq] (fp32)
-  kv_split    keys per split-K chunk (0: library heuristic, SPLIT_STREAM:
-              the stream-K schedule, other values < 0: no split)
+  kv_split    keys per split-K chunk (0: the kernels choose it from the
+              requests' lengths, above 64 requests from the averages;
+              SPLIT_STREAM: the stream-K schedule, other values < 0: no split)
   check       synchronise once and raise ValueError if the kernels flagged
               inconsistent metadata (off by default: the call never syncs)
   out         preallocated output [total_q, Hq, D]
@@ -141,7 +142,10 @@ def _ready(x, esz):
 
 @dataclass
 class TreeAttnPlan:
-    """Host-side launch geometry of one call (for benchmarks and tests)."""
+    """Host-side launch geometry of one call (for benchmarks and tests).
+    kv_split: the chunk asked for, or for 0 the one from the batch's averages
+    (-1: none), which batches of up to 64 requests replace by the kernels'
+    own choice from the requests' lengths."""
     kv_split: int
     workspace_bytes: int
 

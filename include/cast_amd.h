@@ -99,12 +99,12 @@ int cast_tree_bitmask(const int32_t *parent, const int32_t *cu_q, int32_t batch,
  *   sm_scale  > 0 (the Python layer substitutes 1/sqrt(D) for None)
  *   kv_split  keys per split-K chunk (multiple of 64); 0 lets the library
  *             choose; CAST_SPLIT_STREAM (-2) asks for the stream-K schedule;
- *             any other negative value disables split-K.  With 0 (or the
- *             value of cast_tree_attn_default_split) long prefixes are cut
- *             into equal splits so that the work items cover the device once;
- *             for batches of up to 64 requests the kernels choose the chunk
- *             from the requests' lengths (static schedule, longest items
- *             first).
+ *             any other negative value disables split-K.  With 0 long
+ *             prefixes are cut into equal splits so that the work items cover
+ *             the device once: for batches of up to 64 requests the kernels
+ *             choose the chunk from the requests' lengths, larger batches
+ *             take that of cast_tree_attn_default_split (static schedule,
+ *             longest items first).
  *             Stream-K (only when asked for): pairs of workgroups on one XCD
  *             get equal ranges of key tiles over all (request, KV head, row
  *             block) units, and a combine merges the pieces of units cut
@@ -226,9 +226,11 @@ size_t cast_tree_attn_workspace_size(int32_t batch, int32_t total_q, int32_t tot
                                      int32_t num_q_heads, int32_t num_kv_heads,
                                      int32_t head_dim, int32_t dtype, int32_t kv_split);
 
-/* The split-K chunk (keys) that kv_split = 0 stands for, estimated from the
- * batch's averages (-1: no split); passing it back as kv_split is the same
- * as 0. */
+/* A split-K chunk (keys) from the batch's averages, -1 for no split: what
+ * kv_split = 0 takes for batches above 64 requests.  For smaller ones the
+ * kernels choose from the requests' lengths instead, and this is an estimate;
+ * where it is a chunk, a call with kv_split = 0 needs its workspace.  Passed
+ * as kv_split it asks for exactly this chunk (or for no split). */
 int32_t cast_tree_attn_default_split(int32_t batch, int32_t total_q, int32_t total_kv,
                                      int32_t num_q_heads, int32_t num_kv_heads,
                                      int32_t head_dim, int32_t dtype);

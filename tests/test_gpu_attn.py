@@ -371,26 +371,52 @@ def _call(wl, dev, kv_split, qkv=None):
     return out, lse
 
 
+def _call_and_chunk(wl, dev, qkv):
+    """kv_split = 0 with the chunk (keys) the kernels chose: the tiles of 64
+    keys that the first workgroup leaves at the end of the workspace."""
+    from cast_amd import varlen_tree_attention
+    from cast_amd.tree_attn import plan
+    n = plan(wl.B, wl.total_q, wl.total_kv, wl.Hq, wl.Hkv, wl.D, dtype=qkv[0].dtype).workspace_bytes
+    ws = torch.zeros(n, dtype=torch.uint8, device=dev)
+    meta = wl.meta_tensors(dev)
+    mask = torch.from_numpy(_words(wl).view(np.int64).copy()).to(dev)
+    out, lse = varlen_tree_attention(*qkv, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"],
+                                     mask, return_lse=True, check=True, workspace=ws)
+    return out, lse, 64 * int(ws[n - 256:n - 252].view(torch.int32)[0])
+
+
 def test_schedule_choice_ragged_and_uniform(gpu):
-    # The library's own choice (kv_split=0) keeps the static splits on the
-    # benchmark's ragged batch (bit for bit the forced chunk); the forced
-    # stream-K schedule cuts other pieces (other bits, within the bar).  The
-    # uniform headline batch keeps its static splits too.
+    # The library's own choice (kv_split=0) is a static split whose chunk the
+    # kernels take from the lengths: bit for bit the forced chunk of that
+    # size.  On the ragged batch it is another than the averages' estimate,
+    # and that estimate, forced, is taken as it is: each request comes out as
+    # it does alone at the same chunk.  The forced stream-K schedule cuts
+    # other pieces (other bits, within the bar).
     from cast_amd.tree_attn import plan
     wl = SC.qwen3_ragged(seed=0)
     print(f"case schedule-choice ragged: B={wl.B} total_q={wl.total_q} total_kv={wl.total_kv}", flush=True)
     qkv = wl.qkv(device=gpu)
-    chunk = plan(wl.B, wl.total_q, wl.total_kv, wl.Hq, wl.Hkv, wl.D).kv_split
-    auto, sk, static = (_call(wl, gpu, s, qkv) for s in (0, -2, chunk))
-    assert torch.equal(auto[0], static[0]) and torch.equal(auto[1], static[1])
-    assert not torch.equal(sk[0], static[0])
+    estimate = plan(wl.B, wl.total_q, wl.total_kv, wl.Hq, wl.Hkv, wl.D).kv_split
+    auto_o, auto_l, chunk = _call_and_chunk(wl, gpu, qkv)
+    assert chunk > 0 and chunk != estimate
+    sk, static, forced = (_call(wl, gpu, s, qkv) for s in (-2, chunk, estimate))
+    assert torch.equal(auto_o, static[0]) and torch.equal(auto_l, static[1])
+    assert not torch.equal(forced[0], static[0]) and not torch.equal(sk[0], static[0])
     assert (sk[0].float() - static[0].float()).abs().max() <= 2e-2
+    assert (forced[0].float() - static[0].float()).abs().max() <= 2e-2
+    from cast_amd import varlen_tree_attention
+    words = torch.from_numpy(_words(wl).view(np.int64).copy()).to(gpu)
+    for b in range(wl.B):
+        r, s = slice(int(wl.cu_q[b]), int(wl.cu_q[b + 1])), slice(int(wl.cu_kv[b]), int(wl.cu_kv[b + 1]))
+        alone = varlen_tree_attention(qkv[0][r], qkv[1][s], qkv[2][s], [0, r.stop - r.start], [0, s.stop - s.start],
+                                      [int(wl.prefix_len[b])], [int(wl.pack_len[b])], words[r], kv_split=estimate)
+        assert torch.equal(alone, forced[0][r]), f"request {b}"
     wl = SC.qwen3_headline()
     print("case schedule-choice headline", flush=True)
     qkv = wl.qkv(device=gpu, generator_device=gpu)
-    chunk = plan(wl.B, wl.total_q, wl.total_kv, wl.Hq, wl.Hkv, wl.D).kv_split
-    auto, static = (_call(wl, gpu, s, qkv) for s in (0, chunk))
-    assert torch.equal(auto[0], static[0]) and torch.equal(auto[1], static[1])
+    auto_o, auto_l, chunk = _call_and_chunk(wl, gpu, qkv)
+    static = _call(wl, gpu, chunk, qkv)
+    assert torch.equal(auto_o, static[0]) and torch.equal(auto_l, static[1])
 
 
 def test_stream_k_exact_scaling_property(gpu):
