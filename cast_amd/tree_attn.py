@@ -30,6 +30,7 @@ from __future__ import annotations
 
 import functools
 import math
+import operator
 from dataclasses import dataclass
 
 import numpy as np
@@ -73,7 +74,8 @@ def _mask_words(mask, total_q, device):
 @functools.lru_cache(maxsize=256)
 def _workspace_bytes(device_index, *sizes):
     """cast_tree_attn_workspace_size of one call's sizes (a function of them
-    and the device alone: asked once per size, not once per layer)."""
+    and the device alone: asked once per size, not once per layer).  The sizes
+    are plain ints: a tensor would be remembered by its identity."""
     with _lib.on_device(torch.device("cuda", device_index)):
         return _lib.load().cast_tree_attn_workspace_size(*sizes)
 
@@ -167,6 +169,7 @@ def varlen_tree_attention(q, k, v, cu_q, cu_kv, prefix_len, pack_len, ancestor_m
     [total_q, 2].  Returns ``out`` (and ``lse`` with ``return_lse``).
     """
     lib = _lib.load()
+    kv_split = operator.index(kv_split)
     total_q, H_q, D = q.shape
     total_kv, H_kv = k.shape[0], k.shape[1]
     assert H_q % H_kv == 0
@@ -211,7 +214,7 @@ def varlen_tree_attention(q, k, v, cu_q, cu_kv, prefix_len, pack_len, ancestor_m
     args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _lib.ptr(lse), cu_q.data_ptr(), cu_kv.data_ptr(),
             prefix_len.data_ptr(), pack_len.data_ptr(), mask.data_ptr(), words,
             B, total_q, total_kv, H_q, H_kv, D,
-            *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], dt, float(sm_scale), int(kv_split),
+            *q.stride()[:2], *k.stride()[:2], *v.stride()[:2], *out.stride()[:2], dt, float(sm_scale), kv_split,
             _lib.ptr(workspace) if ws_bytes else None, ws_bytes, _lib.ptr(status), _lib.stream_of(q))
     with _lib.on_device(dev):
         if _stage_hook is None:
@@ -248,6 +251,7 @@ def store_tree_attention(q, k_store, v_store, k_pack, v_pack, cu_q, prefix_len, 
     Returns ``out`` [total_q, H_q, D] (and ``lse`` with ``return_lse``).
     """
     lib = _lib.load()
+    kv_split = operator.index(kv_split)
     total_q, H_q, D = q.shape
     if k_store.dim() != 4 or k_pack.dim() != 3:
         raise ValueError("k_store must be [B, H_kv, cap, D] and k_pack [H_kv, total_q, D]")
@@ -297,7 +301,7 @@ def store_tree_attention(q, k_store, v_store, k_pack, v_pack, cu_q, prefix_len, 
             q.data_ptr(), k_store.data_ptr(), v_store.data_ptr(), k_pack.data_ptr(), v_pack.data_ptr(), out.data_ptr(),
             _lib.ptr(lse), cu_q.data_ptr(), prefix_len.data_ptr(), pack_len.data_ptr(), mask.data_ptr(), words,
             B, total_q, total_kv, cap, H_q, H_kv, D, *q.stride()[:2], *k_store.stride()[:3], *v_store.stride()[:3],
-            *k_pack.stride()[1::-1], *v_pack.stride()[1::-1], *out.stride()[:2], dt, float(sm_scale), int(kv_split),
+            *k_pack.stride()[1::-1], *v_pack.stride()[1::-1], *out.stride()[:2], dt, float(sm_scale), kv_split,
             _lib.ptr(workspace) if ws_bytes else None, ws_bytes, _lib.ptr(status), _lib.stream_of(q))
     _lib.check(st, "cast_tree_attn_store_fwd")
     if check:

@@ -74,3 +74,21 @@ def test_missing_workspace_runs_unsplit(gpu):
         outs.append((out, lse))
     for out, lse in outs[1:]:
         assert torch.equal(out, outs[0][0]) and torch.equal(lse, outs[0][1])
+
+
+def test_kv_split_from_a_tensor(gpu):
+    # the workspace size is remembered by value, also where the caller keeps
+    # kv_split in a tensor and changes it in place
+    from cast_amd import varlen_tree_attention
+    wl = _batch("split-tensor", [700, 300], [8, 5], 8, 4, 64)
+    print("case split-tensor", flush=True)
+    q, k, v = wl.qkv(device=gpu)
+    meta = wl.meta_tensors(gpu)
+    mask = torch.from_numpy(_words(wl).view(np.int64).copy()).to(gpu)
+    args = (q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask)
+    split = torch.tensor(-1)
+    assert torch.equal(varlen_tree_attention(*args, kv_split=split), varlen_tree_attention(*args, kv_split=-1))
+    split.fill_(64)
+    assert torch.equal(varlen_tree_attention(*args, kv_split=split), varlen_tree_attention(*args, kv_split=64))
+    with pytest.raises(TypeError):
+        varlen_tree_attention(*args, kv_split=0.5)
