@@ -537,46 +537,126 @@ __device__ __forceinline__ float load_elem(const T *p) {
         return *p;
 }
 
-// One query row against keys [k_begin, k_end) in plain fp32, by one wave: the
-// (unnormalised) output element lane + 64 j in acc[j], and the row's running
-// max (base 2) and sum.  For rows whose split products met an infinity or a
-// NaN: a term that is zero there makes a NaN of what a float product keeps.
+// Waits for every load so far, the first tile's and Q's.  The tile loop needs
+// the former at once; without the wait the compiler may place the one for Q
+// inside the loop, where it also waits for the next tile's loads (d96-shaped
+// calls 28.0 us against 25.9).
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }   // vmcnt(0)
+
+// The same value, of which the compiler cannot know that it was used before:
+// what the rarely taken redo derives from it holds no register in the tile loop.
+__device__ __forceinline__ int fresh(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+// Eight elements from p (16-byte aligned) as floats.
 template <typename T, typename E>
-__device__ void exact_row(const KvView<T> &kv, int S, int k_begin, int k_end, const T *q, int D, uint64_t w0,
-                          uint64_t w1, float c, float (&acc)[4], float &m, float &l) {
-    const int lane = threadIdx.x & 63;
-    m = -INFINITY;
-    l = 0.f;
+__device__ __forceinline__ void load8(const T *p, float (&x)[8]) {
+    if constexpr (sizeof(T) == 2) {
+        const u32x4 w = *reinterpret_cast<const u32x4 *>(p);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = 0.f;
-    for (int k0 = k_begin; k0 < k_end; k0 += 64) {
-        const int kk = k0 + lane;
-        float s = -INFINITY;
-        if (kk < k_end && (kk < S || pack_bit(kk - S, w0, w1))) {
-            const T *kp = kv.key(kk, S);
-            float dot = 0.f;
-            for (int d = 0; d < D; ++d) dot = fmaf(load_elem<T, E>(q + d), load_elem<T, E>(kp + d), dot);
-            s = dot * c;
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t bits = w[i];
+            x[2 * i] = E::widen((uint16_t)bits);
+            x[2 * i + 1] = E::widen((uint16_t)(bits >> 16));
         }
-        float mx = s;
-        for (int off = 32; off; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-        const float mn = fmaxf(m, mx);
-        const float alpha = mn == -INFINITY ? 1.f : exp2f(m - mn);
-        const float p = exp2f(s - (mn == -INFINITY ? 0.f : mn));
-        float ps = p;
-        for (int off = 32; off; off >>= 1) ps += __shfl_xor(ps, off);
-        l = l * alpha + ps;
-        m = mn;
+    } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] *= alpha;
-        for (int i = 0; i < 64 && k0 + i < k_end; ++i) {
-            const float pi = __shfl(p, i);
-            const T *vp = kv.val(k0 + i, S);
+        for (int i = 0; i < 2; ++i) {
+            const floatx4 y = *reinterpret_cast<const floatx4 *>(p + 4 * i);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (lane + 64 * j < D) acc[j] = fmaf(pi, load_elem<T, E>(vp + lane + 64 * j), acc[j]);
+            for (int j = 0; j < 4; ++j) x[4 * i + j] = y[j];
         }
     }
+}
+
+// The query rows (bit l32) of which a sum, the O^T of either lane half or the
+// weights' total, is not finite.
+template <int DB>
+__device__ __forceinline__ uint32_t nonfinite_rows(const floatx16 (&o)[DB], float ltot, bool qvalid) {
+    float z = ltot * 0.f;   // NaN as soon as one of them is not finite
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
+    const uint64_t bad = __ballot(qvalid && !(z == 0.f));
+    return (uint32_t)bad | (uint32_t)(bad >> 32);
+}
+
+// The wave's 32 query rows against keys [k_begin, k_end) with float products
+// (v_mfma_f32_32x32x2_f32): unnormalised O^T as the caller's kernel holds it,
+// running max (base 2; 0 for no key) and sum.  For waves in which a row's split products do
+// not hold what float products hold: an infinity or a NaN, whose remainder
+// after the first 16-bit term is no number.  Operands come from memory, 32
+// keys at a time, so a wave needs no other wave and no LDS: lane (l32, g)
+// takes head-dim elements 16 i + 8 g + [0, 8) of its key and its query, and
+// the values of keys 8 (e / 4) + 4 g + e % 4, whose weights it holds.  Pack
+// blocks no row sees are skipped as in the kernels.
+template <typename T, typename E, int D>
+__device__ void float_rows(const KvView<T> &kv, int S, int k_begin, int k_end, const T *q, int dr, uint64_t w0,
+                           uint64_t w1, float c, floatx16 (&o)[D / 32], float &m, float &l) {
+    const int lane = fresh(threadIdx.x & 63), l32 = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int db = 0; db < D / 32; ++db) o[db] = floatx16{};
+    m = -INFINITY;
+    l = 0.f;
+    const int pre_end = min(k_end, S);
+    for (int k0 = k_begin, n; k0 < k_end; k0 += n) {
+        const bool pack = k0 >= S;
+        n = min(32, (pack ? k_end : pre_end) - k0);
+        if (pack && !block_live(w0, w1, k0 - S, n)) continue;
+        // the block's first row; rows are less than 2^24 bytes apart here
+        const T *kb = pack ? kv.kpack + (int64_t)(k0 - S) * kv.kpack_t : kv.kpre + (int64_t)k0 * kv.kpre_t;
+        const T *vb = pack ? kv.vpack + (int64_t)(k0 - S) * kv.vpack_t : kv.vpre + (int64_t)k0 * kv.vpre_t;
+        const int kt = (int)(pack ? kv.kpack_t : kv.kpre_t), vt = (int)(pack ? kv.vpack_t : kv.vpre_t);
+        const T *kp = kb + min(l32, n - 1) * kt;   // (keys past the block: masked below)
+        floatx16 s = floatx16{};
+#pragma unroll 4
+        for (int d0 = 0; d0 < D; d0 += 16) {
+            // (elements past the head dim are zeros)
+            const int d = d0 + 8 * g, at = min(d, dr - 8);
+            float kx[8], qx[8];
+            load8<T, E>(kp + at, kx);
+            load8<T, E>(q + at, qx);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                s = __builtin_amdgcn_mfma_f32_32x32x2f32(d < dr ? kx[i] : 0.f, d < dr ? qx[i] : 0.f, s, 0, 0, 0);
+        }
+        const int lim = n - 4 * g;
+        uint32_t vis = pack ? vis_window(w0, w1, k0 - S + 4 * g) : ~0u;
+        vis &= lim >= 32 ? ~0u : (lim <= 0 ? 0u : ((1u << lim) - 1u));
+        float lmax = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            s[e] = (vis >> (8 * (e >> 2) + (e & 3))) & 1u ? s[e] : -INFINITY;
+            lmax = fmaxf(lmax, s[e]);
+        }
+        const float mn = fmaxf(m, fmaxf(lmax, partner32(lmax)) * c);
+        const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);
+        const float ms = mn == -INFINITY ? 0.f : mn;
+        l *= alpha;
+        m = mn;
+#pragma unroll
+        for (int db = 0; db < D / 32; ++db) o[db] *= alpha;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int off = 8 * (e >> 2) + 4 * g + (e & 3);
+            const float p = __builtin_amdgcn_exp2f(fmaf(s[e], c, -ms));
+            l += p;
+            const T *vp = vb + min(off, n - 1) * vt;
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db) {
+                const int d = 32 * db + l32;
+                const float x = load_elem<T, E>(vp + min(d, dr - 1));
+                const float v = off < n && d < dr ? x : 0.f;
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, p, o[db], 0, 0, 0);
+            }
+            if ((e & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // few loads in flight: registers
+        }
+    }
+    l += partner32(l);
+    if (m == -INFINITY) m = 0.f;
 }
 
 // What the MFMA kernel's epilogue needs, parked in LDS during the key loop
@@ -841,7 +921,8 @@ __device__ __forceinline__ bool next_unit(const AttnArgs &a, WorkCursor &cur, Un
 // missing elements of K, V and Q are zeros, and P, which the scalar kernel
 // that ran these dims kept in fp32, goes into the value product as E::kTerms
 // 16-bit terms that add up to it (each V^T operand read then feeds kTerms
-// MFMAs).  A row whose result is not finite is computed again in plain fp32.
+// MFMAs).  A row whose result is not finite is computed again with float
+// products (float_rows).
 // B = 4, S of 500 to 2000, P of 16 to 64, 32 / 8 heads of 96, fp16: 549 us on
 // the scalar kernel (no split-K, no matrix cores, each key row read by every
 // 16 query rows), 26.4 us here.
@@ -1231,6 +1312,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
         }
     }
     } else {
+    if constexpr (PAD) wait_loads();
     for (int t = 0; t < ntiles; ++t) {
         const int buf = t % NBUF;
         publish(buf);
@@ -1245,70 +1327,31 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     // O^T element e of lane (l32, g) in block db is d = 32*db + 8*(e/4) + 4*g + e%4.
     if (active) {
         const float ltot = lsum + partner32(lsum);
-        const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-        const float lse2 = ltot > 0.f ? msafe + log2f(ltot) : -INFINITY;
         const EpiArgs e = epi;
         // static split: row (token, head) of the partial rows; stream-K:
         // row wave * 32 + l32 of the workgroup's slot
         const int64_t prow = e.slot >= 0 ? (int64_t)e.slot * ROWS + wave * 32 + l32 : e.prow0 + qtok;
-        bool store_row = qvalid;
-        if constexpr (PAD) {
-            // NaN as soon as one of the row's sums is not finite
-            float z = ltot * 0.f;
+        // (padded instances) the rows to compute again with float products:
+        // those of which some sum is not finite
+        const uint32_t redo = PAD ? nonfinite_rows(o, ltot, qvalid) : 0;
+        auto store = [&](const floatx16(&x)[DB], float mx, float sum, bool mine) __attribute__((always_inline)) {
+            if (!mine || !qvalid) return;
+            const float inv = sum > 0.f ? 1.f / sum : 0.f;
+            const float lse2 = sum > 0.f ? mx + log2f(sum) : -INFINITY;
+            if (e.final_out) {
+                uint16_t *op = static_cast<uint16_t *>(e.out) + (int64_t)qtok * e.o_tok + (int64_t)qhead * e.o_head;
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
+                for (int db = 0; db < DB; ++db)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
-            const uint64_t bad = __ballot(qvalid && !(z == 0.f));
-            const uint32_t redo = (uint32_t)bad | (uint32_t)(bad >> 32);
-            store_row = qvalid && !(redo >> l32 & 1);
-            for (uint32_t left = redo; left; left &= left - 1) {
-                const int i = __builtin_ctz(left);
-                const int tok = bcast(qtok, i), head = bcast(qhead, i);
-                const int64_t row = bcast64(prow, i);
-                const uint64_t w0 = (uint64_t)bcast64((int64_t)mw0, i), w1 = (uint64_t)bcast64((int64_t)mw1, i);
-                float acc[4], mr, lr;
-                exact_row<uint16_t, E>(kv, sq.S, k_begin, k_end, qp + (int64_t)tok * a.q_tok + (int64_t)head * a.q_head,
-                                       dr, w0, w1, c, acc, mr, lr);
-                const float ir = lr > 0.f ? 1.f / lr : 0.f;
-                const float l2 = lr > 0.f ? (mr == -INFINITY ? 0.f : mr) + log2f(lr) : -INFINITY;
-                if (!e.final_out && row >= e.part_rows) {
-                    raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
-                    continue;
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int d = lane + 64 * j;
-                    if (d >= dr) break;
-                    if (e.final_out)
-                        static_cast<uint16_t *>(e.out)[(int64_t)tok * e.o_tok + (int64_t)head * e.o_head + d] =
-                            (uint16_t)E::pack2(acc[j] * ir, 0.f);
-                    else
-                        e.part_o[(row * e.Hq + head) * dr + d] = acc[j] * ir;
-                }
-                if (lane == 0) {
-                    if (!e.final_out)
-                        e.part_lse[row * e.Hq + head] = l2;
-                    else if (e.lse)
-                        e.lse[(int64_t)tok * e.Hq + head] = l2 * kLn2;
-                }
-            }
-        }
-        if (store_row && e.final_out) {
-            uint16_t *op = static_cast<uint16_t *>(e.out) + (int64_t)qtok * e.o_tok + (int64_t)qhead * e.o_head;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4) {
-                    const int d = db * 32 + 8 * r4 + 4 * g;
-                    if (PAD && db * 32 + 8 * r4 >= dr) continue;
-                    const u32x2 w = {E::pack2(o[db][4 * r4] * inv, o[db][4 * r4 + 1] * inv),
-                                     E::pack2(o[db][4 * r4 + 2] * inv, o[db][4 * r4 + 3] * inv)};
-                    *reinterpret_cast<u32x2 *>(op + d) = w;
-                }
-            if (e.lse && g == 0) e.lse[(int64_t)qtok * e.Hq + qhead] = lse2 * kLn2;
-        } else if (store_row) {
-            if (prow >= e.part_rows) {
+                    for (int r4 = 0; r4 < 4; ++r4) {
+                        const int d = db * 32 + 8 * r4 + 4 * g;
+                        if (PAD && db * 32 + 8 * r4 >= dr) continue;
+                        const u32x2 w = {E::pack2(x[db][4 * r4] * inv, x[db][4 * r4 + 1] * inv),
+                                         E::pack2(x[db][4 * r4 + 2] * inv, x[db][4 * r4 + 3] * inv)};
+                        *reinterpret_cast<u32x2 *>(op + d) = w;
+                    }
+                if (e.lse && g == 0) e.lse[(int64_t)qtok * e.Hq + qhead] = lse2 * kLn2;
+            } else if (prow >= e.part_rows) {
                 raise_flag(e.status, CAST_FLAG_BAD_OFFSETS);
             } else {
                 const int64_t orow = e.slot >= 0 ? prow : prow * e.Hq + qhead;
@@ -1319,12 +1362,21 @@ void tree_attn_mfma_kernel(AttnArgs a) {
                     for (int r4 = 0; r4 < 4; ++r4) {
                         const int d = db * 32 + 8 * r4 + 4 * g;
                         if (PAD && db * 32 + 8 * r4 >= dr) continue;
-                        const floatx4 w = {o[db][4 * r4] * inv, o[db][4 * r4 + 1] * inv, o[db][4 * r4 + 2] * inv,
-                                           o[db][4 * r4 + 3] * inv};
+                        const floatx4 w = {x[db][4 * r4] * inv, x[db][4 * r4 + 1] * inv, x[db][4 * r4 + 2] * inv,
+                                           x[db][4 * r4 + 3] * inv};
                         *reinterpret_cast<floatx4 *>(pp + d) = w;
                     }
                 if (g == 0) (e.slot >= 0 ? e.sk_lse : e.part_lse)[orow] = lse2;
             }
+        };
+        store(o, msafe, ltot, !(redo >> l32 & 1));
+        if (PAD && __builtin_expect(redo != 0, 0)) {
+            floatx16 x[DB];
+            float mx, sum;
+            float_rows<uint16_t, E, D>(kv, sq.S, k_begin, k_end,
+                                       qp + (int64_t)fresh(qtok) * a.q_tok + (int64_t)fresh(qhead) * a.q_head, dr, mw0,
+                                       mw1, c, x, mx, sum);
+            store(x, mx, sum, redo >> l32 & 1);
         }
     }
     if constexpr (kStreamK && !kPrefetchNext) has_next = cur.sk && sk_next_segment(a, cur, nxt, skr);
@@ -1347,7 +1399,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
 // round at most as often, so the error against 64 bits is no larger
 // (relative 2-norm, 8 requests of 1k to 4k keys at D = 128: 4.2e-7 against
 // 6.1e-7; with scores six times as wide 5.9e-7 against 1.5e-6).  A row that meets an infinity or a NaN, where a
-// remainder is no number, is computed again in plain fp32 (exact_row).
+// remainder is no number, is computed again with float products (float_rows).
 //
 // K and V are split once per tile while they are staged, Q once, P per tile
 // in registers.  Tiles of 32 keys: K [term][key][d] and V^T [term][d][key']
@@ -1652,6 +1704,7 @@ void tree_attn_f32_kernel(AttnArgs a) {
     };
 
     if (ntiles > 0) fetch(0);
+    wait_loads();
     for (int t = 0; t < ntiles; ++t) {
         const int buf = NBUF == 2 ? t & 1 : 0;
         publish(buf);
@@ -1663,8 +1716,6 @@ void tree_attn_f32_kernel(AttnArgs a) {
 
     if (active) {
         const float ltot = lsum + partner32(lsum);
-        const float inv = ltot > 0.f ? 1.f / ltot : 0.f;
-        const float lse2 = ltot > 0.f ? msafe + log2f(ltot) : -INFINITY;
         const EpiArgs e = epi;
         // static split: row (token, head) of the partial rows; stream-K:
         // row wave * 32 + l32 of the workgroup's slot
@@ -1680,43 +1731,32 @@ void tree_attn_f32_kernel(AttnArgs a) {
                          : e.lse        ? e.lse + (int64_t)qtok * e.Hq + qhead
                                         : nullptr;
         const float lse_unit = e.final_out ? kLn2 : 1.f;
-        // NaN as soon as one of the row's sums is not finite
-        float z = ltot * 0.f;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
-        const uint64_t bad = __ballot(qvalid && !(z == 0.f));
-        const uint32_t redo = (uint32_t)bad | (uint32_t)(bad >> 32);
-        if (qvalid && fits && !(redo >> l32 & 1)) {
-            if (lse_dst && g == 0) *lse_dst = lse2 * lse_unit;
+        // the rows to compute again with float products: those of which some
+        // sum is not finite
+        const uint32_t redo = nonfinite_rows(o, ltot, qvalid);
+        auto store = [&](const floatx16(&x)[DB], float mx, float sum, bool mine) __attribute__((always_inline)) {
+            if (!mine || !qvalid || !fits) return;
+            const float inv = sum > 0.f ? 1.f / sum : 0.f;
+            if (lse_dst && g == 0) *lse_dst = (sum > 0.f ? mx + log2f(sum) : -INFINITY) * lse_unit;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
                     const int d = db * 32 + 8 * r4 + 4 * g;
                     if (PAD && db * 32 + 8 * r4 >= dr) continue;
-                    const floatx4 w = {o[db][4 * r4] * inv, o[db][4 * r4 + 1] * inv, o[db][4 * r4 + 2] * inv,
-                                       o[db][4 * r4 + 3] * inv};
+                    const floatx4 w = {x[db][4 * r4] * inv, x[db][4 * r4 + 1] * inv, x[db][4 * r4 + 2] * inv,
+                                       x[db][4 * r4 + 3] * inv};
                     *reinterpret_cast<floatx4 *>(dst + d) = w;
                 }
-        }
-        for (uint32_t left = redo; left; left &= left - 1) {
-            const int i = __builtin_ctz(left);
-            float *const row = reinterpret_cast<float *>(bcast64(reinterpret_cast<int64_t>(dst), i));
-            float *const row_lse = reinterpret_cast<float *>(bcast64(reinterpret_cast<int64_t>(lse_dst), i));
-            if (!row) continue;
-            float acc[4], mr, lr;
-            exact_row<float, Bf16>(kv, sq.S, k_begin, k_end,
-                                   qp + (int64_t)bcast(qtok, i) * a.q_tok + (int64_t)bcast(qhead, i) * a.q_head, dr,
-                                   (uint64_t)bcast64((int64_t)mw0, i), (uint64_t)bcast64((int64_t)mw1, i), c, acc, mr,
-                                   lr);
-            const float ir = lr > 0.f ? 1.f / lr : 0.f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (lane + 64 * j < dr) row[lane + 64 * j] = acc[j] * ir;
-            if (row_lse && lane == 0)
-                *row_lse = (lr > 0.f ? (mr == -INFINITY ? 0.f : mr) + log2f(lr) : -INFINITY) * lse_unit;
+        };
+        store(o, msafe, ltot, !(redo >> l32 & 1));
+        if (__builtin_expect(redo != 0, 0)) {
+            floatx16 x[DB];
+            float mx, sum;
+            float_rows<float, Bf16, D>(kv, sq.S, k_begin, k_end,
+                                       qp + (int64_t)fresh(qtok) * a.q_tok + (int64_t)fresh(qhead) * a.q_head, dr, mw0,
+                                       mw1, c, x, mx, sum);
+            store(x, mx, sum, redo >> l32 & 1);
         }
     }
     } while (SKI && next_unit(a, cur, wu, skr));

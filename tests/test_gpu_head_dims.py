@@ -173,3 +173,65 @@ def test_fp32_terms_keep_floats(gpu, D, packs, what):
         assert torch.equal(torch.isnan(got), torch.isnan(want))
         fin = rows[..., None] & torch.isfinite(want)
         assert fin.any() and ((got.double() - want).abs()[fin] <= 2e-5).all()
+
+
+@pytest.mark.parametrize("layout", ["concat", "store"])
+@pytest.mark.parametrize("split", [-1, 0, 128])
+@pytest.mark.parametrize("D,dtype", [(64, "fp32"), (128, "fp32"), (256, "fp32"), (40, "fp32"), (200, "fp32"), (8, "bf16"),
+                                     (96, "fp16"), (120, "bf16"), (192, "fp16"), (248, "bf16")])
+def test_rows_again_with_float_products(gpu, D, dtype, split, layout):
+    # one infinity in every (request, head)'s values, in the prefix or the
+    # pack: every row that sees it is computed again, and its other elements
+    # have to match float64 as if nothing had happened
+    wl, q, k, v, meta, mask, words = _case(gpu, D, dtype, 5, [333, 0, 64], [64, 41, 5])
+    print(f"case rows-again D={D} {dtype} split={split} {layout}", flush=True)
+    for b in range(wl.B):
+        for h in range(wl.Hkv):
+            # an inner prefix key, or the pack's root, which every row sees
+            key = 100 if h and wl.prefix_len[b] > 100 else int(wl.prefix_len[b])
+            v[int(wl.cu_kv[b]) + key, h, 3] = math.inf
+    if layout == "concat":
+        out, lse = varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"],
+                                         mask, return_lse=True, kv_split=split, check=True)
+    else:
+        ks = torch.zeros((wl.B, wl.Hkv, 384, D), dtype=q.dtype, device=gpu)
+        vs, kp = torch.zeros_like(ks), torch.empty((wl.Hkv, wl.total_q, D), dtype=q.dtype, device=gpu)
+        vp = torch.empty_like(kp)
+        for b in range(wl.B):
+            a, S, e = int(wl.cu_kv[b]), int(wl.prefix_len[b]), int(wl.cu_kv[b + 1])
+            r = slice(int(wl.cu_q[b]), int(wl.cu_q[b + 1]))
+            for src, st, pk in ((k, ks, kp), (v, vs, vp)):
+                st[b, :, :S] = src[a:a + S].transpose(0, 1)
+                pk[:, r] = src[a + S:e].transpose(0, 1)
+        out, lse = store_tree_attention(q, ks, vs, kp, vp, meta["cu_q"], meta["prefix_len"], meta["pack_len"], mask,
+                                        total_kv=wl.total_kv, return_lse=True, kv_split=split, check=True)
+    want, want_l = _exact(wl, q, k, v.masked_fill(torch.isinf(v), 0.0), words)
+    got = out.double().cpu()
+    assert torch.isposinf(got[:, :, 3]).all()
+    keep = [d for d in range(D) if d != 3]
+    err = (got - want).abs()[..., keep]
+    assert (err <= 0.51 * EPS[dtype] * want.abs()[..., keep] + 2e-5).all(), f"{err.max()}"
+    assert ((lse.double().cpu() - want_l).abs() <= 2e-5).all()
+
+
+@pytest.mark.parametrize("D,dtype", [(128, "fp32"), (96, "fp16")])
+def test_one_nan_costs_little(gpu, D, dtype):
+    # rows that meet a NaN go through float products 32 at a time: measured 2
+    # to 4 times the clean call (row by row it was 30 to 200 times)
+    wl, q, k, v, meta, mask, _ = _case(gpu, D, dtype, 6, [4000] * 4, [64] * 4, Hq=32, Hkv=8)
+    print(f"case nan-cost D={D} {dtype}", flush=True)
+
+    def best():
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    clean = best()
+    v[5, 0, 7] = math.nan
+    assert best() < 12 * clean
