@@ -73,7 +73,8 @@ __device__ __forceinline__ void split_bf16x3(float lo, float hi, uint32_t &w0, u
     w1 = pack_bf16x2(lo, hi);
     lo -= __builtin_bit_cast(float, w1 << 16);
     hi -= __builtin_bit_cast(float, w1 & 0xffff0000u);
-    w2 = pack_bf16x2(lo, hi);
+    // (what is left has at most 8 bits: the upper half is all of it)
+    w2 = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi), __builtin_bit_cast(uint32_t, lo), 0x07060302u);
 }
 
 struct Fp16 {

@@ -1391,14 +1391,19 @@ void tree_attn_mfma_kernel(AttnArgs a) {
 // (tree_attn.py:66,87 cast p to the input dtype): so does this kernel.
 //
 // Structure of the bf16 kernel, with every operand as three bf16 terms that
-// add up to the float (8 bits a term, h + m + l) and six of the nine products
-// of the terms: l h, h l, m m, m h, h m, h h, the smallest first.  The three
-// left out are below 2^-26 of the product.  v_mfma_f32_32x32x2_f32, which ran
+// add up to the float (8 bits a term, h + m + l, each the rounding of what the
+// ones before it leave: |m| <= 2^-8, |l| <= 2^-17 of the float's power of two)
+// and six of the nine products of the terms: l h, h l, m m, m h, h m, h h, the
+// smallest first.  The three left out add up to at most 2^-24 of the product
+// (2^-24.0, rms 2^-26.8, over 40 million pairs), as much as the rounding of a float product,
+// and are of either sign.  v_mfma_f32_32x32x2_f32, which ran
 // here before, takes 16 times the bf16 cycles per product and rounds its sum
 // every 2 products; six bf16 steps of 16 products take 6 / 16 of that and
 // round at most as often, so the error against 64 bits is no larger
 // (relative 2-norm, 8 requests of 1k to 4k keys at D = 128: 4.2e-7 against
-// 6.1e-7; with scores six times as wide 5.9e-7 against 1.5e-6).  A row that meets an infinity or a NaN, where a
+// 6.1e-7; with scores six times as wide 5.9e-7 against 1.5e-6; rows of 2 to 8
+// keys 8.2e-8 against 1.4e-7, with all operands in [1, 1.02) 7.3e-8 against
+// 6.5e-8).  A row that meets an infinity or a NaN, where a
 // remainder is no number, is computed again with float products (float_rows).
 //
 // K and V are split once per tile while they are staged, Q once, P per tile
@@ -1675,10 +1680,11 @@ void tree_attn_f32_kernel(AttnArgs a) {
                 const float p1 = __builtin_amdgcn_exp2f(fmaf(s[8 * hf + 2 * e + 1], c, -msafe));
                 acc += p0;
                 acc += p1;
-                uint32_t x[3];
-                Bf16::split2(p0, p1, x);
-#pragma unroll
-                for (int i = 0; i < 3; ++i) w[i][e] = x[i];
+                uint32_t w0, w1, w2;
+                split_bf16x3(p0, p1, w0, w1, w2);
+                w[0][e] = w0;
+                w[1][e] = w1;
+                w[2][e] = w2;
             }
 #pragma unroll
             for (int i = 0; i < 3; ++i) pb[hf][i] = __builtin_bit_cast(bf16x8, w[i]);
@@ -1704,7 +1710,6 @@ void tree_attn_f32_kernel(AttnArgs a) {
     };
 
     if (ntiles > 0) fetch(0);
-    wait_loads();
     for (int t = 0; t < ntiles; ++t) {
         const int buf = NBUF == 2 ? t & 1 : 0;
         publish(buf);

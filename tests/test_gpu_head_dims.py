@@ -235,3 +235,27 @@ def test_one_nan_costs_little(gpu, D, dtype):
     clean = best()
     v[5, 0, 7] = math.nan
     assert best() < 12 * clean
+
+
+@pytest.mark.parametrize("n", [40, 900])
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+def test_fp32_products_left_out_are_unbiased(gpu, D, n):
+    # values just above 1 whose second and third terms are the largest there
+    # are, the same for every key: the output is the value, whatever the
+    # weights, and what is left out of the products would push all outputs to
+    # one side if the weights' terms had one sign
+    wl, q, k, v, meta, mask, words = _case(gpu, D, "fp32", 7, [n] * 8, [16] * 8)
+    print(f"case fp32-unbiased D={D} keys={n}", flush=True)
+    g = torch.Generator(gpu).manual_seed(D)
+    step = torch.randint(0, 30, (1, 1, D), generator=g, device=gpu)
+    v.copy_((1 + 2.0 ** -8 - 2.0 ** -17 + 2.0 ** -23 * step).expand_as(v))
+    out = varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask,
+                                check=True).double()
+    err = out / v[:1, :1].double() - 1
+    # 2^-24 a rounding: up to 16 in a lane's sum of weights and as many over
+    # tiles, the inverse, the result, 2^-24 left out; singly rounded values
+    # give an rms of 0.29 * 2^-23, a dozen of them 2^-23
+    assert err.abs().max() <= 2.0 ** -19 and err.pow(2).mean().sqrt() <= 2.0 ** -23
+    # of unknown sign, over 16384 outputs and more they cancel to below 2^-27
+    # (weights cut instead of rounded: -2^-26.2 to -2^-25.6)
+    assert err.mean().abs() <= 2.0 ** -27
