@@ -537,6 +537,31 @@ __device__ __forceinline__ float load_elem(const T *p) {
         return *p;
 }
 
+// Three bf16 terms hold the 24 bits of floats of 2^-110 and more; below, the
+// last of them is under bf16's smallest step, 2^-133, and up to 2^-134 of a
+// float is lost.  In a row whose largest element is 2^-100 or more that is
+// 2^-34 of the row; in others it is computed again with float products.
+constexpr float kLeastRow = 0x1p-100f;
+
+// (fp32) Whether the lane's row has outputs, all below kLeastRow: values, or
+// the weights of those that are not zero, may be too small to split.
+template <int DB>
+__device__ __forceinline__ bool small_rows(const floatx16 (&o)[DB], float ltot) {
+    float most = 0.f;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) most = fmaxf(most, fabsf(o[db][i]));
+    most = fmaxf(most, partner32(most));
+    return most > 0.f && most < ltot * kLeastRow;
+}
+
+// The rows (bit l32) for which either lane half says so.
+__device__ __forceinline__ uint32_t odd_rows(bool odd, bool qvalid) {
+    const uint64_t b = __ballot(qvalid && odd);
+    return (uint32_t)b | (uint32_t)(b >> 32);
+}
+
 // Waits for every load so far, the first tile's and Q's.  The tile loop needs
 // the former at once; without the wait the compiler may place the one for Q
 // inside the loop, where it also waits for the next tile's loads (d96-shaped
@@ -580,8 +605,7 @@ __device__ __forceinline__ uint32_t nonfinite_rows(const floatx16 (&o)[DB], floa
     for (int db = 0; db < DB; ++db)
 #pragma unroll
         for (int i = 0; i < 16; ++i) z = fmaf(o[db][i], 0.f, z);
-    const uint64_t bad = __ballot(qvalid && !(z == 0.f));
-    return (uint32_t)bad | (uint32_t)(bad >> 32);
+    return odd_rows(!(z == 0.f), qvalid);
 }
 
 // The wave's 32 query rows against keys [k_begin, k_end) with float products
@@ -1553,6 +1577,7 @@ void tree_attn_f32_kernel(AttnArgs a) {
 
     // Q^T operand: head-dim elements [ds*16 + g*8, +8) of this lane's query
     bf16x8 qf[3][DSTEPS];
+    float qmax = 0.f;
     {
         const float *src = qp + (int64_t)qtok * a.q_tok + (int64_t)qhead * a.q_head + g * 8;
 #pragma unroll
@@ -1565,12 +1590,18 @@ void tree_attn_f32_kernel(AttnArgs a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) x[4 * i + e] = y[e];
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qmax = fmaxf(qmax, fabsf(x[e]));
             u32x4 w[3];
             split8(x, w);
 #pragma unroll
             for (int i = 0; i < 3; ++i) qf[i][ds] = __builtin_bit_cast(bf16x8, w[i]);
         }
     }
+    // A query too small to split, or so large that keys too small to split
+    // show in its scores (what those lose, 2^-134 each, times 2^90).
+    qmax = fmaxf(qmax, partner32(qmax));
+    const bool odd_q = qmax > 0.f && (qmax < kLeastRow || qmax > 0x1p90f);
     uint64_t mw0 = 0, mw1 = 0;
     if (qvalid && k_end > sq.S) {
         const uint64_t *mp = a.mask + (int64_t)qtok * a.mask_words;
@@ -1737,8 +1768,8 @@ void tree_attn_f32_kernel(AttnArgs a) {
                                         : nullptr;
         const float lse_unit = e.final_out ? kLn2 : 1.f;
         // the rows to compute again with float products: those of which some
-        // sum is not finite
-        const uint32_t redo = nonfinite_rows(o, ltot, qvalid);
+        // sum is not finite, and those whose numbers are too small to split
+        const uint32_t redo = nonfinite_rows(o, ltot, qvalid) | odd_rows(small_rows(o, ltot) || odd_q, qvalid);
         auto store = [&](const floatx16(&x)[DB], float mx, float sum, bool mine) __attribute__((always_inline)) {
             if (!mine || !qvalid || !fits) return;
             const float inv = sum > 0.f ? 1.f / sum : 0.f;

@@ -259,3 +259,45 @@ def test_fp32_products_left_out_are_unbiased(gpu, D, n):
     # of unknown sign, over 16384 outputs and more they cancel to below 2^-27
     # (weights cut instead of rounded: -2^-26.2 to -2^-25.6)
     assert err.mean().abs() <= 2.0 ** -27
+
+
+@pytest.mark.parametrize("what", ["v", "q", "k"])
+@pytest.mark.parametrize("e", [-108, -112, -118, -124])
+@pytest.mark.parametrize("D", [64, 96, 128, 256])
+def test_fp32_small_magnitudes(gpu, D, e, what):
+    # below 2^-110 the third bf16 term of a float is under bf16's smallest
+    # step; the products have to keep what float products keep
+    wl, q, k, v, meta, mask, words = _case(gpu, D, "fp32", 8, [300, 0, 40], [8, 5, 20])
+    print(f"case fp32-small D={D} 2^{e} {what}", flush=True)
+    two = 2.0 ** e
+    if what == "v":
+        v *= two
+    elif what == "q":
+        q, k = q * two, k / two
+    else:
+        q, k = q / two, k * two
+    out, lse = varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask,
+                                     return_lse=True, check=True)
+    want, want_l = _exact(wl, q, k, v, words)
+    got = out.double().cpu()
+    # fp32 sums of up to 308 weights and products: 2^-24 * sqrt(308) * 4 < 5e-6,
+    # and results below the smallest normal float on its grid of 2^-149
+    assert (got - want).norm() <= 5e-6 * want.norm() + 2.0 ** -149 * want.numel() ** 0.5
+    assert ((lse.double().cpu() - want_l).abs() <= 2e-5).all()
+
+
+@pytest.mark.parametrize("nats", [40, 80, 84, 86])
+def test_fp32_small_weights(gpu, nats):
+    # a key of value zero holds all the weight but that of one far below it,
+    # which alone makes the output: its weight has to be a float's
+    wl, q, k, v, meta, mask, words = _case(gpu, 128, "fp32", 9, [300], [8])
+    print(f"case fp32-small-weight {nats} nats", flush=True)
+    q.zero_()[..., 0] = 1.0
+    k.zero_()[..., 0] = -4000.0
+    k[0, :, 0], k[1, :, 0] = 0.0, -nats * math.sqrt(128)
+    v[0] = v[2:] = 0.0
+    out = varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask,
+                                check=True)
+    want, _ = _exact(wl, q, k, v, words)
+    # the score in base 2, up to 124, is rounded to 2^-18: 2.6e-6 of the weight, twice
+    assert ((out.double().cpu() - want).abs() <= 1e-5 * want.abs()).all()
