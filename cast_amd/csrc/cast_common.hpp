@@ -52,7 +52,7 @@ struct Bf16 {
     // a float pair as the sum of kTerms pairs of the format, the largest
     // first: three truncations of 8 bits each hold all 24 bits
     static constexpr int kTerms = 3;
-    static constexpr float kTermShift = 0.f;
+    static constexpr float kTermShift = 0.f, kTermSlack = 8.f;
     static __device__ __forceinline__ void split2(float lo, float hi, uint32_t (&w)[3]) {
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
@@ -84,11 +84,12 @@ struct Fp16 {
     }
     static __device__ __forceinline__ uint32_t pack2(float lo, float hi) { return pack_f16x2(lo, hi); }
     static __device__ __forceinline__ float widen(uint16_t h) { return f16_to_float(h); }
-    // two roundings of 11 bits each leave 2^-24 of the value, as float does,
-    // while the second term is a normal half: values of about 1 are scaled by
-    // 2^kTermShift first
+    // Two roundings of 11 bits each leave 2^-24 of the value, as float does,
+    // while the second term is a normal half: values of up to 1 are scaled by
+    // 2^kTermShift, the most that fits (with no slack, kTermSlack, above 1).
+    // Down to 2^-16 that is so; below, 2^-40 is what is left.
     static constexpr int kTerms = 2;
-    static constexpr float kTermShift = 7.f;
+    static constexpr float kTermShift = 15.f, kTermSlack = 0.f;
     static __device__ __forceinline__ void split2(float lo, float hi, uint32_t (&w)[2]) {
         w[0] = pack_f16x2(lo, hi);
         w[1] = pack_f16x2(lo - f16_to_float((uint16_t)w[0]), hi - f16_to_float((uint16_t)(w[0] >> 16)));

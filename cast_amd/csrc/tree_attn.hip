@@ -945,7 +945,11 @@ __device__ __forceinline__ bool next_unit(const AttnArgs &a, WorkCursor &cur, Un
 // missing elements of K, V and Q are zeros, and P, which the scalar kernel
 // that ran these dims kept in fp32, goes into the value product as E::kTerms
 // 16-bit terms that add up to it (each V^T operand read then feeds kTerms
-// MFMAs).  A row whose result is not finite is computed again with float
+// MFMAs): all 24 bits in bf16; in fp16 2^-24 of a weight down to 2^-16 of the
+// largest, 2^-40 of the largest below, which moves an fp16 result by half its
+// smallest step only where the values of such keys add up to 2^15.  (For that
+// range fp16 rescales whenever the maximum moves, with no slack: nothing at
+// D = 96, 3 to 5 % at 80 and 112, 12 to 15 % at 192 and 248.)  A row whose result is not finite is computed again with float
 // products (float_rows).
 // B = 4, S of 500 to 2000, P of 16 to 64, 32 / 8 heads of 96, fp16: 549 us on
 // the scalar kernel (no split-K, no matrix cores, each key row read by every
@@ -956,6 +960,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
     using vec8 = typename E::vec8;
     constexpr int PT = PAD ? E::kTerms : 1;            // 16-bit terms of P
     constexpr float kShift = PAD ? E::kTermShift : 0.f;   // P is scaled by 2^kShift
+    constexpr float kSlack = PAD ? E::kTermSlack : kRescaleSlack;
     constexpr uint32_t kNowhere = 0x7ffffff0u;         // byte offset past every source: loads as zeros
     const int dr = PAD ? a.D : D;                      // the call's head dim
     constexpr int NT = WAVES * 64;
@@ -1226,7 +1231,7 @@ void tree_attn_mfma_kernel(AttnArgs a) {
         for (int e = 1; e < 16; ++e) lmax = fmaxf(lmax, s[0][e]);
 #pragma unroll
         for (int e = 0; e < 16; ++e) lmax = fmaxf(lmax, s[1][e]);
-        if (__any(lmax * c > m + kRescaleSlack)) {
+        if (__any(lmax * c > m + kSlack)) {
             const float mx = fmaxf(lmax, partner32(lmax)) * c;
             const float mn = fmaxf(m, mx);
             const float alpha = mn == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mn);

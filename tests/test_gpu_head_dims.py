@@ -301,3 +301,29 @@ def test_fp32_small_weights(gpu, nats):
     want, _ = _exact(wl, q, k, v, words)
     # the score in base 2, up to 124, is rounded to 2^-18: 2.6e-6 of the weight, twice
     assert ((out.double().cpu() - want).abs() <= 1e-5 * want.abs()).all()
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("D", [40, 96, 120, 192, 248])
+@pytest.mark.parametrize("nats", [5.3, 10.1, 14.2, 16.7, 19.3])
+def test_padded_small_weights(gpu, nats, D, dtype):
+    # a key of value zero holds nearly all the weight; the others, alike and
+    # far below it, make the output: their weights have to be held as floats
+    wl, q, k, v, meta, mask, words = _case(gpu, D, dtype, 10, [400, 90], [16, 33])
+    print(f"case padded-small-weights D={D} {dtype} {nats} nats", flush=True)
+    q.zero_()[..., 0] = 1.0
+    q[..., 1] = 1.0
+    k.zero_()[..., 0] = -nats * math.sqrt(D)
+    k[..., 1] = -nats * math.sqrt(D) - k[..., 0].float()       # what the format's rounding left
+    for b in range(wl.B):
+        first = int(wl.cu_kv[b])
+        k[first] = 0.0
+        v[first] = 0.0
+    v.mul_(100.0)
+    out = varlen_tree_attention(q, k, v, meta["cu_q"], meta["cu_kv"], meta["prefix_len"], meta["pack_len"], mask,
+                                kv_split=-1, check=True)
+    want, _ = _exact(wl, q, k, v, words)
+    # the output's own rounding (half a step, 2^-25 at least in fp16), and of
+    # the values' sum 2^-21 for the scores' and weights' roundings in fp32
+    span = 100 * 4 * 433 * math.exp(-nats) * 2.0 ** -21
+    assert ((out.double().cpu() - want).abs() <= 0.51 * EPS[dtype] * want.abs() + 2.0 ** -25 + span).all()
