@@ -39,6 +39,7 @@
 #include <type_traits>
 
 #include "cast_common.hpp"
+#include "split_choice.hpp"
 
 namespace cast {
 
@@ -302,18 +303,18 @@ __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok) {
     int L = max((int)((float)W * a.hkv_per_slot) - 1, 1);
 #pragma unroll
     for (int i = 0; i < 3; ++i) L += (int64_t)L * a.slots < total ? 1 : 0;   // the exact ceiling
-    const int few = a.esz == 4 ? a.slots : 192, least = a.esz == 4 ? 4 : 8;
-    L = max(L, total < (int64_t)least * few ? max(udiv((int)total, few), a.chunk >> 6) : least);
-    auto cand = [&](int w) { return (L * (w < 3 ? 8 + w : 12) + 7) >> 3; };
+    const bool f32 = a.esz == 4;
+    // (the quotient counts for few tiles only)
+    L = split_start(L, total, udiv((int)min(total, ((int64_t)1 << 22) - 1), split_few(f32, a.slots)), a.chunk >> 6, f32, a.slots);
     const int w = threadIdx.x >> 6;
     if (w < 4) {
-        const int c = cand(w);
+        const int c = split_candidate(L, w);
         const int n = wave_sum(tiles ? rb * udiv(tiles + c - 1, c) : 0);
         if ((threadIdx.x & 63) == 0) fit[w] = (int64_t)n * a.Hkv <= a.slots;
     }
     __syncthreads();
     const int4 f = *reinterpret_cast<const int4 *>(fit);   // one read
-    const int c = cand(f.x ? 0 : f.y ? 1 : f.z ? 2 : f.w ? 3 : 2);
+    const int c = split_candidate(L, split_pick(f.x, f.y, f.z, f.w));
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.split_tiles = c;
     t.ns = tiles ? udiv(tiles + c - 1, c) : 0;
     t.split_len = tiles ? udiv(tiles + t.ns - 1, t.ns) * 64 : 0;
@@ -2401,17 +2402,6 @@ struct SplitPlan {
 // (the longest-first order balances those), or where the averages ask for no
 // split and prefixes are short; and with one chunk of kMinChunk keys when even
 // that cannot give more items than the device holds (single-p16).
-//
-// Bounds of auto_split's result, with c >= L = W * Hkv / slots tiles per split
-// and RB = min(total_q * G / rows_wg + batch, batch * rbmax) >= sum rb: the
-// items fit the slots, or c >= 10/8 L and they are Hkv * sum rb * ceil(tiles / c)
-// <= 8/10 slots + Hkv * RB; an XCD takes at most ceil(groups / nx) groups of
-// each request, so its slots are at most items / nx, plus RB where Hkv is no
-// multiple of nx (workgroups past the last item cost their prologue at the end
-// of the call: 2 us at the headline with a bound of 640 for 256); a request
-// in ns > 1 splits has ns - 1 < tiles / c and P <= rb * rows_wg / G, so the
-// partial rows sum to less than rows_wg * slots / Hq plus the rows of the
-// split requests, which are at most that many again.
 static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, int32_t Hq, int32_t Hkv, int32_t D,
                             int32_t dtype, int32_t kv_split) {
     SplitPlan p{};
@@ -2435,14 +2425,9 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
         p.part_rows = part_rows_bound(total_q, total_kv, p.chunk);
         if ((int64_t)Hkv * rbmax * ((int64_t)total_kv / kMinChunk + batch) > slots) {
             p.slots = (int32_t)slots;
-            const int64_t by_rows = total_q * G / rows_wg + batch, by_pack = batch * rbmax;
-            const int64_t rb_sum = by_rows < by_pack ? by_rows : by_pack;
-            const int64_t once = (rows_wg * slots + Hq - 1) / Hq;
-            const int64_t rows = once + (once < total_q ? once : total_q);
-            if (rows < p.part_rows) p.part_rows = rows;
-            const int64_t second = (slots * 8 + 9) / 10 + Hkv * rb_sum;
-            const int64_t most = second > slots ? second : slots;
-            p.wg_bound = topo.xcds * ((most + topo.xcds - 1) / topo.xcds + (Hkv % topo.xcds ? rb_sum : 0));
+            const SplitBounds most = split_bounds(batch, total_q, Hq, Hkv, rows_wg, rbmax, slots, topo.xcds);
+            if (most.part_rows < p.part_rows) p.part_rows = most.part_rows;
+            p.wg_bound = most.wgs;
         }
         return p;
     }
