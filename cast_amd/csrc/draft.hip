@@ -550,15 +550,20 @@ constexpr int kBulkThreads = 512;
 constexpr int kBulkMin = 40;      // fewer nodes: the sorted path's pops cost less than the levels
 constexpr int kBulkSlack = 32;
 constexpr int kBins = 256;
+constexpr int kBulkLogProbs = 1024;   // L x k of the bulk instance that fits a CU twice
 
-// Where the tree builds of one workgroup keep their tables (LDS).
+// Where the tree builds of one workgroup keep their tables (LDS), for up to LP
+// log-probs.
+template <int LP>
 struct TreeLds {
-    double stl[kLMax * kTopKMax];   // the request's [L][k] log-probs
-    double pneg[kPoolMax];          // pool and bulk path: the candidates pushed so far
-    uint32_t pkey[kPoolMax];        //   their heap_key; bulk path: parent = the parent's place in the pool
-    double nscore[kMaxPack];        // popped nodes: score
-    uint32_t nkey[kMaxPack];        // popped nodes: heap_key
-    // bulk path
+    double stl[LP];            // the request's [L][k] log-probs
+    double pneg[kPoolMax];     // pool and bulk path: the candidates pushed so far
+    uint32_t pkey[kPoolMax];   //   their heap_key; bulk path: parent = the parent's place in the pool
+    double nscore[kMaxPack];   // popped nodes: score
+    uint32_t nkey[kMaxPack];   // popped nodes: heap_key
+};
+template <int LP>
+struct BulkLds : TreeLds<LP> {
     double sneg[kPoolMax];          // one depth's nodes as pushed,
     uint32_t skey[kPoolMax];
     double cneg[kBulkThreads];      // those within tau,
@@ -589,7 +594,8 @@ __device__ __forceinline__ int lane_scan(int x) {
 
 // rank[i] = the nodes of (cneg, ckey)[0, n) before node i; rank starts at
 // zero.  Thread (i, part) compares node i with every parts-th node.
-__device__ void rank_nodes(TreeLds &m, int n) {
+template <int LP>
+__device__ void rank_nodes(BulkLds<LP> &m, int n) {
     const int tid = threadIdx.x;
     const int shift = n <= 64 ? 6 : n <= 128 ? 7 : n <= 256 ? 8 : 9, parts = kBulkThreads >> shift;
     const int i = tid & ((1 << shift) - 1);
@@ -608,7 +614,8 @@ __device__ void rank_nodes(TreeLds &m, int n) {
 // workgroup call it and get the same result.  A depth's nodes enter the pool
 // in the heap's order, so that nodes of one depth compare by their parents'
 // places and (neg, heap_key) is that order for all nodes of the pool.
-__device__ int build_bulk(TreeLds &m, int L, int k, int want) {
+template <int LP>
+__device__ int build_bulk(BulkLds<LP> &m, int L, int k, int want) {
     const int tid = threadIdx.x, lane = tid & 63;
     double tau = INFINITY, worst = -m.stl[k - 1];   // worst: no node of this depth is worse
     if (tid <= kLMax) m.pushed[tid] = m.kept[tid] = 0;
@@ -738,14 +745,20 @@ __device__ int build_bulk(TreeLds &m, int L, int k, int want) {
     return min(n, want);
 }
 
-template <typename LP>
-__global__ __launch_bounds__(kBulkThreads) void build_trees_kernel(const int64_t *__restrict__ top_idx,
+// NT: threads, kBulkThreads with the bulk path or 64 without; NLP: log-probs of
+// a request at most.  Batches above the device's CUs need two workgroups a CU,
+// so the instances keep to 80 KB of LDS (the largest L x k in the bulk path
+// apart): with one kernel of 98 KB for all, 1024 requests of 32 nodes took
+// 50.9 us, 512 of 39 31.1.
+template <typename LP, int NT, int NLP>
+__global__ __launch_bounds__(NT) void build_trees_kernel(const int64_t *__restrict__ top_idx,
                                                          const LP *__restrict__ top_lp, int32_t L, int32_t k,
                                                          const int32_t *__restrict__ budget, int32_t uniform,
                                                          int64_t *token,
                                                          int32_t *depth, int32_t *parent, double *score,
                                                          int32_t *n_nodes, int32_t *status) {
-    __shared__ TreeLds m;
+    constexpr bool kBulk = NT > 64;
+    __shared__ typename std::conditional<kBulk, BulkLds<NLP>, TreeLds<NLP>>::type m;
     double *stl = m.stl, *nscore = m.nscore, *pneg = m.pneg;
     uint32_t *nkey = m.nkey, *pkey = m.pkey;
     const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
@@ -759,7 +772,7 @@ __global__ __launch_bounds__(kBulkThreads) void build_trees_kernel(const int64_t
     // stage the log-probs; check that each position is sorted (NaN fails)
     const int n_lp = L * k;
     bool sorted = true, plain = true;   // plain: finite and at most 0
-    for (int i = tid; i < n_lp; i += kBulkThreads) {
+    for (int i = tid; i < n_lp; i += NT) {
         const double v = (double)tl[i];
         stl[i] = v;
         plain = plain && v <= 0.0 && v > -INFINITY;
@@ -768,9 +781,11 @@ __global__ __launch_bounds__(kBulkThreads) void build_trees_kernel(const int64_t
     sorted = __syncthreads_and(sorted);
     plain = __syncthreads_and(plain);
     int nodes = -1;
-    if (sorted && plain && want >= kBulkMin) nodes = build_bulk(m, L, k, want);
-    if (nodes < 0 && tid >= 64) return;   // the other paths take one wave
-    const int step = nodes < 0 ? 64 : kBulkThreads;
+    if constexpr (kBulk) {
+        if (sorted && plain && want >= kBulkMin) nodes = build_bulk(m, L, k, want);
+        if (nodes < 0 && tid >= 64) return;   // the other paths take one wave
+    }
+    const int step = nodes < 0 ? 64 : NT;
     if (nodes >= 0) {
     } else if (sorted) {
         nodes = 0;
@@ -946,6 +961,9 @@ extern "C" int cast_draft_topk(const void *logits, int64_t logits_ld, int32_t ro
     return hipGetLastError() == hipSuccess ? CAST_OK : CAST_ERR_HIP;
 }
 
+template <int N>
+using Int = std::integral_constant<int, N>;
+
 // budget: per-request node counts, or null for `uniform` in every tree
 static int build_trees_run(const int64_t *top_idx, const void *top_lp, int32_t lp_dtype, int32_t batch, int32_t L,
                            int32_t k, const int32_t *budget, int32_t uniform, int64_t *token, int32_t *depth,
@@ -955,14 +973,22 @@ static int build_trees_run(const int64_t *top_idx, const void *top_lp, int32_t l
     if (batch == 0) return CAST_OK;
     if (!top_idx || !top_lp || !token || !depth || !parent || !score || !n_nodes) return CAST_ERR_NULL_POINTER;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (lp_dtype == CAST_FP32)
-        build_trees_kernel<float><<<batch, kBulkThreads, 0, s>>>(top_idx, static_cast<const float *>(top_lp), L, k,
-                                                                 budget, uniform, token, depth, parent, score, n_nodes,
-                                                                 status);
-    else
-        build_trees_kernel<double><<<batch, kBulkThreads, 0, s>>>(top_idx, static_cast<const double *>(top_lp), L, k,
-                                                                  budget, uniform, token, depth, parent, score,
-                                                                  n_nodes, status);
+    // one wave where the host knows that no tree takes the bulk path
+    const bool bulk = budget || uniform >= kBulkMin;
+    auto run = [&](auto lp, auto threads, auto most) {
+        build_trees_kernel<decltype(lp), decltype(threads)::value, decltype(most)::value>
+            <<<batch, decltype(threads)::value, 0, s>>>(top_idx, static_cast<const decltype(lp) *>(top_lp), L, k, budget,
+                                                        uniform, token, depth, parent, score, n_nodes, status);
+    };
+    auto run_lp = [&](auto lp) {
+        if (!bulk)
+            run(lp, Int<64>{}, Int<kLMax * kTopKMax>{});
+        else if (L * k <= kBulkLogProbs)
+            run(lp, Int<kBulkThreads>{}, Int<kBulkLogProbs>{});
+        else
+            run(lp, Int<kBulkThreads>{}, Int<kLMax * kTopKMax>{});
+    };
+    lp_dtype == CAST_FP32 ? run_lp(float{}) : run_lp(double{});
     return hipGetLastError() == hipSuccess ? CAST_OK : CAST_ERR_HIP;
 }
 

@@ -51,3 +51,47 @@ def test_trees_match_the_heap(gpu, L, k, kind, dtype):
         assert depth[b, :m].tolist() == [x.depth for x in ref]
         assert parent[b, :m].tolist() == [x.parent for x in ref]
         assert score[b, :m].tolist() == [x.score for x in ref]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("L,k", [(15, 8), (64, 16), (65, 16), (255, 16)])
+def test_one_budget_for_all(gpu, L, k, dtype):
+    # an int budget picks the kernel: one wave below 40 nodes, the bulk
+    # instance of up to 1024 log-probs a request, or the one of all others
+    rng = np.random.default_rng(L + k)
+    lp = torch.from_numpy(_lp("gaps", rng, 3, L, k)).to(dtype)
+    idx = torch.from_numpy(rng.integers(0, 1000, size=(3, L, k)))
+    for want in (0, 1, 39, 40, 64, 127):
+        print(f"case one-budget L={L} k={k} {dtype} nodes={want}", flush=True)
+        token, depth, parent, score, n = (x.cpu().numpy() for x in build_trees(idx.to(gpu), lp.to(gpu), want, check=True))
+        for b in range(3):
+            ref = build_tree(idx[b].numpy(), lp[b].double().numpy(), want, k)
+            m = len(ref)
+            assert n[b] == m
+            assert token[b, :m].tolist() == [x.token for x in ref]
+            assert depth[b, :m].tolist() == [x.depth for x in ref]
+            assert parent[b, :m].tolist() == [x.parent for x in ref]
+            assert score[b, :m].tolist() == [x.score for x in ref]
+
+
+def test_large_batches_share_a_cu(gpu):
+    # 1024 requests of 32 nodes: two workgroups a CU (51 us with one, 27 with two)
+    L, k, B = 15, 8, 1024
+    rng = np.random.default_rng(0)
+    lp = torch.from_numpy(_lp("gaps", rng, 8, L, k)).float().repeat(B // 8, 1, 1).to(gpu)
+    idx = torch.from_numpy(rng.integers(0, 1000, size=(8, L, k))).repeat(B // 8, 1, 1).to(gpu)
+    print("case trees-occupancy", flush=True)
+
+    def best(n):
+        times = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                build_trees(idx[:n], lp[:n], 32)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    assert best(B) < 2.5 * best(256)
