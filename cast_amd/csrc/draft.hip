@@ -658,7 +658,8 @@ __device__ int build_bulk(BulkLds<LP> &m, int L, int k, int want) {
             // worst): the upper edge of the bin that reaches the want-th node
             // is the new tau, widened by more than the float steps can lose
             const float width = (float)(tau < worst ? tau : worst) - lo;
-            const float per = width > 0.f ? (kBins - 1) / width : 0.f;
+            // (not for a width that floats cannot divide into bins: tau stays)
+            const float per = width > 1e-30f && width < INFINITY ? (kBins - 1) / width : 0.f;
             auto count = [&](double neg) {
                 if (neg <= tau) atomicAdd(&m.hist[min((int)(fmaxf((float)neg - lo, 0.f) * per), kBins - 1)], 1);
             };

@@ -22,6 +22,9 @@ def _lp(kind, rng, B, L, k):
         lp = -np.sort(rng.random((B, L, k)) * 1e-3, axis=2)
     elif kind == "positive":    # scores that grow along a path: not for the bulk path
         lp = 0.5 - np.cumsum(rng.exponential(0.3, size=(B, L, k)), axis=2)
+    elif kind == "tiny":        # scores whose differences floats cannot hold
+        lp = np.tile(-np.arange(k) * 1e-50, (B, L, 1))
+        lp[..., k - 1] = -1e-40 if k > 1 else 0.0
     else:                       # "masked": candidates of log-probability -inf
         lp = -np.cumsum(rng.exponential(1.0, size=(B, L, k)), axis=2)
         lp[..., max(1, k // 2):] = -np.inf
@@ -29,7 +32,7 @@ def _lp(kind, rng, B, L, k):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("kind", ["gaps", "coarse", "zeros", "flat", "positive", "masked"])
+@pytest.mark.parametrize("kind", ["gaps", "coarse", "zeros", "flat", "positive", "masked", "tiny"])
 @pytest.mark.parametrize("L,k", [(15, 8), (15, 16), (15, 10), (2, 4), (40, 2), (3, 1), (255, 3)])
 def test_trees_match_the_heap(gpu, L, k, kind, dtype):
     rng = np.random.default_rng(L * 100 + k)
