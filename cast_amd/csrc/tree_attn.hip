@@ -2227,14 +2227,25 @@ static int padded_dim(int32_t dtype, int32_t D) {
     return D < 64 ? 64 : D <= 96 ? 96 : D < 128 ? 128 : D <= 192 ? 192 : 256;
 }
 
-// Waves per workgroup (32 query rows each): 8 (256
-// rows, one workgroup per CU) when the average pack fills most of them, else 4
-// (128 rows, two workgroups per CU at head dim 128, three at 64): with few
-// rows a tile's time is the latency of one wave's QK -> softmax -> PV chain
-// (3,700 cycles for 32 KB), and two workgroups have twice the loads in
-// flight.  Best split of each, 4 against 8 waves, us: 32 requests of 132
-// rows 104 against 114, 16 of 96 rows 84 against 108, 32 of 20 rows 90
-// against 117; 8 of 256 rows 92 against 85, one of 512 rows 111 against 95.
+// Waves per workgroup (32 query rows each): 8 (256 rows, one workgroup per CU)
+// when the average pack fills most of them, else 4 (128 rows, two workgroups
+// per CU at head dim 128, three at 64): with few rows a tile's time is the
+// latency of one wave's QK -> softmax -> PV chain (3,700 cycles for 32 KB),
+// and two workgroups have twice the loads in flight.  4 against 8 waves, us:
+// 16 requests of 96 rows 84 against 108, 32 of 20 rows 90 against 117; 8 of
+// 256 rows 92 against 85, one of 512 rows 111 against 95.
+// Averages between one block of 128 rows and two decide by what they are made
+// of.  Ragged packs, many of which fit one block, gain: 32 requests of 300 to
+// 4k keys and 2 to 64 tokens (136 rows) 84 against 93, 16 of 2 to 72 tokens
+// (144) 48 against 65, until about 150 rows (148 to 184: 0.81 to 1.16 times,
+// 1.5 % slower on average).  Equal packs, whose second block is nearly empty,
+// lose: 8 requests of 8k keys and 132 rows 80 against 70, of 188 rows 86
+// against 77, 32 of 2k keys and 160 rows 85 against 76.  The host does not see
+// the packs, but where total_q is no multiple of the batch they are not equal.
+// So in 16 bits at head dim 128 such batches keep 4 waves up to 128 + 16 rows,
+// others up to 128.  At 64 (three workgroups per CU) and in fp32 4 waves hold
+// up to 192 (D = 64, 100 requests of 2k keys and 144 rows 192 against 242; 32
+// of 188 rows 67 against 68).
 // 2 waves (64 rows) were slower than 4 even at 64 rows (one request, 2064
 // keys: 17.5 against 16.4): each thread stages twice as much.
 // Head_dim 256 always runs 4 waves, one per SIMD: fewer threads would each
@@ -2244,19 +2255,25 @@ static int waves_for(int32_t batch, int32_t total_q, int32_t G, int32_t dtype, i
     const int dp = padded_dim(dtype, D);
     if (D == 256 || dp == 256 || (dp && dtype != CAST_FP32)) return 4;
     const int64_t p_avg = ((int64_t)total_q + batch - 1) / batch;
-    return (p_avg < kMaxPack ? p_avg : kMaxPack) * G <= 192 ? 4 : 8;
+    const int most = D == 64 || dtype == CAST_FP32 ? 192 : total_q % batch ? 144 : 128;
+    return (p_avg < kMaxPack ? p_avg : kMaxPack) * G <= most ? 4 : 8;
 }
 
 // The split-K chunk from the batch's averages: what kv_split = 0 means for
-// batches above 64 requests, and for smaller ones whether a call without
-// workspace is refused (below, the kernels choose the chunk themselves).
+// batches above 64 requests, and for smaller ones, where the kernels choose
+// the chunk themselves, whether a call without workspace is refused.  (That
+// stays as it was when 64-row workgroups and the largest pack decided: rows_wg
+// there is no longer that of the kernels.)
 static int32_t resolve_chunk(int32_t batch, int32_t total_q, int32_t total_kv, int32_t Hq, int32_t Hkv,
                              int32_t D, int32_t dtype, int32_t kv_split) {
     if (!mfma_path(dtype, D) || kv_split < 0 || batch <= 0) return kNoSplit;
     if (kv_split > 0) return ((kv_split + 63) / 64) * 64;
     const int64_t pmax = total_q < kMaxPack ? total_q : kMaxPack;
     const int64_t rows = pmax * (Hq / Hkv);
-    const int rows_wg = D == 256 ? 128 : rows <= 64 && dtype != CAST_FP32 ? 64 : rows <= 128 ? 128 : 256;
+    const int rows_wg = batch > 64      ? waves_for(batch, total_q, Hq / Hkv, dtype, D) * 32
+                        : D == 256      ? 128
+                        : rows > 128    ? 256
+                        : rows > 64 || dtype == CAST_FP32 ? 128 : 64;
     const int64_t p_avg = (total_q + batch - 1) / batch;
     const int64_t p_est = p_avg < kMaxPack ? p_avg : kMaxPack;
     const int64_t rb = (p_est * (Hq / Hkv) + rows_wg - 1) / rows_wg;

@@ -45,7 +45,8 @@ def _slots(packs, Hq, Hkv, D):
     """Query rows of a workgroup and the workgroups the device holds at once
     (256 CUs; per CU two of 4 waves at D = 128, three at 64, else one)."""
     G = Hq // Hkv
-    four = D == 256 or -(-sum(packs) // len(packs)) * G <= 192
+    most = 192 if D == 64 else 144 if sum(packs) % len(packs) else 128
+    four = D == 256 or -(-sum(packs) // len(packs)) * G <= most
     return (128, 256 * {256: 1, 128: 2, 64: 3}[D]) if four else (256, 256)
 
 
