@@ -35,6 +35,17 @@ CAST_HOST_DEVICE int split_pick(bool fit0, bool fit1, bool fit2, bool fit3) {
     return fit0 ? 0 : fit1 ? 1 : fit2 ? 2 : fit3 ? 3 : 2;
 }
 
+// Whether a batch whose rows alone fill the device is so even that it is better
+// left whole: its longest request (t_max tiles) no longer, against the average
+// over row blocks, than what the partials of two splits cost beside the keys
+// and values, less a tenth for what a split hides of latency
+// (split_even_limit: rows x 2 x 8 bytes a head dim written and read against
+// keys x 4; the host has the averages of both).
+CAST_HOST_DEVICE bool split_even(int t_max, int rb_sum, int W, float limit) {
+    return (float)t_max * (float)rb_sum <= limit * (float)W;
+}
+inline float split_even_limit(int64_t rows_avg, int64_t t_avg) { return 0.9f + 4.f * (float)rows_avg / (float)t_avg; }
+
 // Bounds of that choice, with c >= L = total / slots tiles per split (total =
 // Hkv * sum of row blocks x tiles) and RB >= sum rb: the items fit the slots,
 // or c >= 10/8 L and they are Hkv * sum rb * ceil(tiles / c) <= 8/10 slots +
@@ -44,7 +55,7 @@ CAST_HOST_DEVICE int split_pick(bool fit0, bool fit1, bool fit2, bool fit3) {
 // 2 us at the headline with a bound of 640 for 256); a request in ns > 1
 // splits has ns - 1 < tiles / c and P <= rb * rows_wg / G, so the partial rows
 // sum to less than rows_wg * slots / Hq plus the rows of the split requests,
-// which are at most that many again.
+// which are at most that many again.  (A batch left whole: Hkv * sum rb items.)
 struct SplitBounds {
     int64_t part_rows;   // partial rows
     int64_t wgs;         // workgroups

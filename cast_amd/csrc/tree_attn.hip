@@ -101,6 +101,7 @@ struct AttnArgs {
     int32_t slots;      // > 0: the kernels choose the split from the batch's lengths (auto_split) for this
                         // many workgroups, the number the device holds at once
     float hkv_per_slot; // Hkv / slots
+    float even_limit;   // split_even's (0: never left whole)
     int32_t *split_tiles;   // slots > 0: the attention kernel's choice (tiles per split), for the combine
     int32_t max_rows;   // longest key source (rows) the MFMA kernel can address
     int32_t xcds;       // XCDs of the device: workgroup x runs on XCD x % xcds
@@ -204,6 +205,12 @@ __device__ __forceinline__ int wave_scan(int x) {
 }
 // The saturated sum of x over the wave, in every lane.
 __device__ __forceinline__ int wave_sum(int x) { return bcast(wave_scan(x), 63); }
+// The wave's maximum, as a wave-uniform (scalar) value.
+__device__ __forceinline__ int wave_max(int x) {
+#pragma unroll
+    for (int off = 32; off; off >>= 1) x = max(x, __shfl_xor(x, off));
+    return __builtin_amdgcn_readfirstlane(x);
+}
 
 __device__ __forceinline__ Seq shfl_seq(const Seq &t, int src) {
     Seq s;
@@ -294,6 +301,12 @@ __device__ __forceinline__ bool batch_fits(const AttnArgs &a, const BatchTotals 
 // 1k to 8k keys, D = 128, 83.6 -> 70.9 us; 32 requests of 300 to 4k keys with
 // packs of 2 to 64 148.9 -> 95.2 us (with 4-wave workgroups, see waves_for);
 // 8 requests of 4k to 8k keys at D = 256 282.6 -> 224.7 us.
+// At D = 128 in 16 bits, where two workgroups a CU wait for memory and not for
+// each other's latency, batches that fill the device are left whole when they
+// are even (split_even): 64 requests of 1k keys and 128 rows over 4 KV heads
+// 62.9 -> 44.5 us, 32 of 700 keys and 64 rows 35.7 -> 30.9, 32 of 2k and 128
+// rows 75.4 -> 70 (with the chunk from the averages, none here, 47.0, 33.0 and
+// 73.6; a combine launch and the grid's spare workgroups are left).
 __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok) {
     __shared__ __attribute__((aligned(16))) int fit[4];
     const int tiles = ok && t.P > 0 ? (int)(((uint32_t)t.T + 63) >> 6) : 0;
@@ -306,6 +319,12 @@ __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok) {
     const bool f32 = a.esz == 4;
     // (the quotient counts for few tiles only)
     L = split_start(L, total, udiv((int)min(total, ((int64_t)1 << 22) - 1), split_few(f32, a.slots)), a.chunk >> 6, f32, a.slots);
+    int t_max = 0;
+    bool even = false;
+    if (a.even_limit > 0.f) {
+        t_max = max(wave_max(tiles), 1);
+        even = split_even(t_max, wave_sum(rb), W, a.even_limit);
+    }
     const int w = threadIdx.x >> 6;
     if (w < 4) {
         const int c = split_candidate(L, w);
@@ -314,7 +333,7 @@ __device__ void auto_split(const AttnArgs &a, Seq &t, bool ok) {
     }
     __syncthreads();
     const int4 f = *reinterpret_cast<const int4 *>(fit);   // one read
-    const int c = split_candidate(L, split_pick(f.x, f.y, f.z, f.w));
+    const int c = even ? t_max : split_candidate(L, split_pick(f.x, f.y, f.z, f.w));
     if (blockIdx.x == 0 && threadIdx.x == 0) *a.split_tiles = c;
     t.ns = tiles ? udiv(tiles + c - 1, c) : 0;
     t.split_len = tiles ? udiv(tiles + t.ns - 1, t.ns) * 64 : 0;
@@ -744,13 +763,6 @@ struct SkPlan {
 // Key tiles of a request: its prefix in 64-key tiles, then its pack.
 __device__ __forceinline__ int seq_tiles_pre(const Seq &t) { return (t.S + 63) >> 6; }
 __device__ __forceinline__ int seq_tiles(const Seq &t) { return ((t.S + 63) >> 6) + ((t.P + 63) >> 6); }
-
-// The wave's maximum, as a wave-uniform (scalar) value.
-__device__ __forceinline__ int wave_max(int x) {
-#pragma unroll
-    for (int off = 32; off; off >>= 1) x = max(x, __shfl_xor(x, off));
-    return __builtin_amdgcn_readfirstlane(x);
-}
 
 // Lane and member of workgroup x, and back: the two members of a lane run
 // on one XCD (workgroups are dealt to the XCDs round-robin).
@@ -2411,6 +2423,7 @@ struct SplitPlan {
     bool optional;       // runs unsplit without a workspace
     int64_t part_rows;   // partial rows the split can write
     int64_t wg_bound;    // workgroups the split can need (0: the general bound)
+    float even_limit;    // split_even's (0: never left whole)
 };
 
 // kv_split = 0 and up to 64 requests: the device chooses (a chunk the caller
@@ -2445,6 +2458,10 @@ static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, in
             const SplitBounds most = split_bounds(batch, total_q, Hq, Hkv, rows_wg, rbmax, slots, topo.xcds);
             if (most.part_rows < p.part_rows) p.part_rows = most.part_rows;
             p.wg_bound = most.wgs;
+            if (p.optional && D == 128 && dtype != CAST_FP32) {
+                const int64_t p_avg = ((int64_t)total_q + batch - 1) / batch;
+                p.even_limit = split_even_limit((p_avg < kMaxPack ? p_avg : kMaxPack) * G, t_avg);
+            }
         }
         return p;
     }
@@ -2604,10 +2621,11 @@ static int tree_attn_run(const void *q, const KvSource &kv, void *out, float *ls
     a.sk_min_tiles = kMinChunk / 64;
     const size_t split_need = split_bytes(sp, num_q_heads, head_dim);
     if (sp.optional && (!workspace || workspace_bytes < split_need || (reinterpret_cast<uintptr_t>(workspace) & 255)))
-        sp = SplitPlan{kNoSplit, 0, false, 0, 0};
+        sp = SplitPlan{kNoSplit, 0, false, 0, 0, 0.f};
     a.chunk = sp.chunk;
     a.by_chunk = fast_div((uint32_t)a.chunk);
     a.slots = sp.slots;
+    a.even_limit = sp.even_limit;
     a.hkv_per_slot = sp.slots ? (float)num_kv_heads / (float)sp.slots : 0.f;
     if (sp.slots)
         a.split_tiles = reinterpret_cast<int32_t *>(static_cast<char *>(workspace) + split_need - align256(sizeof(int32_t)));

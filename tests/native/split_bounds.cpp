@@ -1,7 +1,7 @@
 // Random batches through the split choice of split_choice.hpp and the
 // longest-first schedule's deal of groups to XCDs: the grid and the partial
 // rows that split_bounds allows have to hold what the choice makes.  Prints
-// how often each candidate was taken (4: none fits) and how often a bound was
+// how often each candidate was taken (4: none fits, 5: left whole) and how often a bound was
 // met exactly; exits 1 at the first batch that breaks one.
 #include <algorithm>
 #include <cstdio>
@@ -16,7 +16,7 @@ int main(int argc, char **argv) {
     const int rounds = argc > 1 ? std::atoi(argv[1]) : 20000;
     std::mt19937 rng(7);
     auto pick = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
-    long taken[5] = {0, 0, 0, 0, 0}, exact_wgs = 0, exact_rows = 0;
+    long taken[6] = {0, 0, 0, 0, 0, 0}, exact_wgs = 0, exact_rows = 0;
     for (int r = 0; r < rounds; ++r) {
         const int nx = pick(0, 3) ? 8 : pick(1, 6), Hkv = pick(1, 16), G = pick(1, 16), Hq = Hkv * G;
         const bool f32 = pick(0, 3) == 0;
@@ -44,8 +44,14 @@ int main(int argc, char **argv) {
         bool fit[4];
         for (int w = 0; w < 4; ++w) fit[w] = items(cast::split_candidate(start, w)) <= slots;
         const int w = cast::split_pick(fit[0], fit[1], fit[2], fit[3]);
-        const int c = cast::split_candidate(start, w);
-        ++taken[fit[w] ? w : 4];
+        const int t_max = *std::max_element(tiles.begin(), tiles.end());
+        long rb_sum = 0, keys = 0;
+        for (int b = 0; b < B; ++b) rb_sum += rb[b], keys += S[b] + P[b];
+        const float limit =
+            pick(0, 1) ? cast::split_even_limit(std::min((total_q + B - 1) / B, 128L) * G, (keys + B - 1) / B) : 0.f;
+        const bool even = cast::split_even(t_max, (int)rb_sum, (int)W, limit);
+        const int c = even ? t_max : cast::split_candidate(start, w);
+        ++taken[even ? 5 : fit[w] ? w : 4];
         long part = 0;
         for (int b = 0; b < B; ++b) {
             ns[b] = (tiles[b] + c - 1) / c;
@@ -72,7 +78,7 @@ int main(int argc, char **argv) {
         exact_wgs += wgs == most.wgs;
         exact_rows += part == most.part_rows;
     }
-    std::printf("taken %ld %ld %ld %ld %ld exact %ld %ld ok\n", taken[0], taken[1], taken[2], taken[3], taken[4],
-                exact_wgs, exact_rows);
+    std::printf("taken %ld %ld %ld %ld %ld %ld exact %ld %ld ok\n", taken[0], taken[1], taken[2], taken[3], taken[4],
+                taken[5], exact_wgs, exact_rows);
     return 0;
 }

@@ -52,11 +52,17 @@ def _slots(packs, Hq, Hkv, D):
 
 def _choice(prefix, packs, Hq, Hkv, D):
     """The split of a 16-bit batch from its lengths: the candidate taken (None:
-    no candidate's items fit the slots) and its tiles of 64 keys."""
+    no candidate's items fit the slots, "whole": no split) and its tiles of 64
+    keys."""
     rows_wg, slots = _slots(packs, Hq, Hkv, D)
     tiles = [-(-(s + p) // 64) if p else 0 for s, p in zip(prefix, packs)]
     rb = [-(-p * (Hq // Hkv) // rows_wg) for p in packs]
     total = Hkv * sum(t * r for t, r in zip(tiles, rb))
+    B, G = len(packs), Hq // Hkv
+    t_avg, rows_avg = -(-(sum(prefix) + sum(packs)) // B), min(-(-sum(packs) // B), 128) * G
+    p = plan(B, sum(packs), sum(prefix) + sum(packs), Hq, Hkv, D)
+    if p.kv_split == -1 and D == 128 and max(tiles) * sum(rb) * Hkv <= (0.9 + 4 * rows_avg / t_avg) * total:
+        return "whole", max(tiles)
     start = max(-(-total // slots), 1, 8 if total >= 8 * 192 else max(total // 192, 2))
     sizes = [(start * w + 7) // 8 for w in (8, 9, 10, 12)]
     fits = [Hkv * sum(r * -(-t // c) for t, r in zip(tiles, rb)) <= slots for c in sizes]
@@ -82,7 +88,8 @@ def _one_long(first, rest, n, pack, Hq, Hkv, D):
 CHOICES = [
     (0, _one_long(1000, 60, 9, 8, 32, 8, 128)), (1, _one_long(9000, 700, 24, 8, 32, 8, 128)),
     (2, _one_long(5000, 700, 28, 8, 32, 8, 128)), (3, _one_long(1000, 700, 32, 8, 32, 8, 128)),
-    (None, _one_long(1000, 900, 32, 8, 32, 8, 128)),
+    (None, _one_long(1200, 800, 32, 8, 32, 8, 128)), ("whole", _one_long(1000, 900, 32, 24, 32, 8, 128)),
+    ("whole", _one_long(700, 700, 31, 16, 32, 8, 128)),
     (0, _one_long(1000, 10, 9, 100, 20, 5, 128)), (1, _one_long(1000, 60, 9, 100, 20, 5, 128)),
     (2, _one_long(2000, 100, 20, 100, 20, 5, 128)), (3, _one_long(2000, 10, 17, 100, 20, 5, 128)),
     (None, _one_long(2000, 10, 19, 100, 20, 5, 128)),

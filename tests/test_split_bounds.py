@@ -21,5 +21,5 @@ def test_grid_and_partial_rows_hold_the_choice(tmp_path):
     run = subprocess.run([str(exe), "60000"], capture_output=True, text=True, timeout=120)
     assert run.returncode == 0, run.stdout + run.stderr
     word = run.stdout.split()
-    assert word[-1] == "ok" and all(int(n) > 100 for n in word[1:6])   # every candidate, and none fitting
-    assert int(word[7]) > 0                                            # the grid is no larger than need be
+    assert word[-1] == "ok" and all(int(n) > 100 for n in word[1:7])   # every candidate, none fitting, left whole
+    assert int(word[8]) > 0                                            # the grid is no larger than need be
