@@ -609,7 +609,7 @@ def attn_workload(dev, name, steps, warmup, cpu=False):
                combine_us=round(t["combine_us"], 2), steps=steps, warmup=warmup, dtype=wl.dtype,
                bound=rl["bound"], frac=rl["frac"],
                hbm_frac=round(wl.algorithmic_bytes() / (t["call_us"] * 1e-6) / PEAK_HBM, 4),
-               tokens=int(wl.total_q), kv_tokens=int(wl.total_kv), kv_split=h.plan.kv_split,
+               tokens=int(wl.total_q), kv_tokens=int(wl.total_kv), kv_split=h.kv_split, kv_split_estimate=h.plan.kv_split,
                algorithmic_bytes=wl.algorithmic_bytes(), algorithmic_flops=wl.algorithmic_flops(),
                whole_call_traffic=whole_call_traffic(wl, traffic_of(name)))
     log(f"  {name}: {t['call_us']:.1f} us/call (attn {t['attn_us']:.1f}, combine {t['combine_us']:.1f}), "
@@ -840,7 +840,7 @@ def main():
     log(f"device: {torch.cuda.get_device_name(dev)}")
     wl = scenarios.qwen3_headline()
     h = Harness(wl, dev, sets=args.sets, kv_split=args.kv_split)
-    log(f"workload {wl.name}: total_q={wl.total_q} total_kv={wl.total_kv} kv_split={h.plan.kv_split} "
+    log(f"workload {wl.name}: total_q={wl.total_q} total_kv={wl.total_kv} kv_split={h.kv_split} (from averages {h.plan.kv_split}) "
         f"workspace={h.plan.workspace_bytes / 2**20:.1f} MiB")
     t = h.time(args.steps, args.warmup)
     log(f"  call {t['call_us']:.1f} us (mean {t['call_mean_us']:.1f}), attention kernel {t['attn_us']:.1f} us, "
@@ -858,7 +858,7 @@ def main():
         "data": "synthetic (seeded Gaussian Q/K/V, trees from seeded N(0,5) 15x151936 block scores)",
         "config": {"workload": wl.name, "batch": wl.B, "prefix": int(wl.prefix_len[0]),
                    "pack": int(wl.pack_len[0]), "q_heads": wl.Hq, "kv_heads": wl.Hkv, "head_dim": wl.D,
-                   "kv_split": h.plan.kv_split, "kv_sets": args.sets},
+                   "kv_split": h.kv_split, "kv_split_estimate": h.plan.kv_split, "kv_sets": args.sets},
         "roofline": rl,
         "hbm_frac": round(wl.algorithmic_bytes() / call_s / PEAK_HBM, 4),
         "tokens_per_s": round(wl.total_q / call_s, 1),

@@ -420,7 +420,12 @@ using namespace cast;
 // against 6.7, 100 rows 13.2 against 11.2, 150 rows 14.2 against 14.2, more
 // rows slower cut; fp32 x 151936, 42 rows 26.9 against 10.3, 200 rows 38.8
 // against 27.5, 300 rows 42.5 against 38.0, 400 rows 47.3 against 48.0.  More
-// than 8 segments were slower almost everywhere.
+// than 8 segments were slower almost everywhere.  The same limits hold at other
+// lengths (the whole call): bf16 x 128256, 16 rows 10.2 against 7.5, 128 rows
+// 12.6 against 10.8; fp32 x 128256, 100 rows 24.3 against 14.5, 300 rows 27.8
+// against 27.4; fp32 x 32000, 16 rows 8.6 against 7.2, 300 rows 12.1 against
+// 10.6; bf16 x 32000 7.5 either way from 16 to 128 rows.  (Rows against 256
+// CUs: this library is built for one device.)
 constexpr int kSegmentBytes = 16 << 10;
 static int accept_splits(int32_t total_q, int32_t vocab, int32_t dtype) {
     const bool f32 = dtype == CAST_FP32;

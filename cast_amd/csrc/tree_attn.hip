@@ -1453,10 +1453,12 @@ void tree_attn_mfma_kernel(AttnArgs a) {
 // (keys permuted as in the bf16 kernel) take 57 KB at D = 128.  8 waves
 // double-buffer them, one workgroup per CU; 4 waves take one buffer and two
 // barriers a tile, two workgroups per CU; D = 256 takes one buffer of 112 KB
-// and one wave per SIMD.  Bound by the MFMA pipe and the splitting beside it:
-// 8 requests of 1k to 4k keys, packs of 2 to 64, D = 128 169.2 -> 98.1 us; 8 of
-// 2000 keys, packs of 128 295 -> 202 us; D = 64 130 -> 86 us; D = 256 (whose
-// one wave per SIMD spills 60 registers) 590 -> 508 us.
+// and one wave per SIMD.  Bound by the MFMA pipe and the splitting beside it,
+// which wait for each other at the tile's barriers: at the headline's shapes
+// the pipe is busy for 65 % of the time and the VALU issues for 36 %; at D =
+// 256 (whose one wave per SIMD spills 60 registers) 33 %.  8 requests of 1k to
+// 4k keys, packs of 2 to 64: D = 128 167 -> 95 us, D = 64 95 -> 55, D = 256 with
+// 16 heads 328 -> 209; 8 of 2000 keys, packs of 128, D = 128 286 -> 183.
 // --------------------------------------------------------------------------
 // PAD: head dims the instances do not name (multiples of 8 below D), the
 // missing elements zeros.
@@ -2427,11 +2429,18 @@ struct SplitPlan {
 };
 
 // kv_split = 0 and up to 64 requests: the device chooses (a chunk the caller
-// names is taken as it is).  Not worth the
-// combine launch where the rows alone fill the device one and a half times
-// (the longest-first order balances those), or where the averages ask for no
-// split and prefixes are short; and with one chunk of kMinChunk keys when even
-// that cannot give more items than the device holds (single-p16).
+// names is taken as it is).  Not worth the combine launch
+// - where the rows alone fill the device one and a half times; the
+//   longest-first order balances those (32 requests of 256 to 4k keys and full
+//   packs 218 us, split where that balances better 225; 64 of 500 to 3k keys
+//   and 256 rows 173 against 180; 64 of 500 to 2k keys and 8 tokens over 16 KV
+//   heads 136 against 132);
+// - where the averages ask for no split and prefixes are short (D = 128, 32
+//   requests of 200 keys and 4 tokens 14.7 us against 18.2, of 400 and 16
+//   tokens 21.3 against 25.5, of 10 to 900 keys and 4 tokens 26.9 against 25.3,
+//   64 of those 31.9 against 38.3);
+// and with one chunk of kMinChunk keys when even that cannot give more items
+// than the device holds (single-p16).
 static SplitPlan split_plan(int32_t batch, int32_t total_q, int32_t total_kv, int32_t Hq, int32_t Hkv, int32_t D,
                             int32_t dtype, int32_t kv_split) {
     SplitPlan p{};
