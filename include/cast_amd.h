@@ -93,11 +93,13 @@ int cast_tree_bitmask(const int32_t *parent, const int32_t *cu_q, int32_t batch,
  *   mask   uint64 [total_q][mask_words], mask_words 1 (int64 reference
  *          layout) or 2
  *   dtype  cast_dtype of q, k, v and out: CAST_BF16, CAST_FP16 or CAST_FP32
- *   head_dim  64, 128 or 256 on the MFMA kernels; any other multiple of 8
- *          up to 256 on a scalar kernel (the reference takes any power of
- *          two)
+ *   head_dim  64, 128 or 256, or any other multiple of 8 up to 256 on padded
+ *          instances of the same kernels (the reference takes any power of
+ *          two); of the latter, tensors that are not aligned to 16 bytes or
+ *          past the kernels' addressing take a scalar kernel
  *   sm_scale  > 0 (the Python layer substitutes 1/sqrt(D) for None)
- *   kv_split  keys per split-K chunk (multiple of 64); 0 lets the library
+ *   kv_split  keys per split-K chunk (multiple of 64; used at head dims 64,
+ *             128 and 256, the others do not split by it); 0 lets the library
  *             choose; CAST_SPLIT_STREAM (-2) asks for the stream-K schedule;
  *             any other negative value disables split-K.  With 0 long
  *             prefixes are cut into equal splits so that the work items cover

@@ -284,8 +284,8 @@ def test_mfma_ceiling_host_validation():
 
 
 def test_head_dim_bounds(lib):
-    # MFMA kernels take 64 and 128; the scalar kernel any other multiple of 8
-    # up to 256.  Out-of-range head dims are refused before any launch.
+    # 64, 128 and 256 have instances of their own, any other multiple of 8 up to
+    # 256 padded ones or the scalar kernel.  Out-of-range head dims are refused before any launch.
     fake = 1 << 20
     ptrs = dict(q=fake, k=fake, v=fake, out=fake, cu_q=fake, cu_kv=fake, prefix=fake, pack=fake, mask=fake)
     for D in (264, 100, 4, 512):

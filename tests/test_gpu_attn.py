@@ -146,7 +146,7 @@ def test_fp16_inputs(gpu):
 def test_head_dims_above_128(gpu):
     # the reference kernel takes any power-of-two head_dim (tl.arange(0, D),
     # tree_attn.py:36): 256 runs the MFMA kernels at one wave per SIMD (bf16,
-    # fp16 and fp32); the other multiples of 8 take the scalar kernel
+    # fp16 and fp32); the other multiples of 8 take the padded instances
     for Hq, Hkv, D, dt in [(8, 2, 256, "bf16"), (4, 4, 256, "fp32"), (8, 4, 192, "bf16"), (4, 1, 136, "fp32")]:
         wl = SC.random_parent_batch(seed=D + Hq, B=3, Hq=Hq, Hkv=Hkv, D=D, s_lo=20, s_hi=300, p_lo=1, p_hi=129,
                                     dtype=dt, qkv_scale=0.5)
